@@ -16,6 +16,9 @@ namespace mh {
 // A float4 as a clang vector type: arrays and struct members of it stay in registers, where
 // HIP's union float4 can be put in scratch memory.
 typedef float vf4 __attribute__((ext_vector_type(4)));
+// The same at any 4-byte boundary: gfx950 loads and stores 16 bytes there in one instruction,
+// so rows and columns of odd lengths move as quads too.
+typedef float vf4u __attribute__((ext_vector_type(4), aligned(4)));
 
 // ---------------------------------------------------------------------------------------
 // context
@@ -226,8 +229,20 @@ __device__ __forceinline__ void st_nt4(float* p, int64_t q, float4 v) {
 __device__ __forceinline__ void st_ntv(float* p, int64_t q, vf4 v) {
     __builtin_nontemporal_store(v, reinterpret_cast<vf4*>(p) + q);
 }
+// The quad at p and its store, at any 4-byte boundary.
+__device__ __forceinline__ vf4 ld_ntu(const float* p) {
+    return __builtin_nontemporal_load(reinterpret_cast<const vf4u*>(p));
+}
+__device__ __forceinline__ void st_ntu(float* p, vf4 v) {
+    __builtin_nontemporal_store(v, reinterpret_cast<vf4u*>(p));
+}
 __device__ __forceinline__ float ld_nt(const float* p) { return __builtin_nontemporal_load(p); }
 __device__ __forceinline__ void st_nt(float* p, float v) { __builtin_nontemporal_store(v, p); }
+
+// Whether a quad load at the end of row `row` (of nrows rows of B elements) leaves the tensor.
+__device__ __forceinline__ bool row_edge(int64_t row, int64_t nrows, int64_t B) {
+    return (nrows - 1 - row) * B < ((4 - (B & 3)) & 3);
+}
 
 // Component j of a float4.
 __device__ __forceinline__ float comp(const float4& q, int j) {

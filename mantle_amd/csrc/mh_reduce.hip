@@ -5,7 +5,8 @@
 //   C == 1, B <= 32 : 64 rows (a one-wavefront block) staged in LDS by coalesced float4
 //                     loads, one thread per row (unaligned x: one thread per row straight
 //                     from memory);
-//   C == 1, B < 2048: one wavefront (64 lanes) per row, 128-bit loads, butterfly shuffle;
+//   C == 1, B < 2048: one wavefront (64 lanes) per row, 128-bit loads at any alignment,
+//                     butterfly shuffle;
 //   C == 1, B >= 2048: 2048-element chunks, one 4-wave block each (two quads per thread),
 //                     whose partials reduce again along the row the same way;
 //   C  > 1, C % 4 == 0 and >= 1024 columns: one thread per column quad over a split of the
@@ -103,7 +104,7 @@ struct RMaxCntArg {
 };
 
 // ---------------------------------------------------------------------------------------
-// loaders: get(i) -> R::T at element i; get4 for 16-byte aligned quads
+// loaders: get(i) -> R::T at element i; get4 the quad from element i on, at any alignment
 // ---------------------------------------------------------------------------------------
 template <class R>
 struct LdPlain {
@@ -111,8 +112,9 @@ struct LdPlain {
     __device__ void setup() {}
     __device__ typename R::T get(int64_t i) const { return R::lift(ld_nt(x + i)); }
     __device__ void get4(int64_t i, typename R::T* o) const {
-        float4 q = ld_nt4(x + i, 0);
-        o[0] = R::lift(q.x); o[1] = R::lift(q.y); o[2] = R::lift(q.z); o[3] = R::lift(q.w);
+        const vf4 q = ld_ntu(x + i);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = R::lift(q[j]);
     }
 };
 
@@ -121,27 +123,26 @@ struct LdArg {  // x, each element with its index (tensors of fewer than 2^32 el
     __device__ void setup() {}
     __device__ MCI get(int64_t i) const { return MCI{ld_nt(x + i), 1u, (uint32_t)i}; }
     __device__ void get4(int64_t i, MCI* o) const {
-        const float4 q = ld_nt4(x + i, 0);
-        const uint32_t k = (uint32_t)i;
-        o[0] = MCI{q.x, 1u, k}; o[1] = MCI{q.y, 1u, k + 1}; o[2] = MCI{q.z, 1u, k + 2}; o[3] = MCI{q.w, 1u, k + 3};
+        const vf4 q = ld_ntu(x + i);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = MCI{q[j], 1u, (uint32_t)i + j};
     }
 };
 
 // Split partials of RMaxCnt (LdPairs) and RMaxCntArg (LdPairsArg): the maxima at m, the counts
 // at c. The combines above the first level need no indices (only the first level's feed the
-// routing), so LdPairsArg leaves them at their initial value. get4 is called at quad-aligned
-// offsets only (counts of partials a multiple of 4 in 64-float-aligned scratch): two quad
-// loads.
+// routing), so LdPairsArg leaves them at their initial value.
+typedef uint32_t vu4u __attribute__((ext_vector_type(4), aligned(4)));
 struct LdPairsArg {
     const float* m;
     const uint32_t* c;
     __device__ void setup() {}
     __device__ MCI get(int64_t k) const { return MCI{m[k], c[k], 0xffffffffu}; }
     __device__ void get4(int64_t k, MCI* o) const {
-        const float4 a = *reinterpret_cast<const float4*>(m + k);
-        const uint4 b = *reinterpret_cast<const uint4*>(c + k);
-        o[0] = MCI{a.x, b.x, 0xffffffffu}; o[1] = MCI{a.y, b.y, 0xffffffffu};
-        o[2] = MCI{a.z, b.z, 0xffffffffu}; o[3] = MCI{a.w, b.w, 0xffffffffu};
+        const vf4u a = *reinterpret_cast<const vf4u*>(m + k);
+        const vu4u b = *reinterpret_cast<const vu4u*>(c + k);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = MCI{a[j], b[j], 0xffffffffu};
     }
 };
 
@@ -151,9 +152,10 @@ struct LdPairs {
     __device__ void setup() {}
     __device__ MC get(int64_t i) const { return MC{m[i], c[i]}; }
     __device__ void get4(int64_t i, MC* o) const {
-        const float4 a = *reinterpret_cast<const float4*>(m + i);
-        const uint4 b = *reinterpret_cast<const uint4*>(c + i);
-        o[0] = MC{a.x, b.x}; o[1] = MC{a.y, b.y}; o[2] = MC{a.z, b.z}; o[3] = MC{a.w, b.w};
+        const vf4u a = *reinterpret_cast<const vf4u*>(m + i);
+        const vu4u b = *reinterpret_cast<const vu4u*>(c + i);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = MC{a[j], b[j]};
     }
 };
 
@@ -260,14 +262,12 @@ struct LdPowGrad {
     }
     template <bool FRAC, bool GX>
     __device__ void get4_t(int64_t i, float* o) const {
-        const float4 q = ld_nt4(x + i, 0);
-        const float4 u = ld_nt4(ug + i, 0);
-        float4 g = GX ? ld_nt4(gx + i, 0) : make_float4(0.f, 0.f, 0.f, 0.f);
-        o[0] = elem<FRAC, GX>(q.x, u.x, g.x);
-        o[1] = elem<FRAC, GX>(q.y, u.y, g.y);
-        o[2] = elem<FRAC, GX>(q.z, u.z, g.z);
-        o[3] = elem<FRAC, GX>(q.w, u.w, g.w);
-        if constexpr (GX) st_nt4(gx + i, 0, g);
+        const vf4 q = ld_ntu(x + i), u = ld_ntu(ug + i);
+        const vf4 g0 = GX ? ld_ntu(gx + i) : vf4{0.f, 0.f, 0.f, 0.f};
+        float g[4] = {g0.x, g0.y, g0.z, g0.w};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = elem<FRAC, GX>(q[j], u[j], g[j]);
+        if constexpr (GX) st_ntu(gx + i, vf4{g[0], g[1], g[2], g[3]});
     }
     __device__ float get(int64_t i) const {
         if (gx) return frac ? get_t<true, true>(i) : get_t<false, true>(i);
@@ -290,8 +290,7 @@ struct LdPowGrad {
 // ug / t2; operand 1 ((-t1) / (t2 * t2)) * ug, or (f * t1) * ug with f = -1 / (s * s) for
 // a scalar t2). `a` is the full-shape operand; `t2` of DIV's operand 1 has the grad's shape
 // and is read at the element's output line (i / (B*C)) * C + i % C. get4 takes a quad in
-// one row (C == 1) or over four consecutive lines (C % 4 == 0), with 16-byte loads when
-// `al`, else four scalar loads, so the reduction runs in the same order either way. COL1
+// one row (C == 1) or over four consecutive lines of one slab. COL1
 // (DIV's operand 1 only): C == 1, known when the kernel is compiled, so the divisor's load has
 // one form (under a branch between the two, the compiler waited at the join for every load
 // issued before it, and a thread's rows in flight went out one after another).
@@ -302,7 +301,6 @@ struct LdBinRg {
     const float* t2;
     int64_t BC, C;
     FastDiv fbc, fc;
-    bool al;
     float f;
     __device__ void setup() {
         if constexpr (DIVS) {
@@ -330,24 +328,15 @@ struct LdBinRg {
         return term(ld_nt(ug + i), ld_nt(a + i), d);
     }
     __device__ void get4(int64_t i, float* o) const {
-        float4 u, v;
-        if (al) {
-            u = ld_nt4(ug + i, 0);
-            v = ld_nt4(a + i, 0);
-        } else {
-            u = make_float4(ld_nt(ug + i), ld_nt(ug + i + 1), ld_nt(ug + i + 2), ld_nt(ug + i + 3));
-            v = make_float4(ld_nt(a + i), ld_nt(a + i + 1), ld_nt(a + i + 2), ld_nt(a + i + 3));
-        }
-        float4 d = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        const vf4 u = ld_ntu(ug + i), v = ld_ntu(a + i);
+        vf4 d = vf4{0.0f, 0.0f, 0.0f, 0.0f};
         if constexpr (OP == MH_DIV && ID == 1 && !DIVS) {
             const int64_t l = line(i);
-            if constexpr (COL1) d = make_float4(t2[l], t2[l], t2[l], t2[l]);
-            else d = make_float4(t2[l], t2[l + 1], t2[l + 2], t2[l + 3]);
+            if constexpr (COL1) d = vf4{t2[l], t2[l], t2[l], t2[l]};
+            else d = *reinterpret_cast<const vf4u*>(t2 + l);
         }
-        o[0] = term(u.x, v.x, d.x);
-        o[1] = term(u.y, v.y, d.y);
-        o[2] = term(u.z, v.z, d.z);
-        o[3] = term(u.w, v.w, d.w);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = term(u[j], v[j], d[j]);
     }
 };
 
@@ -404,7 +393,7 @@ __device__ __forceinline__ void part_store2(float* pm, int64_t npart, int64_t o,
 }
 
 // RMaxCnt over lanes whose counts are below 16 (a first-level chunk: each lane combines at most
-// eight elements): the maximum by six float shuffles, the count as four ballots, one per count
+// nine elements): the maximum by six float shuffles, the count as four ballots, one per count
 // bit, over the lanes at that maximum. The same count as wave_reduce<RMaxCnt> and a maximum
 // equal to its as a float (only the sign of a zero tie may differ), with half its shuffles:
 // the first pass of an all-element MAX backward took 49 us over 2^26 elements with the
@@ -598,57 +587,53 @@ __global__ void __launch_bounds__(kLdsRows)
     }
 }
 
-// One wavefront per (row, chunk): virtual row vr = r * S + s covers elements
-// [r*B + s*L, r*B + min((s+1)*L, B)). S == 1 writes the epilogue, S > 1 writes partials.
-template <class R, class LD, bool VEC>
+// One wavefront per row of B elements: the row's whole quads at lanes 0..63, 64..127, ... (at
+// any alignment), groups of four quads in flight, then its last B % 4 elements on the lane after
+// the last quad. Bound by memory. Rows of an odd length went one element per lane, 256 bytes an
+// instruction: [32768, 1023] SUM took 42 us that way, 22 us in quads.
+template <class R, class LD>
 __global__ void __launch_bounds__(kRThreads)
-    k_rows_wave(LD ld, int64_t nvrows, int64_t S, int64_t B, int64_t L, float* out, float* out2,
-                int epi, float div, float* part) {
+    k_rows_wave(LD ld, int64_t nrows, int64_t B, float* out, float* out2, int epi, float div) {
     ld.setup();
     using T = typename R::T;
     const int lane = threadIdx.x & 63;
-    const int64_t vr = (int64_t)blockIdx.x * (kRThreads / 64) + (threadIdx.x >> 6);
-    if (vr >= nvrows) return;  // uniform per wavefront; no block-level barrier follows
-    const int64_t r = vr / S, s = vr - r * S;
-    const int64_t start = r * B + s * L;
-    const int64_t rem = B - s * L;
-    const int64_t len = rem < L ? rem : L;
+    const int64_t r = (int64_t)blockIdx.x * (kRThreads / 64) + (threadIdx.x >> 6);
+    if (r >= nrows) return;  // uniform per wavefront; no block-level barrier follows
+    const int64_t start = r * B;
+    const int64_t nq = B >> 2;
+    T a4[4][4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) a4[u][j] = R::init();
+    int64_t q = lane;
+    for (; q + 192 < nq; q += 256) {
+        T v[4][4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) ld.get4(start + (q + 64 * u) * 4, v[u]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) a4[u][j] = R::comb(a4[u][j], v[u][j]);
+    }
+    for (; q < nq; q += 64) {
+        T v[4];
+        ld.get4(start + q * 4, v);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) a4[0][j] = R::comb(a4[0][j], v[j]);
+    }
+    if (q == nq) {  // the lane after the last quad
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+            if (q * 4 + j < B) a4[0][j] = R::comb(a4[0][j], ld.get(start + q * 4 + j));
+    }
     T acc = R::init();
-    if (VEC) {
-        const int64_t nq = len >> 2;
-        T a4[4][4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < 4; ++u)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) a4[u][j] = R::init();
-        int64_t q = lane;
-        for (; q + 192 < nq; q += 256) {
-            T v[4][4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) ld.get4(start + (q + 64 * u) * 4, v[u]);
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) a4[u][j] = R::comb(a4[u][j], v[u][j]);
-        }
-        for (; q < nq; q += 64) {
-            T v[4];
-            ld.get4(start + q * 4, v);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) a4[0][j] = R::comb(a4[0][j], v[j]);
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc = R::comb(acc, a4[u][j]);
-    } else {
-        for (int64_t j = lane; j < len; j += 64) acc = R::comb(acc, ld.get(start + j));
-    }
+        for (int j = 0; j < 4; ++j) acc = R::comb(acc, a4[u][j]);
     acc = wave_reduce<R>(acc);
-    if (lane == 0) {
-        if (S == 1) epi_store(out, out2, r, acc, epi, div);
-        else part_store2(part, nvrows, vr, acc);
-    }
+    if (lane == 0) epi_store(out, out2, r, acc, epi, div);
 }
 
 // Short columns (B <= 64) of a serial accumulation (EPI_SEQ_ACCUM / _NEG): one thread per
@@ -730,7 +715,7 @@ __global__ void __launch_bounds__(kRThreads)
 // row): 1024 threads, each with all of its (up to eight) quads' loads in flight, so the row
 // takes one memory round trip; the sixteen wave results combine by a fixed butterfly.
 constexpr int kCombThreads = 1024;
-template <class R, class LD, bool VEC>
+template <class R, class LD>
 __global__ void __launch_bounds__(kCombThreads)
     k_row_comb(LD ld, int64_t B, float* out, float* out2, int epi, float div) {
     using T = typename R::T;
@@ -739,23 +724,20 @@ __global__ void __launch_bounds__(kCombThreads)
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int64_t r = blockIdx.x, start = r * B;
     T acc = R::init();
-    if (VEC) {
-        constexpr int U = 8;  // kCombineMax / (4 * kCombThreads)
-        T v[U][4];
+    constexpr int U = 8;  // kCombineMax / (4 * kCombThreads)
+    T v[U][4];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int64_t e = ((int64_t)u * kCombThreads + t) * 4;
-            if (e < B) ld.get4(start + e, v[u]);
-        }
+    for (int u = 0; u < U; ++u) {
+        const int64_t e = ((int64_t)u * kCombThreads + t) * 4;
+        if (e + 3 < B) ld.get4(start + e, v[u]);
+    }
+    if (t < (int)(B & 3)) acc = R::comb(acc, ld.get(start + (B & ~(int64_t)3) + t));  // the last B % 4
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int64_t e = ((int64_t)u * kCombThreads + t) * 4;
-            if (e < B)
+    for (int u = 0; u < U; ++u) {
+        const int64_t e = ((int64_t)u * kCombThreads + t) * 4;
+        if (e + 3 < B)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc = R::comb(acc, v[u][j]);
-        }
-    } else {
-        for (int64_t e = t; e < B; e += kCombThreads) acc = R::comb(acc, ld.get(start + e));
+            for (int j = 0; j < 4; ++j) acc = R::comb(acc, v[u][j]);
     }
     acc = wave_reduce<R>(acc);
     if (lane == 0) ws[w] = acc;
@@ -825,7 +807,7 @@ __global__ void __launch_bounds__(kRThreads)
 // vr = r * S + s covers elements [r*B + s*L, r*B + min((s+1)*L, B)); the four wave results
 // combine in wave order. S == 1 writes the row's epilogue, S > 1 the partial part[vr].
 constexpr int64_t kRowChunk = 2048;
-template <class R, class LD, bool VEC>
+template <class R, class LD>
 __global__ void __launch_bounds__(kRThreads)
     k_rows_block(LD ld, int64_t S, int64_t B, int64_t L, float* out, float* out2, int epi, float div,
                  float* part, int64_t npart) {
@@ -840,28 +822,29 @@ __global__ void __launch_bounds__(kRThreads)
     const int64_t len = rem < L ? rem : L;
     T acc = R::init();
     constexpr bool kMaxCntFirst = std::is_same<R, RMaxCnt>::value && std::is_same<LD, LdPlain<RMaxCnt>>::value;
-    if constexpr (VEC && kMaxCntFirst) {
+    const int64_t nq = len >> 2;
+    const int tail = t < (int)(len & 3) ? 1 : 0;  // threads 0.. take the last len % 4 elements
+    if constexpr (kMaxCntFirst) {
         // a first-level max-count chunk (L <= kRowChunk: at most two quads per thread): the
         // lane's maximum by comparisons, then its count as the elements equal to it, which is
         // RMaxCnt's count (NaN, also the filler of a missing quad, is neither) without the
         // pairwise combining (46.8 -> 39.4 us over 2^26 elements, the plain maximum's time)
         static_assert(kRowChunk <= 8 * kRThreads, "a first-level chunk is at most two quads per thread");
-        const int64_t nq = len >> 2;
         const float nan = __builtin_nanf("");
-        const float4 fq = make_float4(nan, nan, nan, nan);
+        const vf4 fq = vf4{nan, nan, nan, nan};
         const float* xs = ld.x + start;
-        const float4 qa = t < nq ? ld_nt4(xs, t) : fq;
-        const float4 qb = t + kRThreads < nq ? ld_nt4(xs, t + kRThreads) : fq;
-        const float v[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
+        const vf4 qa = t < nq ? ld_ntu(xs + 4 * t) : fq;
+        const vf4 qb = t + kRThreads < nq ? ld_ntu(xs + 4 * (t + kRThreads)) : fq;
+        const float vt = tail ? ld_nt(xs + 4 * nq + t) : nan;
+        const float v[9] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w, vt};
         float m = -FLT_MAX;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) m = v[j] > m ? v[j] : m;
+        for (int j = 0; j < 9; ++j) m = v[j] > m ? v[j] : m;
         uint32_t c = 0;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) c += v[j] == m ? 1u : 0u;
+        for (int j = 0; j < 9; ++j) c += v[j] == m ? 1u : 0u;
         acc = MC{m, c};
-    } else if (VEC) {
-        const int64_t nq = len >> 2;
+    } else {
         T a2[2][4];
 #pragma unroll
         for (int u = 0; u < 2; ++u)
@@ -883,15 +866,14 @@ __global__ void __launch_bounds__(kRThreads)
 #pragma unroll
             for (int j = 0; j < 4; ++j) a2[0][j] = R::comb(a2[0][j], v[j]);
         }
+        if (tail) a2[1][3] = R::comb(a2[1][3], ld.get(start + 4 * nq + t));
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
             for (int j = 0; j < 4; ++j) acc = R::comb(acc, a2[u][j]);
-    } else {
-        for (int64_t j = t; j < len; j += kRThreads) acc = R::comb(acc, ld.get(start + j));
     }
     if constexpr (std::is_same<R, RMaxCnt>::value && std::is_same<LD, LdPlain<RMaxCnt>>::value)
-        acc = wave_reduce_mc_small(acc);  // L <= kRowChunk: at most eight elements per lane
+        acc = wave_reduce_mc_small(acc);  // L <= kRowChunk: at most nine elements per lane
     else
         acc = wave_reduce<R>(acc);
     if (lane == 0) ws[w] = acc;
@@ -964,10 +946,44 @@ __global__ void __launch_bounds__(kRThreads)
     }
 }
 
-// MAX backward over rows of B <= 16384 elements (B % 4 == 0), one pass: the row is held in
+// A row's quads tr, tr + NT, ... into registers, elements past the row's B as `pad`. A quad that
+// runs past the row reads on into the next row; `edge` (uniform over the row's threads) marks the
+// tensor's last row, where it would leave the tensor and its elements load one by one. The two
+// forms are one uniform branch around all of a thread's loads, so these stay in flight together.
+template <int NQ, int NT>
+__device__ __forceinline__ void load_row_quads(vf4 (&v)[NQ], const float* xr, int tr, int64_t B, bool edge, float pad) {
+    const int64_t nqc = (B + 3) >> 2;
+    if (!edge) {
+#pragma unroll
+        for (int k = 0; k < NQ; ++k) {
+            const int64_t qi = tr + (int64_t)k * NT;
+            if (qi < nqc) v[k] = ld_ntu(xr + 4 * qi);
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < NQ; ++k) {
+            const int64_t e = 4 * (tr + (int64_t)k * NT);
+            if (e + 3 < B) {
+                v[k] = ld_ntu(xr + e);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) v[k][j] = e + j < B ? ld_nt(xr + e + j) : pad;
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) {
+        const int64_t e = 4 * (tr + (int64_t)k * NT);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[k][j] = e + j < B ? v[k][j] : pad;
+    }
+}
+// MAX backward over rows of B <= 16384 elements, one pass: the row is held in
 // registers (NQ quads per thread, WPR waves per row), its max and count reduced across the
 // row's threads, then grad[i] = grad[i] + (x[i] == m ? fl(1/c) * ug[row] : 0) from the same
-// registers (basics.mojo:581-615 for a last-axis reduce): x is read once.
+// registers (basics.mojo:581-615 for a last-axis reduce): x is read once. Rows of any length and
+// alignment (odd lengths took a max-count pass and a gathering pass: the SUM, MEAN and MAX passes
+// over [65536, 1001] together 650 us, 448 us now).
 template <int WPR, int NQ>
 __global__ void __launch_bounds__(kRThreads)
     k_max_bwd_rowreg(float* __restrict__ grad, const float* __restrict__ x, const float* __restrict__ ug,
@@ -978,36 +994,25 @@ __global__ void __launch_bounds__(kRThreads)
     if (row >= nrows) return;  // WPR == 1: uniform per wave, and that path has no barrier
     const int tr = WPR == 1 ? lane : (int)threadIdx.x;
     constexpr int NT = 64 * WPR;
-    const int64_t Bq = B >> 2;
     const float* xr = x + row * B;
     float* gr = grad + row * B;
+    const bool edge = row_edge(row, nrows, B);
     // One wave per row (WPR == 1): the row's x and grad quads and its ug are loaded together,
     // one wait for memory, the grad quads held in registers while the row's max and count
     // are found ([64, 512, 1024]: 47.5 -> 46.1 us). Four waves per row keep the grad loads
     // after the reduction: holding them would take 8 of 16 quads' registers and cut the
     // resident waves from 8 to 5 per SIMD ([8192, 8192] axis 1: 80.9 -> 82.1 us).
     constexpr bool PRE = WPR == 1;
-    float4 v[NQ], o[NQ];
-#pragma unroll
-    for (int k = 0; k < NQ; ++k) {
-        const int64_t qi = tr + (int64_t)k * NT;
-        if (qi < Bq) {
-            v[k] = ld_nt4(xr, qi);
-            if (PRE) o[k] = ld_nt4(gr, qi);
-        }
-    }
+    const float nan = __builtin_nanf("");  // neither a maximum nor counted
+    vf4 v[NQ], o[NQ];
+    load_row_quads<NQ, NT>(v, xr, tr, B, edge, nan);
+    if (PRE) load_row_quads<NQ, NT>(o, gr, tr, B, edge, 0.0f);
     const float u = PRE ? ug[row] : 0.0f;
     MC acc = RMaxCnt::init();
 #pragma unroll
-    for (int k = 0; k < NQ; ++k) {
-        const int64_t qi = tr + (int64_t)k * NT;
-        if (qi < Bq) {
-            acc = RMaxCnt::comb(acc, RMaxCnt::lift(v[k].x));
-            acc = RMaxCnt::comb(acc, RMaxCnt::lift(v[k].y));
-            acc = RMaxCnt::comb(acc, RMaxCnt::lift(v[k].z));
-            acc = RMaxCnt::comb(acc, RMaxCnt::lift(v[k].w));
-        }
-    }
+    for (int k = 0; k < NQ; ++k)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc = RMaxCnt::comb(acc, RMaxCnt::lift(v[k][j]));
     acc = wave_reduce<RMaxCnt>(acc);
     if (WPR == 4) {
         if (lane == 0) ws[w] = acc;
@@ -1017,14 +1022,20 @@ __global__ void __launch_bounds__(kRThreads)
     const float f = 1.0f / (float)acc.c;  // basics.mojo:609
     const float g = f * (PRE ? u : ug[row]);
     const float m = acc.m;
+    if (!PRE) load_row_quads<NQ, NT>(o, gr, tr, B, edge, 0.0f);
 #pragma unroll
     for (int k = 0; k < NQ; ++k) {
-        const int64_t qi = tr + (int64_t)k * NT;
-        if (qi < Bq) {
-            const float4 ok = PRE ? o[k] : ld_nt4(gr, qi);
-            const float4 n = make_float4(ok.x + (v[k].x == m ? g : 0.0f), ok.y + (v[k].y == m ? g : 0.0f),
-                                         ok.z + (v[k].z == m ? g : 0.0f), ok.w + (v[k].w == m ? g : 0.0f));
-            if (bits_differ4(ok.x, ok.y, ok.z, ok.w, n.x, n.y, n.z, n.w)) st_nt4(gr, qi, n);  // a sparse accumulation
+        const int64_t e = 4 * (tr + (int64_t)k * NT);
+        vf4 n;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) n[j] = o[k][j] + (v[k][j] == m ? g : 0.0f);
+        if (!bits_differ4(o[k].x, o[k].y, o[k].z, o[k].w, n.x, n.y, n.z, n.w)) continue;  // a sparse accumulation
+        if (e + 3 < B) {
+            st_ntu(gr + e, n);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+                if (e + j < B) st_nt(gr + e + j, n[j]);
         }
     }
 }
@@ -1045,6 +1056,11 @@ __global__ void __launch_bounds__(kRThreads)
 // store issued between loads would hold every later wait for loaded data until the store
 // completes (vmcnt counts stores as well as loads), which cost the column route a third of
 // its time. A third change in one thread stores at once.
+__device__ __forceinline__ float4 ld_q(const float* p, int64_t q) {  // quad q of p, at any alignment
+    const vf4 v = ld_ntu(p + 4 * q);
+    return make_float4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ void st_q(float* p, int64_t q, float4 v) { st_ntu(p + 4 * q, vf4{v.x, v.y, v.z, v.w}); }
 struct PendingStores {
     int64_t q0 = 0, q1 = 0;
     float4 v0, v1;
@@ -1055,12 +1071,12 @@ struct PendingStores {
         } else if (n == 1) {
             q1 = q; v1 = v; n = 2;
         } else {
-            st_nt4(gr, q, v);
+            st_q(gr, q, v);
         }
     }
     __device__ __forceinline__ void flush(float* gr) const {
-        if (n > 0) st_nt4(gr, q0, v0);
-        if (n > 1) st_nt4(gr, q1, v1);
+        if (n > 0) st_q(gr, q0, v0);
+        if (n > 1) st_q(gr, q1, v1);
     }
 };
 // grad quad g plus add[j] where hit[j], else plus +0; queued when its bits change.
@@ -1149,9 +1165,9 @@ __global__ void __launch_bounds__(kRThreads)
     pd.flush(grad);
 }
 
-// Rows (C == 1, B % 4 == 0, 16-byte aligned grad and x): a block per chunk vr = r * S + s of
-// kRowChunk elements (the reduction's row chunks), two quads per thread; whether the chunk
-// reads x is uniform over the block.
+// Rows (C == 1): a block per chunk vr = r * S + s of kRowChunk elements (the reduction's row
+// chunks), two quads per thread and a row's last B % 4 elements one each; whether the chunk reads
+// x is uniform over the block.
 __global__ void __launch_bounds__(kRThreads)
     k_max_route_rows(float* __restrict__ grad, const float* __restrict__ x, const float* __restrict__ m,
                      const float* __restrict__ f, const float* __restrict__ ug, const float* __restrict__ pm,
@@ -1159,8 +1175,11 @@ __global__ void __launch_bounds__(kRThreads)
     const int64_t vr = blockIdx.x;
     const int64_t r = vr / S, s = vr - r * S;
     const int64_t rem = B - s * kRowChunk;
-    const int64_t nq = (rem < kRowChunk ? rem : kRowChunk) >> 2;
-    const int64_t q0 = (r * B + s * kRowChunk) >> 2;
+    const int64_t len = rem < kRowChunk ? rem : kRowChunk;
+    const int64_t nq = len >> 2;
+    const int64_t e0 = r * B + s * kRowChunk;
+    grad += e0;
+    x += e0;
     const float mr = m[r];
     const float ad = f[r] * ug[r];
     const float mv[4] = {mr, mr, mr, mr}, add[4] = {ad, ad, ad, ad};
@@ -1169,12 +1188,15 @@ __global__ void __launch_bounds__(kRThreads)
     const int t = threadIdx.x;
     static_assert(kRowChunk == 8 * kRThreads, "two quads per thread cover a chunk");
     const bool ha = t < nq, hb = t + kRThreads < nq;
-    const float4 ga = ha ? ld_nt4(grad, q0 + t) : z, gb = hb ? ld_nt4(grad, q0 + t + kRThreads) : z;
-    const float4 xa = ha && need ? ld_nt4(x, q0 + t) : z, xb = hb && need ? ld_nt4(x, q0 + t + kRThreads) : z;
+    const float4 ga = ha ? ld_q(grad, t) : z, gb = hb ? ld_q(grad, t + kRThreads) : z;
+    const float4 xa = ha && need ? ld_q(x, t) : z, xb = hb && need ? ld_q(x, t + kRThreads) : z;
+    const bool ht = t < (int)(len & 3);
+    const float gt = ht ? ld_nt(grad + 4 * nq + t) : 0.0f, xt = ht && need ? ld_nt(x + 4 * nq + t) : 0.0f;
     PendingStores pd;
-    if (ha) route_quad_x(pd, grad, q0 + t, ga, xa, need, mv, add);
-    if (hb) route_quad_x(pd, grad, q0 + t + kRThreads, gb, xb, need, mv, add);
+    if (ha) route_quad_x(pd, grad, t, ga, xa, need, mv, add);
+    if (hb) route_quad_x(pd, grad, t + kRThreads, gb, xb, need, mv, add);
     pd.flush(grad);
+    if (ht) st_nt(grad + 4 * nq + t, gt + (need && xt == mr ? ad : 0.0f));
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1213,7 +1235,7 @@ __device__ __forceinline__ float mom_std(const Mom& m, int64_t B) {
     return __builtin_sqrtf((float)v / (float)B);
 }
 
-// tstd over rows of B % 4 == 0, B <= 16384 elements: WPR waves per row, the row's quads
+// tstd over rows of B <= 16384 elements, of any length and alignment: WPR waves per row, the row's quads
 // loaded together, fp64 moments (above) summed per lane in quad order, then the butterfly and
 // the waves in order.
 template <int WPR, int NQ>
@@ -1225,27 +1247,19 @@ __global__ void __launch_bounds__(kRThreads)
     if (row >= nrows) return;  // WPR == 1: uniform per wave, and that path has no barrier
     const int tr = WPR == 1 ? lane : (int)threadIdx.x;
     constexpr int NT = 64 * WPR;
-    const int64_t Bq = B >> 2;
     const float* xr = x + row * B;
-    // the row's quads load before K is needed (a quad past the row loads the last quad, then
-    // holds K: x - K = 0 adds nothing to either moment), so K's load is not waited for first
+    // the row's quads load before K is needed (an element past the row becomes K: x - K = 0 adds
+    // nothing to either moment), so K's load is not waited for first
     vf4 v[NQ];
-#pragma unroll
-    for (int k = 0; k < NQ; ++k) {
-        const int64_t qi = tr + (int64_t)k * NT;
-        v[k] = ld_ntv(xr, qi < Bq ? qi : Bq - 1);
-    }
+    load_row_quads<NQ, NT>(v, xr, tr, B, row_edge(row, nrows, B), 0.0f);
     __builtin_amdgcn_sched_barrier(0);
     const float kf = xr[0];
     const double K = (double)kf;
-#pragma unroll
-    for (int k = 0; k < NQ; ++k)
-        if (tr + (int64_t)k * NT >= Bq) v[k] = vf4{kf, kf, kf, kf};
     Mom m{0.0, 0.0};
 #pragma unroll
     for (int k = 0; k < NQ; ++k)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) mom_add(m, v[k][j], K);
+        for (int j = 0; j < 4; ++j) mom_add(m, 4 * (tr + (int64_t)k * NT) + j < B ? v[k][j] : kf, K);
     m = mom_wave(m);
     if (WPR == 4) {
         if (lane == 0) ws[w] = m;
@@ -1259,10 +1273,9 @@ __global__ void __launch_bounds__(kRThreads)
     if (tr == 0) res[row] = mom_std(m, B);
 }
 
-// Rows: block vr = r * S + s sums elements [s * L, min((s + 1) * L, B)) of row r (VEC: two
-// quads per thread in flight), its four waves in order; S == 1 writes the row's result,
-// S > 1 the partial part[vr].
-template <bool VEC>
+// Rows: block vr = r * S + s sums elements [s * L, min((s + 1) * L, B)) of row r (whole quads
+// at any alignment, then the last len % 4 elements on the first threads), its four waves in
+// order; S == 1 writes the row's result, S > 1 the partial part[vr].
 __global__ void __launch_bounds__(kRThreads)
     k_tstd_mom_rows(float* __restrict__ res, const float* __restrict__ x, int64_t B, int64_t L, int64_t S,
                     Mom* __restrict__ part) {
@@ -1273,46 +1286,42 @@ __global__ void __launch_bounds__(kRThreads)
     const int64_t start = r * B + s * L;
     const int64_t rem = B - s * L;
     const int64_t len = rem < L ? rem : L;
-    Mom m{0.0, 0.0};
-    if (VEC) {
-        // four quads in flight; element j of every quad goes to accumulator chain j, and the
-        // chains are added in order (one chain had 16 dependent fp64 adds per pass of a
-        // 16384-element chunk: all-element tstd over 2^26 elements took 49.9 us)
-        const int64_t nq = len >> 2;
-        const float* xs = x + start;
-        // K (the row's first element) as a vector load, which the first quads' loads follow
-        // without waiting for it: a scalar load here was waited for before any of them issued
-        const float kf = __hip_atomic_load(x + r * B, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        Mom mc[4] = {Mom{0.0, 0.0}, Mom{0.0, 0.0}, Mom{0.0, 0.0}, Mom{0.0, 0.0}};
-        for (int64_t q = t; q < nq; q += 4 * kRThreads) {
-            // a quad past the chunk loads the chunk's last quad, then holds K: x - K = 0 adds
-            // nothing to either moment
-            vf4 v[4];
+    // four quads in flight; element j of every quad goes to accumulator chain j, and the
+    // chains are added in order (one chain had 16 dependent fp64 adds per pass of a
+    // 16384-element chunk: all-element tstd over 2^26 elements took 49.9 us)
+    const int64_t nq = len >> 2;
+    const float* xs = x + start;
+    // K (the row's first element) as a vector load, which the first quads' loads follow
+    // without waiting for it: a scalar load here was waited for before any of them issued
+    const float kf = __hip_atomic_load(x + r * B, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const float vt = t < (int)(len & 3) ? ld_nt(xs + 4 * nq + t) : 0.0f;
+    Mom mc[4] = {Mom{0.0, 0.0}, Mom{0.0, 0.0}, Mom{0.0, 0.0}, Mom{0.0, 0.0}};
+    for (int64_t q = t; q < nq; q += 4 * kRThreads) {
+        // a quad past the chunk loads the chunk's last quad, then holds K: x - K = 0 adds
+        // nothing to either moment
+        vf4 v[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int64_t qi = q + u * kRThreads;
-                v[u] = ld_ntv(xs, qi < nq ? qi : nq - 1);
-            }
-            float kq = kf;
-            asm volatile("" : "+v"(kq) : : "memory");  // K's wait and conversion after the loads above
-            const double K = (double)kq;
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (q + u * kRThreads >= nq) v[u] = vf4{kq, kq, kq, kq};
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) mom_add(mc[j], v[u][j], K);
+        for (int u = 0; u < 4; ++u) {
+            const int64_t qi = q + u * kRThreads;
+            v[u] = ld_ntu(xs + 4 * (qi < nq ? qi : nq - 1));
         }
-        m = mc[0];
+        float kq = kf;
+        asm volatile("" : "+v"(kq) : : "memory");  // K's wait and conversion after the loads above
+        const double K = (double)kq;
 #pragma unroll
-        for (int j = 1; j < 4; ++j) {
-            m.s1 = m.s1 + mc[j].s1;
-            m.s2 = m.s2 + mc[j].s2;
-        }
-    } else {
-        const double K = (double)x[r * B];
-        for (int64_t j = t; j < len; j += kRThreads) mom_add(m, ld_nt(x + start + j), K);
+        for (int u = 0; u < 4; ++u)
+            if (q + u * kRThreads >= nq) v[u] = vf4{kq, kq, kq, kq};
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) mom_add(mc[j], v[u][j], K);
+    }
+    if (t < (int)(len & 3)) mom_add(mc[0], vt, (double)kf);
+    Mom m = mc[0];
+#pragma unroll
+    for (int j = 1; j < 4; ++j) {
+        m.s1 = m.s1 + mc[j].s1;
+        m.s2 = m.s2 + mc[j].s2;
     }
     m = mom_wave(m);
     if (lane == 0) ws[w] = m;
@@ -1700,26 +1709,24 @@ static int reduce_t(LD ld, bool vec_ok, int epi, int64_t A, int64_t B, int64_t C
                                B, out, out2, epi, div);
             return MH_OK;
         }
-        const bool vec = vec_ok && B % 4 == 0;
-        if (!rows_chunked(B)) {  // one wavefront per row
-            dim3 g((unsigned)((A + 3) / 4)), b(kRThreads);
-            if (vec) hipLaunchKernelGGL((k_rows_wave<R, LD, true>), g, b, 0, st, ld, A, (int64_t)1, B, B, out, out2, epi, div, tmp);
-            else hipLaunchKernelGGL((k_rows_wave<R, LD, false>), g, b, 0, st, ld, A, (int64_t)1, B, B, out, out2, epi, div, tmp);
+        // one wavefront per row; the POW terms, which cost a log and an exp each, take a block
+        // (1023 elements: 11.5 us on one wavefront, 4.5 us)
+        if (!rows_chunked(B) && !std::is_same<LD, LdPowGrad>::value) {
+            hipLaunchKernelGGL((k_rows_wave<R, LD>), dim3((unsigned)((A + 3) / 4)), dim3(kRThreads), 0, st, ld, A, B,
+                               out, out2, epi, div);
             return MH_OK;
         }
         const int64_t S = row_chunks(B, combine);
         if (combine && S == 1 && A <= 0x7fffffff) {  // one block per row (k_row_comb)
-            dim3 g((unsigned)A), b(kCombThreads);
-            if (vec) hipLaunchKernelGGL((k_row_comb<R, LD, true>), g, b, 0, st, ld, B, out, out2, epi, div);
-            else hipLaunchKernelGGL((k_row_comb<R, LD, false>), g, b, 0, st, ld, B, out, out2, epi, div);
+            hipLaunchKernelGGL((k_row_comb<R, LD>), dim3((unsigned)A), dim3(kCombThreads), 0, st, ld, B, out, out2, epi,
+                               div);
             return MH_OK;
         }
         const int64_t L = S == 1 ? B : kRowChunk;
         const int64_t nv = A * S;
         if (split && S > 1) *split = RedSplit{S, L};
-        dim3 g((unsigned)nv), b(kRThreads);
-        if (vec) hipLaunchKernelGGL((k_rows_block<R, LD, true>), g, b, 0, st, ld, S, B, L, out, out2, epi, div, tmp, nv);
-        else hipLaunchKernelGGL((k_rows_block<R, LD, false>), g, b, 0, st, ld, S, B, L, out, out2, epi, div, tmp, nv);
+        hipLaunchKernelGGL((k_rows_block<R, LD>), dim3((unsigned)nv), dim3(kRThreads), 0, st, ld, S, B, L, out, out2,
+                           epi, div, tmp, nv);
         if (S > 1) {  // the chunk partials [A, S] reduce again along their rows
             using PL = PartLoader<R>;
             return reduce_t<R, typename PL::type>(PL::make(tmp, nv), true, epi, A, S, 1, out, out2, div,
@@ -2100,7 +2107,6 @@ static int binrg_reduce(float* grad, const float* ug, const float* a, const floa
         ld.fbc = make_fastdiv((uint32_t)(B * C > 0 ? B * C : 1));
         ld.fc = make_fastdiv((uint32_t)C);
     }
-    ld.al = al;
     if constexpr (!BIG && (COL1 || !DV)) {
         if (C == 1 && B <= 32 && al && A < kMaxGridRows) {  // short rows, staged as quads
             const unsigned blocks = (unsigned)((A + kLdsRows - 1) / kLdsRows);
@@ -2171,7 +2177,7 @@ int unbroadcast_binrg(int op, int id, bool divs, float* grad, const mh_shape& sg
     return MH_OK;
 }
 
-// The POW backward over whole aligned quads (LdPowGrad's terms, and with gx the x gradient) in
+// The POW backward over quads at any alignment (LdPowGrad's terms, and with gx the x gradient) in
 // one-shot one-wavefront blocks, every load issued before the first quad's log and exp work.
 // Each run of 64 quads (a quad per lane) adds into one partial the same way whatever the
 // launch shape: a lane adds its quad's four terms as ((0 + t0) + (0 + t1)) + ((0 + t2) + (0 + t3)),
@@ -2182,7 +2188,9 @@ int unbroadcast_binrg(int op, int id, bool divs, float* grad, const mh_shape& sg
 // four quads per thread, 0.73-0.75 ms for 256-thread blocks taking loads and work one quad at
 // a time).
 constexpr int kPowThreads = 64;
-constexpr int64_t kPowStreamMinQuads = 1 << 16;
+// Shorter tensors take one 256-thread block (at most two quads a thread, each a log and an exp an
+// element): one launch instead of two.
+constexpr int64_t kPowStreamMinQuads = 512;
 template <bool GX>
 constexpr int pow_runs() { return GX ? 1 : 2; }
 template <int NQ>
@@ -2198,9 +2206,9 @@ __device__ __forceinline__ void pow_load_quads(const LdPowGrad& ld, int64_t nq, 
     for (int k = 0; k < NQ; ++k) {
         const int64_t q = base + k * kPowThreads;
         const int64_t qc = q < nq ? q : nq - 1;
-        t.xs[k] = ld_nt4(ld.x, qc);
-        t.us[k] = ld_nt4(ld.ug, qc);
-        t.gs[k] = GX ? ld_nt4(ld.gx, qc) : make_float4(0.f, 0.f, 0.f, 0.f);
+        t.xs[k] = ld_q(ld.x, qc);
+        t.us[k] = ld_q(ld.ug, qc);
+        t.gs[k] = GX ? ld_q(ld.gx, qc) : make_float4(0.f, 0.f, 0.f, 0.f);
     }
 }
 
@@ -2241,16 +2249,18 @@ __device__ __forceinline__ void pow_block_quads(const LdPowGrad& ld, int64_t nq,
                 r3 = ld.elem<false, GX>(xq.w, uq.w, g.w);
             }
             s[k] = pow_quad_sum(r0, r1, r2, r3);
-            if constexpr (GX) st_nt4(ld.gx, q, g);
+            if constexpr (GX) st_q(ld.gx, q, g);
         }
     }
 }
 
 // The quads' loads go out before the exponent is read (setup): read first, every wave waited
-// for that scalar load before its quads' loads issued. part[r] is run r's sum, r < nruns.
+// for that scalar load before its quads' loads issued. part[r] is run r's sum, r < nruns; the last
+// n % 4 elements, where there are any, go to the first block's first thread and part[nruns].
 template <bool GX>
-__global__ void __launch_bounds__(kPowThreads) k_pow_grad_quads(LdPowGrad ld, int64_t nq, int64_t nruns,
+__global__ void __launch_bounds__(kPowThreads) k_pow_grad_quads(LdPowGrad ld, int64_t n, int64_t nruns,
                                                                 float* part) {
+    const int64_t nq = n >> 2;
     constexpr int NQ = pow_runs<GX>();
     PowQuads<NQ> t;
     pow_load_quads<GX, NQ>(ld, nq, t);
@@ -2265,34 +2275,39 @@ __global__ void __launch_bounds__(kPowThreads) k_pow_grad_quads(LdPowGrad ld, in
         const int64_t r = (int64_t)blockIdx.x * NQ + k;
         if (threadIdx.x == 0 && r < nruns) part[r] = a;
     }
+    if (blockIdx.x == 0 && threadIdx.x == 0 && (n & 3) != 0) {
+        float a = 0.0f;
+        for (int64_t i = nq << 2; i < n; ++i) a = a + ld.get(i);
+        part[nruns] = a;
+    }
 }
 
 int pow_exponent_grad(float* grad, const float* x, const float* exponent, const float* ug, int64_t n,
                       float* grad_x) {
     LdPowGrad ld{x, ug, exponent, 0.0f, grad_x, 0.0f, false};
-    const bool vec = al16(x) && al16(ug) && (!grad_x || al16(grad_x));
     float* tmp = nullptr;
-    if (vec && n % 4 == 0 && n / 4 >= kPowStreamMinQuads && n / 4 / kPowThreads < 0x7fffffff) {
+    if (n / 4 >= kPowStreamMinQuads && n / 4 / kPowThreads < 0x7fffffff) {
         // run partials, then a row reduction of them into grad
         const int64_t nq = n / 4;
         const int64_t G = (nq + kPowThreads - 1) / kPowThreads;  // runs of 64 quads
-        const size_t t = pad64((size_t)G) + tmp_floats_t<RSum>(1, G, 1, true);
+        const int64_t np = G + (n % 4 != 0 ? 1 : 0);
+        const size_t t = pad64((size_t)np) + tmp_floats_t<RSum>(1, np, 1, true);
         MH_TRY(scratch((t + 64) * sizeof(float), reinterpret_cast<void**>(&tmp)));
         if (grad_x) {
             constexpr int NQ = pow_runs<true>();
             hipLaunchKernelGGL(k_pow_grad_quads<true>, dim3((unsigned)((G + NQ - 1) / NQ)), dim3(kPowThreads), 0,
-                               ctx().stream, ld, nq, G, tmp);
+                               ctx().stream, ld, n, G, tmp);
         } else {
             constexpr int NQ = pow_runs<false>();
             hipLaunchKernelGGL(k_pow_grad_quads<false>, dim3((unsigned)((G + NQ - 1) / NQ)), dim3(kPowThreads), 0,
-                               ctx().stream, ld, nq, G, tmp);
+                               ctx().stream, ld, n, G, tmp);
         }
-        return reduce_t<RSum, LdPlain<RSum>>(LdPlain<RSum>{tmp}, true, EPI_ACCUM, 1, G, 1, grad, nullptr, 0.0f,
-                                             tmp + pad64((size_t)G), false, true);
+        return reduce_t<RSum, LdPlain<RSum>>(LdPlain<RSum>{tmp}, true, EPI_ACCUM, 1, np, 1, grad, nullptr, 0.0f,
+                                             tmp + pad64((size_t)np), false, true);
     }
     const size_t t = tmp_floats_t<RSum>(1, n, 1, true);
     MH_TRY(scratch((t + 64) * sizeof(float), reinterpret_cast<void**>(&tmp)));
-    return reduce_t<RSum, LdPowGrad>(ld, vec, EPI_ACCUM, 1, n, 1, grad, nullptr, 0.0f, tmp);
+    return reduce_t<RSum, LdPowGrad>(ld, true, EPI_ACCUM, 1, n, 1, grad, nullptr, 0.0f, tmp);
 }
 
 // elementwise helpers (mh_elementwise.hip)
@@ -2382,9 +2397,9 @@ int mh_tstd(float* res, const float* x, const mh_shape* psx, int32_t axis) {
     if (A * C == 0) return MH_OK;
     if (!res || (!x && B > 0)) return fail(MH_ERR_NULL, "mh_tstd: null tensor");
     MH_TRY(require_init());
-    if (C == 1 && B >= 4 && B % 4 == 0 && B <= 16384 && al16(x) && A < ((int64_t)1 << 31)) {
+    if (C == 1 && B >= 1 && B <= 16384 && A < ((int64_t)1 << 31)) {
         // rows held in registers: one pass over x
-        const int64_t Bq = B / 4;
+        const int64_t Bq = (B + 3) / 4;
         hipStream_t st = ctx().stream;
         if (Bq <= 64 * 16) {  // one wave per row, four rows per block
             const int nq = Bq <= 64 ? 1 : Bq <= 128 ? 2 : Bq <= 256 ? 4 : Bq <= 512 ? 8 : 16;
@@ -2418,10 +2433,7 @@ int mh_tstd(float* res, const float* x, const mh_shape* psx, int32_t axis) {
         if (S == 1) L = B;
         Mom* part = nullptr;
         if (S > 1) MH_TRY(scratch((size_t)(A * S) * sizeof(Mom), reinterpret_cast<void**>(&part)));
-        const bool vec = al16(x) && B % 4 == 0;
-        dim3 g((unsigned)(A * S)), b(kRThreads);
-        if (vec) hipLaunchKernelGGL(k_tstd_mom_rows<true>, g, b, 0, st, res, x, B, L, S, part);
-        else hipLaunchKernelGGL(k_tstd_mom_rows<false>, g, b, 0, st, res, x, B, L, S, part);
+        hipLaunchKernelGGL(k_tstd_mom_rows, dim3((unsigned)(A * S)), dim3(kRThreads), 0, st, res, x, B, L, S, part);
         if (S > 1)
             hipLaunchKernelGGL(k_tstd_mom_combine_rows, dim3((unsigned)A), dim3(kMomCombThreads), 0, st, res, part, S, B);
         return finish("mh_tstd");
@@ -2470,16 +2482,16 @@ int mh_tstd(float* res, const float* x, const mh_shape* psx, int32_t axis) {
 // not fit those kernels (the caller routes every element).
 static bool max_route_split(float* grad, const float* x, int64_t A, int64_t B, int64_t C, const float* m,
                             const float* f, const float* ug, float* tmp, const RedSplit& sp, bool arg) {
-    if (sp.S <= 1 || !al16(x) || !al16(grad)) return false;
+    if (sp.S <= 1) return false;
     hipStream_t st = ctx().stream;
     if (C == 1) {
         const int64_t nv = A * sp.S;
-        if (arg || B % 4 != 0 || sp.span != kRowChunk || nv > 0x7fffffff) return false;
+        if (arg || sp.span != kRowChunk || nv > 0x7fffffff) return false;
         hipLaunchKernelGGL(k_max_route_rows, dim3((unsigned)nv), dim3(kRThreads), 0, st, grad, x, m, f, ug, tmp,
                            sp.S, B);
         return true;
     }
-    if (!arg || C % 4 != 0 || sp.S > 65535) return false;
+    if (!arg || C % 4 != 0 || sp.S > 65535 || !al16(x) || !al16(grad)) return false;
     const int64_t np = sp.S * A * C;
     const uint32_t* pc = reinterpret_cast<const uint32_t*>(tmp + np);
     const uint32_t* pi = reinterpret_cast<const uint32_t*>(tmp + 2 * np);
@@ -2526,9 +2538,9 @@ int mh_reduce_bwd_accum(int op, float* grad, const float* x, const mh_shape* psx
         else
             hipLaunchKernelGGL(k_max_bwd_rows<32>, dim3(blocks), dim3(kLdsRows), 0, ctx().stream, grad, x, ug, A,
                                (int)B, fdB);
-    } else if (C == 1 && B % 4 == 0 && B <= 16384 && al16(x) && al16(grad) && A < ((int64_t)1 << 31)) {
+    } else if (C == 1 && B <= 16384 && A < ((int64_t)1 << 31)) {
         // MAX over rows held in registers: one pass
-        const int64_t Bq = B / 4;
+        const int64_t Bq = (B + 3) / 4;
         hipStream_t st = ctx().stream;
         if (Bq <= 64 * 16) {  // one wave per row, four rows per block
             const int nq = Bq <= 64 ? 1 : Bq <= 128 ? 2 : Bq <= 256 ? 4 : Bq <= 512 ? 8 : 16;

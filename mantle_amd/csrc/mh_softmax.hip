@@ -26,8 +26,8 @@
 //   64 < classes < 2048
 //                    k_rows_wave's order (per lane, quads lane + 64 q accumulated in groups
 //                    of four, the tail into the first group, the sixteen partials summed in
-//                    order, then an xor butterfly; lane-strided elements when classes is not
-//                    a multiple of 4): one wavefront per row, the row across its lanes.
+//                    order, then an xor butterfly; the last classes % 4 elements on the lane
+//                    after the last quad): one wavefront per row, the row across its lanes.
 // Only the all-element sum of a loss graph (MEAN or SUM) runs in another order (the rtol
 // class).
 //
@@ -811,12 +811,13 @@ __global__ void __launch_bounds__(kORows)
 // ---------------------------------------------------------------------------------------
 // wavefront engine: 64 < classes <= 2047, one wavefront per row, k_rows_wave's order
 // ---------------------------------------------------------------------------------------
-// Lane slot i holds element 4 (lane + 64 (i / 4)) + i % 4 (VEC: classes % 4 == 0, quads
-// lane + 64 q) or lane + 64 i (otherwise).
-template <bool VEC>
-__device__ __forceinline__ int slot_elem(int lane, int i) {
-    return VEC ? 4 * (lane + 64 * (i >> 2)) + (i & 3) : lane + 64 * i;
-}
+// A row on LPR lanes (64, or 32 for rows of up to 128 classes, two rows to a wavefront: the lanes
+// of the upper half would hold only values that add nothing, so every sum keeps its bits). Lane
+// slot i holds element 4 (lane + 64 (i / 4)) + i % 4: the row's quads lane, lane + 64, ..., the
+// last one with the row's last K % 4 elements. VEC: K % 4 == 0. NE: the slots, no more than the
+// class count needs (with 16 for every row of up to 1024 classes, and one row per wavefront, the
+// CrossEntropy forward and backward over [100000, 68] took 160 us, now 43 us).
+__device__ __forceinline__ int slot_elem(int lane, int i) { return 4 * (lane + 64 * (i >> 2)) + (i & 3); }
 
 struct OpAdd {
     __device__ float operator()(float a, float b) const { return a + b; }
@@ -825,136 +826,143 @@ struct OpMax {
     __device__ float operator()(float a, float b) const { return a > b ? a : b; }
 };
 
-// One row's reduction in the order of k_rows_wave<R, LD, VEC> with a single chunk.
-template <bool VEC, int NE, class OP>
+// Whether slot i holds an element of the row. NE is the least of its sizes that K needs, so the
+// first half of the slots always do (K > 64 NE / 2 for NE >= 8), known when compiling.
+template <int NE>
+__device__ __forceinline__ bool slot_live(int lane, int i, int K) {
+    return (i >> 2) < NE / 8 || slot_elem(lane, i) < K;
+}
+
+// One row's reduction in the order of k_rows_wave. Slots past the row are passed over by selects:
+// a branch on each cost more than the work it saved.
+template <bool VEC, int NE, int LPR, class OP>
 __device__ __forceinline__ float wave_row_reduce(const float* v, int lane, int K, float init, OP op) {
-    float acc = init;
-    if constexpr (VEC) {
-        constexpr int NQ = NE / 4;
-        const int nq = K >> 2;
-        float a4[4][4];
+    constexpr int NQ = NE / 4;
+    const int nq = K >> 2;
+    float a4[4][4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < 4; ++u)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) a4[u][j] = init;
-        int done = 0;  // quads taken by the four-quad main loop (a prefix of the groups)
+        for (int j = 0; j < 4; ++j) a4[u][j] = init;
+    auto rest = [&](int q) {  // quad q into the first group
 #pragma unroll
-        for (int q0 = 0; q0 + 3 < NQ; q0 += 4) {
-            if (lane + 64 * (q0 + 3) < nq) {
+        for (int j = 0; j < 4; ++j) {
+            const float w = op(a4[0][j], v[q * 4 + j]);
+            a4[0][j] = slot_live<NE>(lane, VEC ? 4 * q : 4 * q + j, K) ? w : a4[0][j];
+        }
+    };
+    if constexpr (NQ < 4) {
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) rest(q);
+    } else {
+#pragma unroll
+        for (int q0 = 0; q0 < NQ; q0 += 4) {
+            if (lane + 64 * (q0 + 3) < nq) {  // four whole quads, one to each group
 #pragma unroll
                 for (int u = 0; u < 4; ++u)
 #pragma unroll
                     for (int j = 0; j < 4; ++j) a4[u][j] = op(a4[u][j], v[(q0 + u) * 4 + j]);
-                done = q0 + 4;
+            } else {  // the row's rest, its last K % 4 elements among them
+#pragma unroll
+                for (int u = 0; u < 4; ++u) rest(q0 + u);
             }
         }
+    }
+    float acc = init;
 #pragma unroll
-        for (int q = 0; q < NQ; ++q) {
-            if (q >= done && lane + 64 * q < nq) {
+    for (int u = 0; u < (NQ < 4 ? 1 : 4); ++u)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) a4[0][j] = op(a4[0][j], v[q * 4 + j]);
-            }
-        }
+        for (int j = 0; j < 4; ++j) acc = op(acc, a4[u][j]);
+    if constexpr (NQ < 4) {  // the other groups, which hold only init
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc = op(acc, a4[u][j]);
-    } else {
-#pragma unroll
-        for (int i = 0; i < NE; ++i)
-            if (lane + 64 * i < K) acc = op(acc, v[i]);
+        for (int u = 0; u < 12; ++u) acc = op(acc, init);
     }
 #pragma unroll
-    for (int mm = 32; mm >= 1; mm >>= 1) acc = op(acc, __shfl_xor(acc, mm));
+    for (int mm = LPR / 2; mm >= 1; mm >>= 1) acc = op(acc, __shfl_xor(acc, mm));
     return acc;
 }
 
-template <bool VEC, int NE>
-__device__ __forceinline__ void load_row(float* v, const float* __restrict__ src, int lane, int K, bool al) {
-    if (VEC && al) {
+// A row into its lanes' slots, as quads at any alignment: rows of an odd length went one element
+// per lane (CrossEntropy over [32768, 1001]: 154 us, 130 us in quads). A slot past the row loads
+// the row's last quad again (no branch around a load) and is never used. A quad that runs past
+// the row reads on into the next one; `edge` marks the tensor's last rows, where it would leave
+// the tensor.
+template <bool VEC, int NE, int LPR>
+__device__ __forceinline__ void load_row(float* v, const float* __restrict__ src, int lane, int K, bool edge) {
+    if (VEC || !edge) {
+        const int last = (K - 1) & ~3;
 #pragma unroll
         for (int q = 0; q < NE / 4; ++q) {
-            const int qi = lane + 64 * q;
-            if (4 * qi < K) {
-                const float4 f = ld_nt4(src, qi);
-                v[4 * q] = f.x;
-                v[4 * q + 1] = f.y;
-                v[4 * q + 2] = f.z;
-                v[4 * q + 3] = f.w;
-            } else {
-                v[4 * q] = v[4 * q + 1] = v[4 * q + 2] = v[4 * q + 3] = 0.0f;
-            }
+            const int e = slot_elem(lane, 4 * q);
+            const vf4 f = ld_ntu(src + (slot_live<NE>(lane, 4 * q, K) ? e : last));
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[4 * q + j] = f[j];
         }
     } else {
 #pragma unroll
-        for (int i = 0; i < NE; ++i) {
-            const int k = slot_elem<VEC>(lane, i);
-            v[i] = k < K ? ld_nt(src + k) : 0.0f;
-        }
+        for (int i = 0; i < NE; ++i) v[i] = slot_elem(lane, i) < K ? ld_nt(src + slot_elem(lane, i)) : 0.0f;
     }
 }
 
-template <bool VEC, int NE>
-__device__ __forceinline__ void store_row(float* __restrict__ dst, const float* v, int lane, int K, bool al) {
-    if (VEC && al) {
+template <bool VEC, int NE, int LPR>
+__device__ __forceinline__ void store_row(float* __restrict__ dst, const float* v, int lane, int K) {
 #pragma unroll
-        for (int q = 0; q < NE / 4; ++q) {
-            const int qi = lane + 64 * q;
-            if (4 * qi < K)
-                st_nt4(dst, qi, make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]));
-        }
-    } else {
+    for (int q = 0; q < NE / 4; ++q) {
+        const int e = slot_elem(lane, 4 * q);
+        if (VEC ? e < K : e + 3 < K) {
+            st_ntu(dst + e, vf4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]});
+        } else if (!VEC) {
 #pragma unroll
-        for (int i = 0; i < NE; ++i) {
-            const int k = slot_elem<VEC>(lane, i);
-            if (k < K) st_nt(dst + k, v[i]);
+            for (int j = 0; j < 3; ++j)
+                if (e + j < K) st_nt(dst + e + j, v[4 * q + j]);
         }
     }
 }
 
 // Row max (MAX.forward's order), e = exp(x - m) and s = sum e (SUM.forward's order).
-template <bool VEC, int NE>
+template <bool VEC, int NE, int LPR>
 __device__ __forceinline__ void wave_row_softmax(const float* xv, float* e, int lane, int K, float* m_out,
                                                  float* s_out) {
-    const float m = wave_row_reduce<VEC, NE>(xv, lane, K, -FLT_MAX, OpMax{});
+    const float m = wave_row_reduce<VEC, NE, LPR>(xv, lane, K, -FLT_MAX, OpMax{});
 #pragma unroll
-    for (int i = 0; i < NE; ++i) e[i] = slot_elem<VEC>(lane, i) < K ? mexp(xv[i] - m) : 0.0f;
+    for (int i = 0; i < NE; ++i) e[i] = mexp(xv[i] - m);
     *m_out = m;
-    *s_out = wave_row_reduce<VEC, NE>(e, lane, K, 0.0f, OpAdd{});
+    *s_out = wave_row_reduce<VEC, NE, LPR>(e, lane, K, 0.0f, OpAdd{});
 }
 
-template <int V, bool VEC, int NE>
+template <int V, bool VEC, int NE, int LPR>
 __global__ void __launch_bounds__(kSThreads)
     k_roww_fwd(const float* __restrict__ x, const float* __restrict__ tg, float* __restrict__ out, int64_t rows,
-               int K, bool al, float* __restrict__ part) {
+               int K, float* __restrict__ part) {
     __shared__ float ws[4];
     constexpr bool LOSS = V == G_SMLM || V == G_CE;
-    const int lane = threadIdx.x & 63;
-    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & (LPR - 1);
+    const int64_t row = (int64_t)blockIdx.x * (kSThreads / LPR) + threadIdx.x / LPR;
     float rowsum = 0.0f;
-    if (row < rows) {  // uniform per wavefront
+    if (row < rows) {  // uniform over a row's lanes
         const int64_t base = row * (int64_t)K;
-        float xv[NE], e[NE];
-        load_row<VEC, NE>(xv, x + base, lane, K, al);
+        const bool edge = row_edge(row, rows, K);
+        float xv[NE], e[NE], tv[LOSS ? NE : 1];
+        load_row<VEC, NE, LPR>(xv, x + base, lane, K, edge);
+        if constexpr (LOSS) load_row<VEC, NE, LPR>(tv, tg + base, lane, K, edge);
         float m, s;
-        wave_row_softmax<VEC, NE>(xv, e, lane, K, &m, &s);
+        wave_row_softmax<VEC, NE, LPR>(xv, e, lane, K, &m, &s);
         const float ls = (V == G_CE || V == G_LOGSOFTMAX) ? mlog(s) : 0.0f;
         if constexpr (LOSS) {
-            float tv[NE];
-            load_row<VEC, NE>(tv, tg + base, lane, K, al);
 #pragma unroll
             for (int i = 0; i < NE; ++i) {
-                if (slot_elem<VEC>(lane, i) < K) {
-                    if constexpr (V == G_SMLM) {
-                        if (!smlm_skip(tv[i], e[i])) rowsum = rowsum + mlog(e[i] / s) * tv[i];
-                    }
-                    else rowsum = rowsum + tv[i] * ((xv[i] - m) - ls);
+                const bool live = slot_live<NE>(lane, VEC ? i & ~3 : i, K);
+                if constexpr (V == G_SMLM) {
+                    if (live && !smlm_skip(tv[i], e[i])) rowsum = rowsum + mlog(e[i] / s) * tv[i];
+                } else {
+                    const float w = rowsum + tv[i] * ((xv[i] - m) - ls);
+                    rowsum = live ? w : rowsum;
                 }
             }
         } else {
 #pragma unroll
             for (int i = 0; i < NE; ++i) xv[i] = V == G_SOFTMAX ? e[i] / s : (xv[i] - m) - ls;
-            store_row<VEC, NE>(out + base, xv, lane, K, al);
+            store_row<VEC, NE, LPR>(out + base, xv, lane, K);
         }
     }
     if constexpr (LOSS) {  // every wavefront reaches the barrier
@@ -963,35 +971,38 @@ __global__ void __launch_bounds__(kSThreads)
     }
 }
 
-template <int V, bool VEC, int NE>
-__global__ void __launch_bounds__(kSThreads)
+// WPE caps the wavefronts per SIMD: whole-quad rows of nearly 1024 classes stream best with three
+// (CrossEntropy over [32768, 1000] 130.2 us for both passes without a cap, 127.4 with four,
+// 125.7 with three); at 520 classes the cap costs 6 %, at 768 1 %.
+template <int V, bool VEC, int NE, int LPR, int WPE>
+__global__ void __launch_bounds__(kSThreads) __attribute__((amdgpu_waves_per_eu(1, WPE)))
     k_roww_bwd(float* __restrict__ g, const float* __restrict__ x, const float* __restrict__ up,
-               const float* __restrict__ ug, int64_t rows, int K, bool al, float c) {
-    const int lane = threadIdx.x & 63;
-    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (row >= rows) return;  // uniform per wavefront; no block barrier below
+               const float* __restrict__ ug, int64_t rows, int K, float c) {
+    const int lane = threadIdx.x & (LPR - 1);
+    const int64_t row = (int64_t)blockIdx.x * (kSThreads / LPR) + threadIdx.x / LPR;
+    if (row >= rows) return;  // uniform over a row's lanes; no block barrier below
     const int64_t base = row * (int64_t)K;
+    const bool edge = row_edge(row, rows, K);
     float xv[NE], e[NE], pre[NE], tmp[NE];
-    load_row<VEC, NE>(xv, x + base, lane, K, al);
+    load_row<VEC, NE, LPR>(xv, x + base, lane, K, edge);
+    load_row<VEC, NE, LPR>(tmp, up + base, lane, K, edge);
     float m, s;
-    wave_row_softmax<VEC, NE>(xv, e, lane, K, &m, &s);
+    wave_row_softmax<VEC, NE, LPR>(xv, e, lane, K, &m, &s);
     // the max with its count, as MAX.backward recomputes it (lane order, then a butterfly)
     float mb = -FLT_MAX;
     uint32_t cntm = 0;
 #pragma unroll
     for (int i = 0; i < NE; ++i) {
-        if (slot_elem<VEC>(lane, i) < K) {
-            const float v = xv[i];
-            max_count_add(mb, cntm, v);  // a NaN element is not counted
-        }
+        // a NaN element is not counted; neither is a slot past the row, taken as NaN
+        const float v = slot_live<NE>(lane, VEC ? i & ~3 : i, K) ? xv[i] : __builtin_nanf("");
+        max_count_add(mb, cntm, v);
     }
 #pragma unroll
-    for (int mm = 32; mm >= 1; mm >>= 1) {
+    for (int mm = LPR / 2; mm >= 1; mm >>= 1) {
         const float om = __shfl_xor(mb, mm);
         const uint32_t oc = (uint32_t)__shfl_xor((int)cntm, mm);
         max_count_merge(mb, cntm, om, oc);
     }
-    load_row<VEC, NE>(tmp, up + base, lane, K, al);
     const float gconst = V == G_SMLM ? 0.0f + c * ug[0] : V == G_CE ? 0.0f + 1.0f * (0.0f + ug[0] * c) : 0.0f;
     float gS;
     if constexpr (from_softmax<V>()) {
@@ -999,7 +1010,7 @@ __global__ void __launch_bounds__(kSThreads)
         const bool skip_ok = V == G_SMLM && gconst - gconst == 0.0f;
 #pragma unroll
         for (int i = 0; i < NE; ++i) {
-            if (skip_ok && (slot_elem<VEC>(lane, i) >= K || smlm_skip(tmp[i], e[i]))) {
+            if (skip_ok && smlm_skip(tmp[i], e[i])) {
                 pre[i] = 0.0f;  // the values of the full expression (slots past the row are unused)
                 tmp[i] = -0.0f;
             } else {
@@ -1008,7 +1019,7 @@ __global__ void __launch_bounds__(kSThreads)
                 tmp[i] = ((-e[i]) / s2) * gsm;
             }
         }
-        gS = 0.0f + wave_row_reduce<VEC, NE>(tmp, lane, K, 0.0f, OpAdd{});
+        gS = 0.0f + wave_row_reduce<VEC, NE, LPR>(tmp, lane, K, 0.0f, OpAdd{});
     } else {
 #pragma unroll
         for (int i = 0; i < NE; ++i) {
@@ -1016,7 +1027,7 @@ __global__ void __launch_bounds__(kSThreads)
             pre[i] = 0.0f + glsm;
             tmp[i] = glsm;
         }
-        gS = 0.0f + (0.0f + (-wave_row_reduce<VEC, NE>(tmp, lane, K, 0.0f, OpAdd{}))) / s;
+        gS = 0.0f + (0.0f + (-wave_row_reduce<VEC, NE, LPR>(tmp, lane, K, 0.0f, OpAdd{}))) / s;
     }
     const float rgs = 1.0f * gS;
 #pragma unroll
@@ -1024,11 +1035,11 @@ __global__ void __launch_bounds__(kSThreads)
         if constexpr (from_softmax<V>()) pre[i] = 0.0f + e[i] * (pre[i] + rgs);
         else pre[i] = pre[i] + e[i] * (0.0f + rgs);
     }
-    const float sg = (1.0f / (float)cntm) * (0.0f + (-wave_row_reduce<VEC, NE>(pre, lane, K, 0.0f, OpAdd{})));
-    load_row<VEC, NE>(tmp, g + base, lane, K, al);
+    const float sg = (1.0f / (float)cntm) * (0.0f + (-wave_row_reduce<VEC, NE, LPR>(pre, lane, K, 0.0f, OpAdd{})));
+    load_row<VEC, NE, LPR>(tmp, g + base, lane, K, edge);
 #pragma unroll
     for (int i = 0; i < NE; ++i) tmp[i] = (tmp[i] + pre[i]) + (xv[i] == mb ? sg : 0.0f);
-    store_row<VEC, NE>(g + base, tmp, lane, K, al);
+    store_row<VEC, NE, LPR>(g + base, tmp, lane, K);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1509,18 +1520,21 @@ static int launch_fwd(const float* x, const float* tg, float* out, int64_t rows,
 #undef MH_RT
         return MH_OK;
     }
-    const int64_t nb = (rows + 3) / 4;
+    const int rpb = K <= 128 ? kSThreads / 32 : kSThreads / 64;
+    const int64_t nb = (rows + rpb - 1) / rpb;
     if (nb > 0x7fffffff) return fail(MH_ERR_OVERFLOW, "too many rows");
     *nblocks_out = nb;
     dim3 g((unsigned)nb), b(kSThreads);
-#define MH_RW(VEC, NE) hipLaunchKernelGGL((k_roww_fwd<V, VEC, NE>), g, b, 0, st, x, tg, out, rows, K, al, part)
-    if (K % 4 == 0) {
-        if (K <= 1024) MH_RW(true, 16);
-        else MH_RW(true, kSLaneElems);
-    } else {
-        if (K <= 1024) MH_RW(false, 16);
-        else MH_RW(false, kSLaneElems);
-    }
+#define MH_RW(NE, LPR)                                                                                         \
+    do {                                                                                                       \
+        if (K % 4 == 0) hipLaunchKernelGGL((k_roww_fwd<V, true, NE, LPR>), g, b, 0, st, x, tg, out, rows, K, part); \
+        else hipLaunchKernelGGL((k_roww_fwd<V, false, NE, LPR>), g, b, 0, st, x, tg, out, rows, K, part);            \
+    } while (0)
+    if (K <= 128) MH_RW(4, 32);
+    else if (K <= 256) MH_RW(4, 64);
+    else if (K <= 512) MH_RW(8, 64);
+    else if (K <= 1024) MH_RW(16, 64);
+    else MH_RW(kSLaneElems, 64);
 #undef MH_RW
     return MH_OK;
 }
@@ -1583,16 +1597,25 @@ static int launch_bwd(float* gx, const float* x, const float* up, const float* u
 #undef MH_RT
         return MH_OK;
     }
-    const int64_t nb = (rows + 3) / 4;
+    const int rpb = K <= 128 ? kSThreads / 32 : kSThreads / 64;
+    const int64_t nb = (rows + rpb - 1) / rpb;
     if (nb > 0x7fffffff) return fail(MH_ERR_OVERFLOW, "too many rows");
     dim3 g((unsigned)nb), b(kSThreads);
-#define MH_RW(VEC, NE) hipLaunchKernelGGL((k_roww_bwd<V, VEC, NE>), g, b, 0, st, gx, x, up, ug, rows, K, al, c)
+#define MH_RW(VEC, NE, LPR, WPE) \
+    hipLaunchKernelGGL((k_roww_bwd<V, VEC, NE, LPR, WPE>), g, b, 0, st, gx, x, up, ug, rows, K, c)
     if (K % 4 == 0) {
-        if (K <= 1024) MH_RW(true, 16);
-        else MH_RW(true, kSLaneElems);
+        if (K <= 128) MH_RW(true, 4, 32, 8);
+        else if (K <= 256) MH_RW(true, 4, 64, 8);
+        else if (K <= 512) MH_RW(true, 8, 64, 8);
+        else if (K <= 832) MH_RW(true, 16, 64, 8);
+        else if (K <= 1024) MH_RW(true, 16, 64, 3);
+        else MH_RW(true, kSLaneElems, 64, 8);
     } else {
-        if (K <= 1024) MH_RW(false, 16);
-        else MH_RW(false, kSLaneElems);
+        if (K <= 128) MH_RW(false, 4, 32, 8);
+        else if (K <= 256) MH_RW(false, 4, 64, 8);
+        else if (K <= 512) MH_RW(false, 8, 64, 8);
+        else if (K <= 1024) MH_RW(false, 16, 64, 8);
+        else MH_RW(false, kSLaneElems, 64, 8);
     }
 #undef MH_RW
     return MH_OK;

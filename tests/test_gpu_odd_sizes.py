@@ -1,0 +1,101 @@
+"""Rows and columns of every length modulo 4 and at every 4-byte alignment: the kernels move them as
+unaligned quads, the last few elements of a line apart. Lines at the edges of the kernels' ranges
+against the oracle, and views of a larger tensor (offsets of 1-3 floats) against the same values
+at an aligned address."""
+import numpy as np
+import pytest
+
+from mantle_amd import synth
+from util import O, OPS, GpuEngine, Graph, OracleEngine, assert_bitexact, assert_sum_close, softmax_nodes
+
+pytestmark = pytest.mark.gpu
+ORC = OracleEngine()
+SUM, MEAN, MAX = OPS["SUM"], OPS["MEAN"], OPS["MAX"]
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    return GpuEngine()
+
+
+@pytest.fixture(autouse=True)
+def _nelts():
+    O.set_nelts(32)
+    yield
+
+
+def view(gpu, a, off):
+    """`a` at `off` floats past an aligned address, with nothing after its last element's quad."""
+    buf = gpu.T(np.concatenate([np.full(off, 7.0, np.float32), np.asarray(a, np.float32).reshape(-1)]))
+    return gpu.m.Tensor(gpu.m.TensorShape(*np.asarray(a).shape), _ptr=buf.ptr + 4 * off, _owner=buf)
+
+
+def reductions_match(gpu, shape, axis, off=0):
+    """SUM, MEAN, MAX forward and backward, and tstd, of one shape against the oracle; x holds
+    ties, the gradient -0, +0 and NaN (the sums go by the condition of their terms)."""
+    m = gpu.m
+    x = synth.normal(shape, 0, 1, 2100)
+    if shape[axis] > 2:
+        synth.inject_ties(x, axis, 2101)
+    red = tuple(1 if i == axis else d for i, d in enumerate(shape))
+    ug = synth.normal(red, 0, 1, 2102)
+    g0 = synth.normal(shape, 0, 1, 2103).reshape(-1)
+    g0[::3], g0[1::7], g0[2::11] = np.float32(-0.0), np.float32(0.0), np.float32(np.nan)
+    g0 = g0.reshape(shape)
+    tx, tu = view(gpu, x, off), view(gpu, ug, off)
+    x64 = x.astype(np.float64)
+    for op, ex, mag in ((SUM, x64.sum(axis=axis, keepdims=True), np.abs(x64).sum(axis=axis, keepdims=True)),
+                        (MEAN, x64.mean(axis=axis, keepdims=True), np.abs(x64).mean(axis=axis, keepdims=True)),
+                        (MAX, None, None)):
+        res, g = view(gpu, np.zeros(red, np.float32), off), view(gpu, g0, off)
+        m.forward_op(op, res, tx, attributes={"axis": axis})
+        ref = ORC.forward(op, x, axis=axis)
+        if op == MAX:
+            assert np.array_equal(res.to_numpy(), ref)  # equal as floats: a zero tie's sign follows the order
+        else:
+            assert_sum_close(res.to_numpy(), ref, ex, f"{shape} axis {axis} op {op}", terms_abs=mag)
+        m.backward_op(0, op, tu, tx, None, g, attributes={"axis": axis})
+        assert_bitexact(g.to_numpy(), ORC.backward(0, op, ug, x, axis=axis, grad=g0), f"{shape} axis {axis} op {op} bwd")
+    assert_sum_close(m.tstd(tx, axis).to_numpy(), ORC.tstd(x, axis), x64.std(axis=axis, keepdims=True),
+                     f"tstd {shape} axis {axis}")
+
+
+@pytest.mark.parametrize("off", [0, 1, 3])
+@pytest.mark.parametrize("b", [1, 2, 5, 33, 65, 67, 255, 257, 1021, 1023, 1026, 2047, 2049, 2051, 4095, 8191, 16383,
+                               16385, 20479])
+def test_rows(gpu, b, off):
+    """Last-axis lines: the short-row tiles, one wavefront, rows in registers and chunks of 2048."""
+    reductions_match(gpu, (5, b), 1, off)
+
+
+@pytest.mark.parametrize("n", [262145, 262146 + 4 * 2048, 1 << 20, (1 << 20) + 3])
+def test_every_element(gpu, n):
+    """All elements as one row of chunks, whose last one is ragged."""
+    x = synth.normal((n,), 0, 1, 2110)
+    x[n // 2] = x[n - 1] = np.float32(9.0)
+    x64 = x.astype(np.float64)
+    assert_sum_close(gpu.forward(SUM, x), ORC.forward(SUM, x), np.array([x64.sum()]), terms_abs=np.array([np.abs(x64).sum()]))
+    assert np.array_equal(gpu.forward(MAX, x), ORC.forward(MAX, x))
+    ug = np.array([0.75], np.float32)
+    assert_bitexact(gpu.backward(0, MAX, ug, x), ORC.backward(0, MAX, ug, x), "MAX bwd")
+    assert_sum_close(gpu.tstd(x), ORC.tstd(x), np.array([x64.std()]), "tstd")
+
+
+@pytest.mark.parametrize("off", [0, 2])
+@pytest.mark.parametrize("rows,classes", [(1, 65), (2, 66), (3, 67), (9, 127), (8, 128), (5, 129), (3, 131), (4, 255),
+                                          (5, 256), (5, 257), (3, 511), (2, 513), (7, 832), (3, 836), (1, 1021),
+                                          (2, 1022), (3, 1023), (2, 1024), (1, 1025), (2, 2045), (1, 2047)])
+def test_softmax_rows(gpu, rows, classes, off):
+    """Fused Softmax at the class counts where the lanes per row and the elements per lane change,
+    and at the tensor's last row, whose last quad would leave it: bit for bit the op-by-op graph."""
+    m = gpu.m
+    x, gout = synth.normal((rows, classes), 0, 2, 2120), synth.normal((rows, classes), 0, 1, 2121)
+    g0 = synth.normal((rows, classes), 0, 1, 2122)
+    g = Graph(softmax_nodes("x", 1), ["x"])
+    v = g.forward(gpu, {"x": x})
+    gr = g.backward(gpu, v, seed=gout, init={"x": g0})
+    out, tg, tx = view(gpu, np.zeros_like(x), off), view(gpu, g0, off), view(gpu, x, off)
+    m.softmax_forward(out, tx)
+    m.softmax_backward(tg, tx, view(gpu, gout, off))
+    assert_bitexact(out.to_numpy(), v["sm"], "softmax")
+    assert_bitexact(tg.to_numpy(), gr["x"], "softmax backward")
