@@ -9,14 +9,15 @@
 //                     butterfly shuffle;
 //   C == 1, B >= 2048: 2048-element chunks, one 4-wave block each (two quads per thread),
 //                     whose partials reduce again along the row the same way;
-//   C  > 1, C % 4 == 0 and >= 1024 columns: one thread per column quad over a split of the
-//                     rows (about four blocks per CU; splits on grid x), the split partials
-//                     combined in one short launch (k_parts_comb);
-//   C  > 1, C % 4 == 0 and >= 128 columns: a block per (strip of 64 column quads, split of
-//                     rows), its four waves interleaving the rows, combined through LDS;
-//   C  > 1 otherwise  : one thread per output column (a quad of columns when C % 4 == 0);
+//   C  >= 1024      : one thread per column quad over a split of the rows (about four blocks
+//                     per CU; splits on grid x);
+//   C  >= 128       : a block per (strip of 64 column quads, split of rows), its four waves
+//                     interleaving the rows, combined through LDS;
+//   C  > 1 otherwise: one thread per column quad (below 4 columns: per column);
 //   in every column form the rows split across blocks when that is needed to fill the chip,
-//   and a second pass combines the split partials in fixed split order.
+//   and one short launch combines the split partials in fixed order (k_parts_comb). Column
+//   quads are at any alignment; the last quad of a slab whose C is not a multiple of 4 starts
+//   at column C - 4 and writes only the columns the quad before it leaves (col_quad).
 // No atomics: each output's summation order is fixed by the launch shape, so a call repeated
 // on the same input returns the same bits.
 // MAX backward over axis 0 and all elements routes from the split partials its max-count
@@ -661,8 +662,16 @@ __global__ void __launch_bounds__(kRThreads)
     epi_store(out, out2, o, acc, epi, div);
 }
 
-// Column reduction: item = a quad (VEC) or one element of the flattened [A, C] output; the
-// rows [b0, b1) of split blockIdx.y. S == 1 writes the epilogue, S > 1 writes partials at
+// Column quad cq of a slab of C >= 4 columns: its first column c and the first of its four
+// elements that is its own (lo > 0 only in the last quad of a C that is not a multiple of 4).
+__device__ __forceinline__ void col_quad(int64_t cq, int64_t C, int64_t* c, int* lo) {
+    const int64_t c4 = 4 * cq;
+    *c = c4 + 4 <= C ? c4 : C - 4;
+    *lo = (int)(c4 - *c);
+}
+
+// Column reduction: item = a column quad (VEC, C >= 4) or one column of slab a of the [A, C]
+// output; the rows [b0, b1) of one split. S == 1 writes the epilogue, S > 1 writes partials at
 // s * (A * C) + o.
 template <class R, class LD, bool VEC, bool SPLIT_X = false>
 __global__ void __launch_bounds__(kRThreads)
@@ -671,11 +680,14 @@ __global__ void __launch_bounds__(kRThreads)
     ld.setup();
     using T = typename R::T;
     constexpr int W = VEC ? 4 : 1;
-    const int64_t AC = A * C;
+    const int64_t AC = A * C, CW = VEC ? (C + 3) >> 2 : C;
     const int64_t item = (int64_t)(SPLIT_X ? blockIdx.y : blockIdx.x) * kRThreads + threadIdx.x;
-    const int64_t o = item * W;
-    if (o >= AC) return;
-    const int64_t a = o / C, c = o - a * C;
+    if (item >= A * CW) return;
+    const int64_t a = item / CW;
+    int64_t c = item - a * CW;
+    int lo = 0;
+    if (VEC) col_quad(c, C, &c, &lo);
+    const int64_t o = a * C + c;
     const int64_t s = SPLIT_X ? blockIdx.x : blockIdx.y;
     const int64_t b0 = s * rps;
     const int64_t b1 = (b0 + rps < B) ? b0 + rps : B;
@@ -706,6 +718,7 @@ __global__ void __launch_bounds__(kRThreads)
     }
 #pragma unroll
     for (int j = 0; j < W; ++j) {
+        if (VEC && j < lo) continue;
         if (S == 1) epi_store(out, out2, o + j, acc[j], epi, div);
         else part_store2(part, S * AC, s * AC + o + j, acc[j]);
     }
@@ -752,53 +765,61 @@ __global__ void __launch_bounds__(kCombThreads)
     }
 }
 
-// Combine of S split partials [S, n] (n % 4 == 0) in one launch with few memory round trips:
+// Combine of S split partials [S, n] (n >= 4) in one launch with few memory round trips:
 // a block is kPcQuads column quads x kPcGroups row groups; group r adds the partial rows
 // [r * rpg, min((r + 1) * rpg, S)) in order, eight rows' loads in flight, and the groups' results
 // fold in LDS as a fixed tree (group r with r + h for h = 16, 8, ..., 1), after which group 0
 // writes the epilogue. Folding the groups one after another into group 0 cost 2-2.5 us more
 // with max-count pairs ([8192, 8192] axis 0, 128 splits: 8.5 against 6.0 us in a probe).
+// Outputs of fewer than four columns (VEC = false) go one column a thread.
 constexpr int kPcQuads = 8, kPcGroups = kRThreads / kPcQuads;
-template <class R, class LD>
+template <class R, class LD, bool VEC>
 __global__ void __launch_bounds__(kRThreads)
     k_parts_comb(LD ld, int64_t S, int64_t n, int64_t rpg, float* out, float* out2, int epi, float div) {
     using T = typename R::T;
-    __shared__ T lds[kPcGroups][kPcQuads][4];
+    constexpr int W = VEC ? 4 : 1;
+    __shared__ T lds[kPcGroups][kPcQuads][W];
     ld.setup();
     const int q = threadIdx.x % kPcQuads, r = threadIdx.x / kPcQuads;
-    const int64_t o = ((int64_t)blockIdx.x * kPcQuads + q) * 4;
-    const bool active = o < n;
-    T acc[4];
+    int64_t o = (int64_t)blockIdx.x * kPcQuads + q;
+    const bool active = W * o < n;
+    int lo = 0;
+    if (VEC) col_quad(o, n, &o, &lo);
+    T acc[W];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[j] = R::init();
+    for (int j = 0; j < W; ++j) acc[j] = R::init();
     if (active) {
         const int64_t s0 = r * rpg;
         const int64_t s1 = s0 + rpg < S ? s0 + rpg : S;
         for (int64_t s = s0; s < s1; s += 8) {
-            T v[8][4];
+            T v[8][W];
 #pragma unroll
             for (int u = 0; u < 8; ++u)
-                if (s + u < s1) ld.get4((s + u) * n + o, v[u]);
+                if (s + u < s1) {
+                    if constexpr (VEC) ld.get4((s + u) * n + o, v[u]);
+                    else v[u][0] = ld.get((s + u) * n + o);
+                }
 #pragma unroll
             for (int u = 0; u < 8; ++u)
                 if (s + u < s1)
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) acc[j] = R::comb(acc[j], v[u][j]);
+                    for (int j = 0; j < W; ++j) acc[j] = R::comb(acc[j], v[u][j]);
         }
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j) lds[r][q][j] = acc[j];
+    for (int j = 0; j < W; ++j) lds[r][q][j] = acc[j];
     __syncthreads();
 #pragma unroll
     for (int h = kPcGroups / 2; h >= 1; h >>= 1) {  // every thread reaches every barrier
         if (r < h)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) lds[r][q][j] = R::comb(lds[r][q][j], lds[r + h][q][j]);
+            for (int j = 0; j < W; ++j) lds[r][q][j] = R::comb(lds[r][q][j], lds[r + h][q][j]);
         __syncthreads();
     }
     if (r == 0 && active) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) epi_store(out, out2, o + j, lds[0][q][j], epi, div);
+        for (int j = 0; j < W; ++j)
+            if (j >= lo) epi_store(out, out2, o + j, lds[0][q][j], epi, div);
     }
 }
 
@@ -885,7 +906,7 @@ __global__ void __launch_bounds__(kRThreads)
     }
 }
 
-// Strided-axis reduction over [A, B, C] with C % 4 == 0: block (a * nstrips + strip, s) owns
+// Strided-axis reduction over [A, B, C]: block (a * nstrips + strip, s) owns
 // the 64 column quads [strip * 64, strip * 64 + 64) of slab a (lane = quad) and the rows
 // [s * rps, min((s + 1) * rps, B)), which its four waves interleave (wave w: rows b0 + w,
 // b0 + w + 4, ...). Every wave reads 1 KiB contiguous per row; the wave results combine in
@@ -901,7 +922,10 @@ __global__ void __launch_bounds__(kRThreads)
     const int64_t bx = blockIdx.x;
     const int64_t a = bx / nstrips, strip = bx - a * nstrips;
     const int64_t cq = strip * 64 + lane;
-    const bool active = cq < (C >> 2);
+    const bool active = 4 * cq < C;
+    int64_t c;
+    int lo;
+    col_quad(cq, C, &c, &lo);
     const int64_t s = blockIdx.y;
     const int64_t b0 = s * rps;
     const int64_t b1 = (b0 + rps < B) ? b0 + rps : B;
@@ -909,7 +933,7 @@ __global__ void __launch_bounds__(kRThreads)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[j] = R::init();
     if (active) {
-        const int64_t base = a * B * C + cq * 4;
+        const int64_t base = a * B * C + c;
         int64_t b = b0 + w;
         for (; b + 12 < b1; b += 16) {
             T v[4][4];
@@ -937,9 +961,10 @@ __global__ void __launch_bounds__(kRThreads)
         for (int ww = 0; ww < 3; ++ww)
 #pragma unroll
             for (int j = 0; j < 4; ++j) acc[j] = R::comb(acc[j], lds[ww][lane][j]);
-        const int64_t o = a * C + cq * 4;
+        const int64_t o = a * C + c;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
+            if (j < lo) continue;
             if (S == 1) epi_store(out, out2, o + j, acc[j], epi, div);
             else part_store2(part, S * A * C, s * A * C + o + j, acc[j]);
         }
@@ -1062,41 +1087,40 @@ __device__ __forceinline__ float4 ld_q(const float* p, int64_t q) {  // quad q o
 }
 __device__ __forceinline__ void st_q(float* p, int64_t q, float4 v) { st_ntu(p + 4 * q, vf4{v.x, v.y, v.z, v.w}); }
 struct PendingStores {
-    int64_t q0 = 0, q1 = 0;
+    float *p0 = nullptr, *p1 = nullptr;
     float4 v0, v1;
     int n = 0;
-    __device__ __forceinline__ void put(float* gr, int64_t q, float4 v) {
+    __device__ __forceinline__ void put(float* p, float4 v) {
         if (n == 0) {
-            q0 = q; v0 = v; n = 1;
+            p0 = p; v0 = v; n = 1;
         } else if (n == 1) {
-            q1 = q; v1 = v; n = 2;
+            p1 = p; v1 = v; n = 2;
         } else {
-            st_q(gr, q, v);
+            st_q(p, 0, v);
         }
     }
-    __device__ __forceinline__ void flush(float* gr) const {
-        if (n > 0) st_q(gr, q0, v0);
-        if (n > 1) st_q(gr, q1, v1);
+    __device__ __forceinline__ void flush() const {
+        if (n > 0) st_q(p0, 0, v0);
+        if (n > 1) st_q(p1, 0, v1);
     }
 };
-// grad quad g plus add[j] where hit[j], else plus +0; queued when its bits change.
-__device__ __forceinline__ void route_quad(PendingStores& pd, float* gr, int64_t q, float4 g, const bool (&hit)[4],
+// The grad quad g at p plus add[j] where hit[j], else plus +0; queued when its bits change.
+__device__ __forceinline__ void route_quad(PendingStores& pd, float* p, float4 g, const bool (&hit)[4],
                                            const float (&add)[4]) {
     const float4 n = make_float4(g.x + (hit[0] ? add[0] : 0.0f), g.y + (hit[1] ? add[1] : 0.0f),
                                  g.z + (hit[2] ? add[2] : 0.0f), g.w + (hit[3] ? add[3] : 0.0f));
-    if (bits_differ4(g.x, g.y, g.z, g.w, n.x, n.y, n.z, n.w)) pd.put(gr, q, n);
+    if (bits_differ4(g.x, g.y, g.z, g.w, n.x, n.y, n.z, n.w)) pd.put(p, n);
 }
-__device__ __forceinline__ void route_quad_x(PendingStores& pd, float* gr, int64_t q, float4 g, float4 xv, bool need,
+__device__ __forceinline__ void route_quad_x(PendingStores& pd, float* p, float4 g, float4 xv, bool need,
                                              const float (&mv)[4], const float (&add)[4]) {
     const bool hit[4] = {need && xv.x == mv[0], need && xv.y == mv[1], need && xv.z == mv[2], need && xv.w == mv[3]};
-    route_quad(pd, gr, q, g, hit, add);
+    route_quad(pd, p, g, hit, add);
 }
 
-// Columns (C % 4 == 0, 16-byte aligned grad and x, fewer than 2^32 elements): a thread per
-// (column quad o, split s), the layout of the reduction's column launchers; two rows in
-// flight. SPLIT_X: splits on grid x, column-quad blocks on grid y. pm / pc / pi hold the
-// splits' maxima, counts and indices (RMaxCntArg); they, m and f are 16-byte aligned scratch:
-// one quad load each.
+// Columns (C >= 4, fewer than 2^32 elements): a thread per (column quad, split s), the layout of
+// the reduction's column launchers; two rows in flight. The last quad of a C that is not a multiple
+// of 4 overlaps the one before and stores its own columns one by one. SPLIT_X: splits on grid x, column-quad blocks on grid y. pm / pc / pi hold the
+// splits' maxima, counts and indices (RMaxCntArg).
 template <bool SPLIT_X>
 __global__ void __launch_bounds__(kRThreads)
     k_max_route_cols(float* __restrict__ grad, const float* __restrict__ x, const float* __restrict__ m,
@@ -1104,17 +1128,22 @@ __global__ void __launch_bounds__(kRThreads)
                      const uint32_t* __restrict__ pc, const uint32_t* __restrict__ pi, int64_t A, int64_t B,
                      int64_t C, int64_t rps) {
     const int64_t AC = A * C;
-    const int64_t o = ((int64_t)(SPLIT_X ? blockIdx.y : blockIdx.x) * kRThreads + threadIdx.x) * 4;
-    if (o >= AC) return;
+    const int64_t Cq = (C + 3) >> 2;
+    const int64_t item = (int64_t)(SPLIT_X ? blockIdx.y : blockIdx.x) * kRThreads + threadIdx.x;
+    if (item >= A * Cq) return;
     const int64_t s = SPLIT_X ? blockIdx.x : blockIdx.y;
-    const int64_t a = o / C, c = o - a * C;
+    const int64_t a = item / Cq;
+    int64_t c;
+    int lo;
+    col_quad(item - a * Cq, C, &c, &lo);
+    const int64_t o = a * C + c;
     const int64_t b0 = s * rps, b1 = b0 + rps < B ? b0 + rps : B;
     const int64_t e0 = a * B * C + c;  // element of row 0, column c
     const int64_t k = s * AC + o;      // this split's partials of columns o .. o + 3
-    const float4 m4 = *reinterpret_cast<const float4*>(m + o), f4 = *reinterpret_cast<const float4*>(f + o);
-    const float4 p4 = *reinterpret_cast<const float4*>(pm + k);
-    const uint4 c4 = *reinterpret_cast<const uint4*>(pc + k), i4 = *reinterpret_cast<const uint4*>(pi + k);
-    const float u[4] = {ug[o], ug[o + 1], ug[o + 2], ug[o + 3]};
+    const vf4u m4 = *reinterpret_cast<const vf4u*>(m + o), f4 = *reinterpret_cast<const vf4u*>(f + o);
+    const vf4u p4 = *reinterpret_cast<const vf4u*>(pm + k);
+    const vu4u c4 = *reinterpret_cast<const vu4u*>(pc + k), i4 = *reinterpret_cast<const vu4u*>(pi + k);
+    const vf4u u = *reinterpret_cast<const vf4u*>(ug + o);
     const float mv[4] = {m4.x, m4.y, m4.z, m4.w};
     const float pv[4] = {p4.x, p4.y, p4.z, p4.w};
     const float fv[4] = {f4.x, f4.y, f4.z, f4.w};
@@ -1133,9 +1162,23 @@ __global__ void __launch_bounds__(kRThreads)
         xread = xread || (nj && cv[j] >= 2u);
         sel[j] = nj && cv[j] == 1u ? iv[j] - (eb + (uint32_t)j) : 0xffffffffu;
     }
-    const int64_t q0 = (e0 >> 2) + b0 * (C >> 2), qs = C >> 2;  // quad of row b0 + r: q0 + r * qs
+    float* g0 = grad + e0 + b0 * C;  // row b0
+    const float* x0 = x + e0 + b0 * C;
     const int nr = (int)(b1 - b0);
     const uint32_t uc = (uint32_t)C;
+    if (lo > 0) {  // an overlapping last quad: its own columns, one by one
+        uint32_t rc = 0;
+        for (int r = 0; r < nr; ++r, rc += uc, g0 += C, x0 += C) {
+#pragma unroll
+            for (int j = 1; j < 4; ++j) {
+                if (j < lo) continue;
+                const float g = ld_nt(g0 + j);
+                const float n = g + ((xread ? ld_nt(x0 + j) == mv[j] : rc == sel[j]) ? add[j] : 0.0f);
+                if (__float_as_uint(g) != __float_as_uint(n)) st_nt(g0 + j, n);
+            }
+        }
+        return;
+    }
     // One loop for both ways (x compared, or the row offset against sel): with a loop per way
     // in a branch that is uniform over few waves, the kernel took 61 us against 43 us here
     // ([8192, 8192], axis 0).
@@ -1144,25 +1187,25 @@ __global__ void __launch_bounds__(kRThreads)
     uint32_t rc = 0;  // r * C
     int r = 0;
     for (; r + 1 < nr; r += 2, rc += 2 * uc) {
-        const int64_t qa = q0 + r * qs, qb = qa + qs;
-        const float4 ga = ld_nt4(grad, qa), gb = ld_nt4(grad, qb);
-        const float4 xa = xread ? ld_nt4(x, qa) : z, xb = xread ? ld_nt4(x, qb) : z;
+        float *pa = g0 + r * C, *pb = pa + C;
+        const float4 ga = ld_q(pa, 0), gb = ld_q(pb, 0);
+        const float4 xa = xread ? ld_q(x0 + r * C, 0) : z, xb = xread ? ld_q(x0 + r * C + C, 0) : z;
         const uint32_t rd = rc + uc;
         const bool ha[4] = {xread ? xa.x == mv[0] : rc == sel[0], xread ? xa.y == mv[1] : rc == sel[1],
                             xread ? xa.z == mv[2] : rc == sel[2], xread ? xa.w == mv[3] : rc == sel[3]};
         const bool hb[4] = {xread ? xb.x == mv[0] : rd == sel[0], xread ? xb.y == mv[1] : rd == sel[1],
                             xread ? xb.z == mv[2] : rd == sel[2], xread ? xb.w == mv[3] : rd == sel[3]};
-        route_quad(pd, grad, qa, ga, ha, add);
-        route_quad(pd, grad, qb, gb, hb, add);
+        route_quad(pd, pa, ga, ha, add);
+        route_quad(pd, pb, gb, hb, add);
     }
     if (r < nr) {
-        const int64_t qa = q0 + r * qs;
-        const float4 ga = ld_nt4(grad, qa), xa = xread ? ld_nt4(x, qa) : z;
+        float* pa = g0 + r * C;
+        const float4 ga = ld_q(pa, 0), xa = xread ? ld_q(x0 + r * C, 0) : z;
         const bool ha[4] = {xread ? xa.x == mv[0] : rc == sel[0], xread ? xa.y == mv[1] : rc == sel[1],
                             xread ? xa.z == mv[2] : rc == sel[2], xread ? xa.w == mv[3] : rc == sel[3]};
-        route_quad(pd, grad, qa, ga, ha, add);
+        route_quad(pd, pa, ga, ha, add);
     }
-    pd.flush(grad);
+    pd.flush();
 }
 
 // Rows (C == 1): a block per chunk vr = r * S + s of kRowChunk elements (the reduction's row
@@ -1193,9 +1236,9 @@ __global__ void __launch_bounds__(kRThreads)
     const bool ht = t < (int)(len & 3);
     const float gt = ht ? ld_nt(grad + 4 * nq + t) : 0.0f, xt = ht && need ? ld_nt(x + 4 * nq + t) : 0.0f;
     PendingStores pd;
-    if (ha) route_quad_x(pd, grad, t, ga, xa, need, mv, add);
-    if (hb) route_quad_x(pd, grad, t + kRThreads, gb, xb, need, mv, add);
-    pd.flush(grad);
+    if (ha) route_quad_x(pd, grad + 4 * t, ga, xa, need, mv, add);
+    if (hb) route_quad_x(pd, grad + 4 * (t + kRThreads), gb, xb, need, mv, add);
+    pd.flush();
     if (ht) st_nt(grad + 4 * nq + t, gt + (need && xt == mr ? ad : 0.0f));
 }
 
@@ -1337,7 +1380,7 @@ __global__ void __launch_bounds__(kRThreads)
     }
 }
 
-// Strided axis over [A, B, C]: thread = a quad (VEC) or one element of the [A, C] output,
+// Strided axis over [A, B, C]: thread = a column quad (VEC, C >= 4) or one column of a slab,
 // rows [s * rps, min((s + 1) * rps, B)) of split s in order; K is the line's element at row
 // 0. S == 1 writes the result, S > 1 partials at s * (A * C) + o. SPLIT_X puts the splits on
 // grid x (the column blocks on y), so the round-robin dispatch spreads each column block's
@@ -1347,17 +1390,21 @@ __global__ void __launch_bounds__(kRThreads)
     k_tstd_mom_cols(float* __restrict__ res, const float* __restrict__ x, int64_t A, int64_t B, int64_t C,
                     int64_t rps, int64_t S, Mom* __restrict__ part) {
     constexpr int W = VEC ? 4 : 1;
-    const int64_t AC = A * C;
-    const int64_t o = ((int64_t)(SPLIT_X ? blockIdx.y : blockIdx.x) * kRThreads + threadIdx.x) * W;
-    if (o >= AC) return;
-    const int64_t a = o / C, c = o - a * C;
+    const int64_t AC = A * C, CW = VEC ? (C + 3) >> 2 : C;
+    const int64_t item = (int64_t)(SPLIT_X ? blockIdx.y : blockIdx.x) * kRThreads + threadIdx.x;
+    if (item >= A * CW) return;
+    const int64_t a = item / CW;
+    int64_t c = item - a * CW;
+    int lo = 0;
+    if (VEC) col_quad(c, C, &c, &lo);
+    const int64_t o = a * C + c;
     const int64_t s = SPLIT_X ? blockIdx.x : blockIdx.y;
     const int64_t b0 = s * rps;
     const int64_t b1 = b0 + rps < B ? b0 + rps : B;
     const int64_t base = a * B * C + c;
     auto load = [&](int64_t b, float* v) {
         if (VEC) {
-            const vf4 q = ld_ntv(x + base + b * C, 0);
+            const vf4 q = ld_ntu(x + base + b * C);
 #pragma unroll
             for (int j = 0; j < W; ++j) v[j] = q[j];
         } else {
@@ -1420,6 +1467,7 @@ __global__ void __launch_bounds__(kRThreads)
     }
 #pragma unroll
     for (int j = 0; j < W; ++j) {
+        if (VEC && j < lo) continue;
         Mom t = m[0][j];
 #pragma unroll
         for (int h = 1; h < CH; ++h) {
@@ -1520,10 +1568,10 @@ struct ColSplit {
     int64_t S, rps;
     bool vec;
 };
-static ColSplit col_split(int64_t A, int64_t B, int64_t C, bool vec) {
+static ColSplit col_split(int64_t A, int64_t B, int64_t C) {
     ColSplit cs;
-    cs.vec = vec;
-    const int64_t items = A * C / (vec ? 4 : 1);
+    cs.vec = C >= 4;
+    const int64_t items = A * (cs.vec ? (C + 3) / 4 : C);
     const int64_t bx = (items + kRThreads - 1) / kRThreads;
     const int64_t target = 8 * (int64_t)ctx().num_cus;  // blocks wanted
     int64_t S = 1;
@@ -1541,13 +1589,13 @@ static ColSplit col_split(int64_t A, int64_t B, int64_t C, bool vec) {
     return cs;
 }
 
-// The strip kernel (C % 4 == 0, at least 32 column quads): blocks = A * nstrips * S, with S
+// The strip kernel (at least 32 column quads): blocks = A * nstrips * S, with S
 // raising the block count to about 8 per CU while each wave keeps >= 8 rows.
-static bool use_strip(int64_t C, bool vec) { return vec && C % 4 == 0 && (C >> 2) >= 32; }
+static bool use_strip(int64_t C) { return C >= 128; }
 static ColSplit strip_split(int64_t A, int64_t B, int64_t C, int64_t* nstrips) {
     ColSplit cs;
     cs.vec = true;
-    *nstrips = ((C >> 2) + 63) / 64;
+    *nstrips = ((C + 3) / 4 + 63) / 64;
     const int64_t bx = A * *nstrips;
     const int64_t target = 8 * (int64_t)ctx().num_cus;
     int64_t S = 1;
@@ -1565,15 +1613,15 @@ static ColSplit strip_split(int64_t A, int64_t B, int64_t C, int64_t* nstrips) {
     return cs;
 }
 
-// Wide strided reductions (C % 4 == 0, at least 256 column quads): one thread per column
+// Wide strided reductions (at least 256 column quads): one thread per column
 // quad (k_cols, 2 rows in flight), about four blocks per CU (64-row splits at [8192, 8192]):
 // the best of a sweep of tile shapes on gfx950 (50.4 us against 52 us for 4 rows in flight
 // over 128-row splits; 8 rows in flight, whole-row blocks or strips of 64 quads were slower).
-static bool use_wide_cols(int64_t C, bool vec) { return vec && C % 4 == 0 && (C >> 2) >= 256; }
+static bool use_wide_cols(int64_t C) { return C >= 1024; }
 static ColSplit wide_split(int64_t A, int64_t B, int64_t C) {
     ColSplit cs;
     cs.vec = true;
-    const int64_t bx = (A * (C >> 2) + kRThreads - 1) / kRThreads;
+    const int64_t bx = (A * ((C + 3) / 4) + kRThreads - 1) / kRThreads;
     const int64_t target = 4 * (int64_t)ctx().num_cus;
     int64_t S = (target + bx - 1) / bx;
     int64_t maxS = B / 32;
@@ -1616,30 +1664,27 @@ static size_t row_tmp_floats(int64_t A, int64_t B, bool combine = false) {
 
 // Scratch floats a reduction of [A, B, C] needs for its partials.
 template <class R>
-static size_t tmp_floats_t(int64_t A, int64_t B, int64_t C, bool vec_ok) {
+static size_t tmp_floats_t(int64_t A, int64_t B, int64_t C) {
     if (A * C == 0) return 0;
     if (C == 1) return row_tmp_floats<R>(A, B);
-    // the largest split any column launcher may pick (the choice depends on alignment)
-    int64_t S = 1;
-    if (use_wide_cols(C, vec_ok)) {
-        ColSplit cw = wide_split(A, B, C);
-        S = cw.S > S ? cw.S : S;
+    // the largest split any column launcher may pick
+    int64_t S = col_split(A, B, C).S;
+    if (use_wide_cols(C)) {
+        const int64_t sw = wide_split(A, B, C).S;
+        S = sw > S ? sw : S;
     }
-    if (use_strip(C, vec_ok)) {
+    if (use_strip(C)) {
         int64_t ns;
-        ColSplit cs = strip_split(A, B, C, &ns);
-        S = cs.S > S ? cs.S : S;
+        const int64_t ss = strip_split(A, B, C, &ns).S;
+        S = ss > S ? ss : S;
     }
-    ColSplit c4 = col_split(A, B, C, vec_ok && C % 4 == 0), c1 = col_split(A, B, C, false);
-    S = c4.S > S ? c4.S : S;
-    S = c1.S > S ? c1.S : S;
     return S > 1 ? (size_t)(S * A * C) * part_words<R>() : 0;
 }
 
 size_t reduce_abc_tmp_floats(int op, int64_t A, int64_t B, int64_t C) {
-    if (op == RED_MAXCNT) return tmp_floats_t<RMaxCnt>(A, B, C, true);
-    if (op == RED_MAXCNT_ARG) return tmp_floats_t<RMaxCntArg>(A, B, C, true);
-    return tmp_floats_t<RSum>(A, B, C, true);
+    if (op == RED_MAXCNT) return tmp_floats_t<RMaxCnt>(A, B, C);
+    if (op == RED_MAXCNT_ARG) return tmp_floats_t<RMaxCntArg>(A, B, C);
+    return tmp_floats_t<RSum>(A, B, C);
 }
 
 template <class R>
@@ -1658,11 +1703,24 @@ struct PartLoader<RMaxCntArg> {
     static type make(float* p, int64_t n) { return LdPairsArg{p, reinterpret_cast<const uint32_t*>(p + n)}; }
 };
 
-// nosplit: the combine stage over column-split partials runs as a single pass (tmp unused).
+// Combines the S split partials [S, n] of a column form into the output.
+template <class R>
+static void combine_parts(float* tmp, int64_t S, int64_t n, int epi, float* out, float* out2, float div) {
+    using PL = PartLoader<R>;
+    const int64_t rpg = (S + kPcGroups - 1) / kPcGroups;
+    const dim3 b(kRThreads);
+    if (n >= 4)
+        hipLaunchKernelGGL((k_parts_comb<R, typename PL::type, true>),
+                           dim3((unsigned)(((n + 3) / 4 + kPcQuads - 1) / kPcQuads)), b, 0, ctx().stream,
+                           PL::make(tmp, S * n), S, n, rpg, out, out2, epi, div);
+    else
+        hipLaunchKernelGGL((k_parts_comb<R, typename PL::type, false>), dim3(1), b, 0, ctx().stream,
+                           PL::make(tmp, S * n), S, n, rpg, out, out2, epi, div);
+}
+
 template <class R, class LD>
 static int reduce_t(LD ld, bool vec_ok, int epi, int64_t A, int64_t B, int64_t C, float* out,
-                    float* out2, float div, float* tmp, bool nosplit = false, bool combine = false,
-                    RedSplit* split = nullptr) {
+                    float* out2, float div, float* tmp, bool combine = false, RedSplit* split = nullptr) {
     if (A * C == 0) return MH_OK;
     hipStream_t st = ctx().stream;
     if (C > 1 && B <= 64 && (epi == EPI_SEQ_ACCUM || epi == EPI_SEQ_ACCUM_NEG) && A * C < kMaxGridRows) {
@@ -1730,61 +1788,34 @@ static int reduce_t(LD ld, bool vec_ok, int epi, int64_t A, int64_t B, int64_t C
         if (S > 1) {  // the chunk partials [A, S] reduce again along their rows
             using PL = PartLoader<R>;
             return reduce_t<R, typename PL::type>(PL::make(tmp, nv), true, epi, A, S, 1, out, out2, div,
-                                                  tmp + pad64((size_t)nv * part_words<R>()), false, true);
+                                                  tmp + pad64((size_t)nv * part_words<R>()), true);
         }
         return MH_OK;
     }
     // the wide layout puts the column-quad blocks on grid y (at most 65535 blocks there);
-    // larger outputs take the k_cols launch below (quad blocks on x, splits on y)
-    if (!nosplit && use_wide_cols(C, vec_ok) && (A * C / 4 + kRThreads - 1) / kRThreads <= 65535) {
-        ColSplit cs = wide_split(A, B, C);
-        const int64_t items = A * C / 4;
-        if (split && cs.S > 1) *split = RedSplit{cs.S, cs.rps};
-        dim3 g((unsigned)cs.S, (unsigned)((items + kRThreads - 1) / kRThreads)), b(kRThreads);
+    // larger outputs take the strips below
+    const int64_t quads = A * ((C + 3) / 4);
+    ColSplit cs;
+    if (use_wide_cols(C) && (quads + kRThreads - 1) / kRThreads <= 65535) {
+        cs = wide_split(A, B, C);
+        dim3 g((unsigned)cs.S, (unsigned)((quads + kRThreads - 1) / kRThreads)), b(kRThreads);
         hipLaunchKernelGGL((k_cols<R, LD, true, true>), g, b, 0, st, ld, A, B, C, cs.rps, cs.S, out, out2, epi, div,
                            tmp);
-        if (cs.S > 1) {  // combine the split partials in one launch (k_parts_comb)
-            using PL = PartLoader<R>;
-            const int64_t n = A * C, np = cs.S * n;
-            const unsigned cb = (unsigned)((n / 4 + kPcQuads - 1) / kPcQuads);
-            hipLaunchKernelGGL((k_parts_comb<R, typename PL::type>), dim3(cb), dim3(kRThreads), 0, st,
-                               PL::make(tmp, np), cs.S, n, (cs.S + kPcGroups - 1) / kPcGroups, out, out2, epi, div);
-        }
-        return MH_OK;
-    }
-    if (use_strip(C, vec_ok)) {
+    } else if (use_strip(C)) {
         int64_t ns;
-        ColSplit cs = strip_split(A, B, C, &ns);
-        if (nosplit) {
-            cs.S = 1;
-            cs.rps = B;
-        }
-        if (split && cs.S > 1) *split = RedSplit{cs.S, cs.rps};
+        cs = strip_split(A, B, C, &ns);
         dim3 g((unsigned)(A * ns), (unsigned)cs.S), b(kRThreads);
         hipLaunchKernelGGL((k_cols_strip<R, LD>), g, b, 0, st, ld, A, B, C, ns, cs.rps, cs.S, out, out2, epi, div, tmp);
-        if (cs.S > 1) {
-            using PL = PartLoader<R>;
-            const int64_t np = cs.S * A * C;
-            return reduce_t<R, typename PL::type>(PL::make(tmp, np), true, epi, 1, cs.S, A * C, out, out2, div,
-                                                  nullptr, true);
-        }
-        return MH_OK;
+    } else {
+        cs = col_split(A, B, C);
+        const int64_t items = cs.vec ? quads : A * C;
+        dim3 g((unsigned)((items + kRThreads - 1) / kRThreads), (unsigned)cs.S), b(kRThreads);
+        if (cs.vec) hipLaunchKernelGGL((k_cols<R, LD, true>), g, b, 0, st, ld, A, B, C, cs.rps, cs.S, out, out2, epi, div, tmp);
+        else hipLaunchKernelGGL((k_cols<R, LD, false>), g, b, 0, st, ld, A, B, C, cs.rps, cs.S, out, out2, epi, div, tmp);
     }
-    ColSplit cs = col_split(A, B, C, vec_ok && C % 4 == 0);
-    if (nosplit) {
-        cs.S = 1;
-        cs.rps = B;
-    }
-    const int64_t items = A * C / (cs.vec ? 4 : 1);
-    if (split && cs.S > 1) *split = RedSplit{cs.S, cs.rps};
-    dim3 g((unsigned)((items + kRThreads - 1) / kRThreads), (unsigned)cs.S), b(kRThreads);
-    if (cs.vec) hipLaunchKernelGGL((k_cols<R, LD, true>), g, b, 0, st, ld, A, B, C, cs.rps, cs.S, out, out2, epi, div, tmp);
-    else hipLaunchKernelGGL((k_cols<R, LD, false>), g, b, 0, st, ld, A, B, C, cs.rps, cs.S, out, out2, epi, div, tmp);
     if (cs.S > 1) {
-        using PL = PartLoader<R>;
-        const int64_t np = cs.S * A * C;
-        return reduce_t<R, typename PL::type>(PL::make(tmp, np), sizeof(typename R::T) == 4, epi, 1, cs.S,
-                                              A * C, out, out2, div, nullptr, true);
+        if (split) *split = RedSplit{cs.S, cs.rps};
+        combine_parts<R>(tmp, cs.S, A * C, epi, out, out2, div);
     }
     return MH_OK;
 }
@@ -1795,15 +1826,15 @@ int reduce_abc(int op, int epi, const float* x, int64_t A, int64_t B, int64_t C,
     switch (op) {
         case RED_SUM:
             return reduce_t<RSum, LdPlain<RSum>>(LdPlain<RSum>{x}, al, epi, A, B, C, out, out2, div, tmp, false,
-                                                 false, split);
+                                                 split);
         case RED_MAX:
             return reduce_t<RMax, LdPlain<RMax>>(LdPlain<RMax>{x}, al, epi, A, B, C, out, out2, div, tmp, false,
-                                                 false, split);
+                                                 split);
         case RED_MAXCNT_ARG:
-            return reduce_t<RMaxCntArg, LdArg>(LdArg{x}, al, epi, A, B, C, out, out2, div, tmp, false, false, split);
+            return reduce_t<RMaxCntArg, LdArg>(LdArg{x}, al, epi, A, B, C, out, out2, div, tmp, false, split);
         default:
             return reduce_t<RMaxCnt, LdPlain<RMaxCnt>>(LdPlain<RMaxCnt>{x}, al, epi, A, B, C, out, out2, div, tmp,
-                                                       false, false, split);
+                                                       false, split);
     }
 }
 
@@ -2160,7 +2191,7 @@ int unbroadcast_binrg(int op, int id, bool divs, float* grad, const mh_shape& sg
         C = p.c[0];
     }
     float* tmp = nullptr;
-    const size_t t = tmp_floats_t<RSum>(A, B, C, true);
+    const size_t t = tmp_floats_t<RSum>(A, B, C);
     if (t) MH_TRY(scratch((t + 64) * sizeof(float), reinterpret_cast<void**>(&tmp)));
     const bool al = al16(ug) && al16(a);
     if (op == MH_MUL) {
@@ -2291,7 +2322,7 @@ int pow_exponent_grad(float* grad, const float* x, const float* exponent, const 
         const int64_t nq = n / 4;
         const int64_t G = (nq + kPowThreads - 1) / kPowThreads;  // runs of 64 quads
         const int64_t np = G + (n % 4 != 0 ? 1 : 0);
-        const size_t t = pad64((size_t)np) + tmp_floats_t<RSum>(1, np, 1, true);
+        const size_t t = pad64((size_t)np) + tmp_floats_t<RSum>(1, np, 1);
         MH_TRY(scratch((t + 64) * sizeof(float), reinterpret_cast<void**>(&tmp)));
         if (grad_x) {
             constexpr int NQ = pow_runs<true>();
@@ -2303,9 +2334,9 @@ int pow_exponent_grad(float* grad, const float* x, const float* exponent, const 
                                ctx().stream, ld, n, G, tmp);
         }
         return reduce_t<RSum, LdPlain<RSum>>(LdPlain<RSum>{tmp}, true, EPI_ACCUM, 1, np, 1, grad, nullptr, 0.0f,
-                                             tmp + pad64((size_t)np), false, true);
+                                             tmp + pad64((size_t)np), true);
     }
-    const size_t t = tmp_floats_t<RSum>(1, n, 1, true);
+    const size_t t = tmp_floats_t<RSum>(1, n, 1);
     MH_TRY(scratch((t + 64) * sizeof(float), reinterpret_cast<void**>(&tmp)));
     return reduce_t<RSum, LdPowGrad>(ld, true, EPI_ACCUM, 1, n, 1, grad, nullptr, 0.0f, tmp);
 }
@@ -2438,19 +2469,21 @@ int mh_tstd(float* res, const float* x, const mh_shape* psx, int32_t axis) {
             hipLaunchKernelGGL(k_tstd_mom_combine_rows, dim3((unsigned)A), dim3(kMomCombThreads), 0, st, res, part, S, B);
         return finish("mh_tstd");
     }
-    // strided axis: a thread per column quad, about one block per CU, row splits of at least 64
+    // strided axis: a thread per column quad, about one block per CU, row splits of at least 16
     // rows, eight rows in flight over four accumulator chains. Fewer, longer splits write and
     // combine fewer fp64 partials: at [8192, 8192] axis 0 (a probe, moments + combine) 32 splits
     // took 48.1 us against 52.6 us with 64 splits of four rows in flight, one chain; 128 and
     // 256 splits took 57-60 us. In the bench (moments + combine, streamed) the splits on grid x
     // took 47.2 us against 48.9 us on y; 16 rows in flight 49.4 us, two blocks per CU 59.4 us.
     // With S > 1 there are fewer column blocks than CUs, well inside grid y's limit.
-    const bool vec = al16(x) && C % 4 == 0;
-    const int64_t W = vec ? 4 : 1;
-    const int64_t items = A * C / W;
+    // Single columns where they fill the chip without a split and quads would not ([172, 147, 625]:
+    // 18.9 us against 17.6 + 7.1 us with the combine of three splits).
+    const int64_t chip = (int64_t)ctx().num_cus * kRThreads;
+    const bool vec = C >= 4 && !(A * C >= chip && A * ((C + 3) / 4) < chip && B < 512);
+    const int64_t items = A * (vec ? (C + 3) / 4 : C);
     const int64_t bx = (items + kRThreads - 1) / kRThreads;
     int64_t S = ((int64_t)ctx().num_cus + bx - 1) / bx;
-    int64_t maxS = B / 64;
+    int64_t maxS = B / 16;
     if (maxS < 1) maxS = 1;
     if (S > maxS) S = maxS;
     if (S > 65535) S = 65535;
@@ -2491,11 +2524,11 @@ static bool max_route_split(float* grad, const float* x, int64_t A, int64_t B, i
                            sp.S, B);
         return true;
     }
-    if (!arg || C % 4 != 0 || sp.S > 65535 || !al16(x) || !al16(grad)) return false;
+    if (!arg || C < 4 || sp.S > 65535) return false;
     const int64_t np = sp.S * A * C;
     const uint32_t* pc = reinterpret_cast<const uint32_t*>(tmp + np);
     const uint32_t* pi = reinterpret_cast<const uint32_t*>(tmp + 2 * np);
-    const int64_t qb = (A * C / 4 + kRThreads - 1) / kRThreads;
+    const int64_t qb = (A * ((C + 3) / 4) + kRThreads - 1) / kRThreads;
     const bool sx = qb <= 65535;
     if (!sx && qb > 0x7fffffff) return false;
     const dim3 g = sx ? dim3((unsigned)sp.S, (unsigned)qb) : dim3((unsigned)qb, (unsigned)sp.S), b(kRThreads);

@@ -99,3 +99,30 @@ def test_softmax_rows(gpu, rows, classes, off):
     m.softmax_backward(tg, tx, view(gpu, gout, off))
     assert_bitexact(out.to_numpy(), v["sm"], "softmax")
     assert_bitexact(tg.to_numpy(), gr["x"], "softmax backward")
+
+
+@pytest.mark.parametrize("off", [0, 1, 3])
+@pytest.mark.parametrize("shape", [(1, 70, 3), (1, 5000, 2), (2, 33, 5), (5, 1, 7), (7, 17, 6), (3, 100, 127),
+                                   (2, 65, 129), (1, 300, 1023), (2, 129, 1025), (1, 2100, 1026), (1, 9, 4097),
+                                   (40, 64, 9), (1, 513, 4)], ids=str)
+def test_columns(gpu, shape, off):
+    """Strided axes: single columns, column quads whose last one overlaps the one before, strips
+    and wide forms, in one split and in several."""
+    reductions_match(gpu, shape, 1, off)
+
+
+@pytest.mark.parametrize("op", ["SUB", "MUL", "DIV"])
+@pytest.mark.parametrize("shape,bshape", [((300, 1001), (1, 1001)), ((70, 5), (1, 5)), ((129, 2), (1, 2)),
+                                          ((4099, 130), (130,)), ((3, 200, 67), (3, 1, 67)), ((1000, 3), (3,))],
+                         ids=str)
+def test_unbroadcast_columns(gpu, op, shape, bshape):
+    """The gradient of an operand that repeats over rows, accumulated into a nonzero gradient."""
+    x, b = synth.normal(shape, 0, 1, 2130), synth.uniform(bshape, 0.5, 2, 2131)
+    ug, g0 = synth.normal(shape, 0, 1, 2132), synth.normal(bshape, 0, 1, 2133)
+    x64, b64, u64 = (v.astype(np.float64) for v in (x, b, ug))
+    rg = {"SUB": -u64 + 0 * b64, "MUL": u64 * x64, "DIV": -x64 / (b64 * b64) * u64}[op]
+    lead = rg.ndim - len(bshape)
+    axes = tuple(range(lead)) + tuple(i + lead for i, d in enumerate(bshape) if d == 1 and shape[i + lead] > 1)
+    total = lambda v: v.sum(axis=axes, keepdims=True).reshape(bshape)  # noqa: E731
+    assert_sum_close(gpu.backward(1, OPS[op], ug, x, b, grad=g0), O.backward_op(1, OPS[op], ug, x, b, grad=g0),
+                     total(rg) + g0, f"{op} {shape}", terms_abs=total(np.abs(rg)) + np.abs(g0))
