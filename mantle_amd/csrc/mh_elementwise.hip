@@ -8,8 +8,8 @@
 // broadcast forms of a [rows, K] output have engines of their own: per-row operands ([rows, 1],
 // K >= 4: one fast division per quad) and per-column operands ([1, K], K % 4 == 0: one fast
 // modulo per quad). Other broadcasts decode the output coordinate of each quad with
-// precomputed fast divisors; an inner dimension divisible by 4 keeps 128-bit accesses for
-// every operand whose inner stride is 0 or 1.
+// precomputed fast divisors: collapsed ranks up to 3 with at least 4 elements inside read every
+// operand by one quad or by one value per row touched (k_bc3); the rest go through k_bcast4.
 #include "mh_internal.h"
 #include "mh_math.h"
 
@@ -295,13 +295,6 @@ static inline int bc_static_kinds(int nin, int kinds) {
     return nin == 2 && (kinds == KS_FB || kinds == KS_BF) ? kinds : KS_RUN;
 }
 
-// The general engine's kind of operand k: from the plan, or fixed by KS
-template <int NIN, int KS>
-__device__ __forceinline__ int bc_kind_pl(const ElwPlan& pl, int k) {
-    if constexpr (KS >= 0) return (KS >> (2 * k)) & 3;
-    return pl.kind[k];
-}
-
 // Row-broadcast engine: output [rows, K] with K >= 4 and fewer than 2^31 elements, every
 // IN_BCAST operand a contiguous per-row vector ([rows, 1], as a row max or row sum is), the
 // output and FULL operands 16-byte aligned. One quad per thread: the quad's first row comes
@@ -457,6 +450,105 @@ __global__ void __launch_bounds__(kThreads)
     }
 }
 
+// Broadcast engine for outputs [D0, D1, D2] (a collapsed rank of at most 3) of fewer than 2^31
+// elements with D2 >= 4, the output and FULL operands 16-byte aligned. Bound by memory; one quad
+// per thread in flat order, as the engines above. A broadcast operand is either constant inside a
+// row (BC_ROW: its values at the quad's row and at the next one, both loaded) or contiguous there
+// (BC_QUAD: one quad at any alignment). Where D2 is not a multiple of 4 (INNER4 false) a quad may
+// cross into the next row: the lanes that do, one in D2 / 4, read a BC_QUAD operand's elements
+// again one by one, off the path of the rest. (The gathers this replaces read four scalars per
+// quad and operand under run-time branches: x - b over [256, 96, 729] with b [1, 96, 1] took 32.0
+// us and takes 23.1, the gradient of a SUM over the middle axis of [33, 1025, 1023] 63 and 44 us.) The forms KS are
+// fixed at compile time, two bits per operand, so that all of a thread's loads go out together.
+constexpr int BC_ROW = 2, BC_QUAD = 3;  // beside IN_FULL = 0, IN_SCALAR = 1
+template <int NIN>
+struct Bc3 {
+    int64_t n;
+    uint32_t D1, D2, last_row;
+    FastDiv f1, f2;
+    int32_t s0[NIN], s1[NIN];  // row strides of the broadcast operands
+    int32_t lim[NIN];          // last offset a quad of a BC_QUAD operand can start at
+};
+
+template <class F, int NIN, bool ACCUM, bool INNER4, int KS>
+__global__ void __launch_bounds__(kThreads)
+    k_bc3(float* __restrict__ out, InPtrs<NIN> in, Bc3<NIN> pl, DevScal ds, F f) {
+    const int64_t nq = pl.n >> 2;
+    const int64_t q = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+    constexpr auto form = [](int k) { return (KS >> (2 * k)) & 3; };
+    f.setup(ds);
+    if (q < nq) {
+        const uint32_t e = (uint32_t)(q << 2);
+        const uint32_t r = fdiv(e, pl.f2), c = e - r * pl.D2;
+        const uint32_t i0 = fdiv(r, pl.f1), i1 = r - i0 * pl.D1;
+        uint32_t n0 = i0, n1 = i1;  // the next row (the last one: itself)
+        int jc = 4;                 // the quad's first element in it
+        if constexpr (!INNER4) {
+            const bool wrap = i1 + 1 == pl.D1, last = r == pl.last_row;
+            n0 = last ? i0 : i0 + (wrap ? 1u : 0u);
+            n1 = last ? i1 : (wrap ? 0u : i1 + 1);
+            jc = pl.D2 - c < 4 ? (int)(pl.D2 - c) : 4;
+        }
+        vf4 t[NIN];
+        float a[NIN], b[NIN];
+        int32_t off[NIN], nxt[NIN];
+#pragma unroll
+        for (int k = 0; k < NIN; ++k) {
+            off[k] = (int32_t)i0 * pl.s0[k] + (int32_t)i1 * pl.s1[k];
+            nxt[k] = (int32_t)n0 * pl.s0[k] + (int32_t)n1 * pl.s1[k];
+        }
+#pragma unroll
+        for (int k = 0; k < NIN; ++k) {
+            if (form(k) == BC_ROW) {
+                a[k] = in.p[k][off[k]];
+                b[k] = INNER4 ? a[k] : in.p[k][nxt[k]];
+            } else if (form(k) == BC_QUAD) {
+                const int32_t o = off[k] + (int32_t)c;
+                t[k] = *reinterpret_cast<const vf4u*>(in.p[k] + (INNER4 || o < pl.lim[k] ? o : pl.lim[k]));
+            } else {
+                t[k] = ld_ntv(in.p[k], q);
+            }
+        }
+        vf4 o = vf4{0.f, 0.f, 0.f, 0.f};
+        if (ACCUM) o = ld_ntv(out, q);
+        if constexpr (!INNER4) {
+            if (jc < 4) {
+#pragma unroll
+                for (int k = 0; k < NIN; ++k)
+                    if (form(k) == BC_QUAD)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+                            t[k][j] = in.p[k][j < jc ? off[k] + (int32_t)c + j : nxt[k] + (j - jc)];
+            }
+        }
+        vf4 res;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            float v[NIN];
+#pragma unroll
+            for (int k = 0; k < NIN; ++k) v[k] = form(k) == BC_ROW ? (j < jc ? a[k] : b[k]) : t[k][j];
+            const float fv = f(v);
+            res[j] = ACCUM ? o[j] + fv : fv;
+        }
+        if (!(ACCUM && kSparseAccum<F>) || bits_differ4(o[0], o[1], o[2], o[3], res[0], res[1], res[2], res[3]))
+            st_ntv(out, q, res);
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        for (int64_t i = nq << 2; i < pl.n; ++i) {
+            const uint32_t r = fdiv((uint32_t)i, pl.f2), c = (uint32_t)i - r * pl.D2;
+            const uint32_t i0 = fdiv(r, pl.f1), i1 = r - i0 * pl.D1;
+            float v[NIN];
+#pragma unroll
+            for (int k = 0; k < NIN; ++k) {
+                const int32_t off = (int32_t)i0 * pl.s0[k] + (int32_t)i1 * pl.s1[k];
+                v[k] = in.p[k][form(k) == IN_FULL ? (int32_t)i : form(k) == BC_ROW ? off : off + (int32_t)c];
+            }
+            const float fv = f(v);
+            out[i] = ACCUM ? out[i] + fv : fv;
+        }
+    }
+}
+
 // Broadcast engine, 128-bit path: the output and every FULL operand stream as flat float4
 // quads whatever the shape (all must be 16-byte aligned); only the broadcast operands are
 // gathered, with 32-bit offsets below 2^31 elements and a decode loop bounded by MAXR.
@@ -466,7 +558,7 @@ __global__ void __launch_bounds__(kThreads)
 // the next one, whose offsets follow by addition while the next-outer coordinate does not
 // wrap (a full decode per element only for rows shorter than 4 or at such a wrap); an
 // operand constant along the inner dim is read once per row touched.
-template <class F, int NIN, bool ACCUM, bool INNER4, bool BIG, int MAXR, int KS = KS_RUN>
+template <class F, int NIN, bool ACCUM, bool INNER4, bool BIG, int MAXR>
 __global__ void __launch_bounds__(kThreads)
     k_bcast4(float* __restrict__ out, InPtrs<NIN> in, ElwPlan pl, DevScal ds, F f) {
     constexpr int NA = NIN > 0 ? NIN : 1;
@@ -474,7 +566,7 @@ __global__ void __launch_bounds__(kThreads)
     f.setup(ds);
     float sv[NA];
 #pragma unroll
-    for (int k = 0; k < NIN; ++k) sv[k] = bc_kind_pl<NIN, KS>(pl, k) == IN_SCALAR ? in.p[k][0] : 0.0f;
+    for (int k = 0; k < NIN; ++k) sv[k] = pl.kind[k] == IN_SCALAR ? in.p[k][0] : 0.0f;
     const int inner = pl.rank - 1;
     const int64_t dinner = pl.dims[inner];
     const int64_t douter = inner > 0 ? pl.dims[inner - 1] : 1;
@@ -499,16 +591,12 @@ __global__ void __launch_bounds__(kThreads)
                 slow = true;
             }
         }
-        // with the kinds fixed (KS), broadcast operands go first: their loads sit under run-time
-        // branches on the stride, whose joins wait for the loads issued before them, so a full
-        // operand loaded ahead would be waited for there (two memory round trips per quad)
 #pragma unroll
-        for (int kk = 0; kk < NIN; ++kk) {
-            const int k = KS == KS_FB ? NIN - 1 - kk : kk;
-            if (bc_kind_pl<NIN, KS>(pl, k) == IN_SCALAR) {
+        for (int k = 0; k < NIN; ++k) {
+            if (pl.kind[k] == IN_SCALAR) {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) v[j][k] = sv[k];
-            } else if (bc_kind_pl<NIN, KS>(pl, k) == IN_FULL) {
+            } else if (pl.kind[k] == IN_FULL) {
                 const float4 t = ld_nt4(in.p[k], q);
                 v[0][k] = t.x; v[1][k] = t.y; v[2][k] = t.z; v[3][k] = t.w;
             } else if (INNER4) {
@@ -547,7 +635,7 @@ __global__ void __launch_bounds__(kThreads)
                 }
 #pragma unroll
                 for (int k = 0; k < NIN; ++k)
-                    if (bc_kind_pl<NIN, KS>(pl, k) == IN_BCAST) v[j][k] = in.p[k][oj[k]];
+                    if (pl.kind[k] == IN_BCAST) v[j][k] = in.p[k][oj[k]];
             }
         }
         const float4 o = ACCUM ? ld_nt4(out, q) : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -568,7 +656,7 @@ __global__ void __launch_bounds__(kThreads)
             float v1[NA];
 #pragma unroll
             for (int k = 0; k < NIN; ++k)
-                v1[k] = bc_kind_pl<NIN, KS>(pl, k) == IN_SCALAR ? sv[k] : (bc_kind_pl<NIN, KS>(pl, k) == IN_FULL ? in.p[k][i] : in.p[k][off1[k]]);
+                v1[k] = pl.kind[k] == IN_SCALAR ? sv[k] : (pl.kind[k] == IN_FULL ? in.p[k][i] : in.p[k][off1[k]]);
             const float r1 = f(v1);
             out[i] = ACCUM ? out[i] + r1 : r1;
         }
@@ -670,6 +758,87 @@ static inline unsigned grid_for(int64_t items, int per_block) { return (unsigned
 LaunchShape elw_same_launch(int64_t n) {
     const int64_t nq = n >> 2;
     return LaunchShape{0, kThreads, grid_blocks(nq < kMaxLaunchQuads ? nq : kMaxLaunchQuads, kThreads), launch_count(nq)};
+}
+
+// The forms k_bc3 is built for, by operand count: a broadcast operand in either place of a binary
+// op (two of them: an outer product), last or in the middle of a DIV gradient's three, and the
+// three line operands of a MAX routing. A gradient's first operand is its ug, always full.
+template <int... KS>
+struct FormList {};
+template <class F, int NIN>
+struct Bc3Forms {
+    using type = FormList<>;
+};
+template <class F>
+struct Bc3Forms<F, 1> {
+    using type = FormList<BC_ROW, BC_QUAD>;
+};
+template <class F>
+struct Bc3Forms<F, 2> {
+    using type = FormList<(BC_ROW << 2), (BC_QUAD << 2)>;
+};
+template <int OP>
+struct Bc3Forms<FBin<OP>, 2> {
+    using type = FormList<(BC_ROW << 2), (BC_QUAD << 2), BC_ROW, BC_QUAD, BC_ROW | (BC_QUAD << 2), BC_QUAD | (BC_ROW << 2),
+                          BC_QUAD | (BC_QUAD << 2)>;
+};
+template <class F>
+struct Bc3Forms<F, 3> {
+    using type = FormList<(BC_ROW << 4), (BC_QUAD << 4), (BC_ROW << 2), (BC_QUAD << 2)>;
+};
+template <class F>
+struct Bc3Forms<F, 4> {
+    using type = FormList<(BC_ROW << 2) | (BC_ROW << 4) | (BC_ROW << 6), (BC_QUAD << 2) | (BC_QUAD << 4) | (BC_QUAD << 6)>;
+};
+
+// Launches k_bc3 where it covers the plan (the output and FULL operands are aligned, n < 2^31);
+// false where it does not.
+template <class F, int NIN, bool ACCUM, int... KS>
+static bool launch_bc3_form(FormList<KS...>, int ks, bool inner4, float* out, const InPtrs<NIN>& in, const Bc3<NIN>& p,
+                            const DevScal& ds, F f) {
+    const dim3 g(grid_for(p.n >> 2, kThreads)), b(kThreads);
+    bool done = false;
+    auto one = [&](auto kc) {
+        constexpr int K = decltype(kc)::value;
+        if (K != ks) return;
+        if (inner4) hipLaunchKernelGGL((k_bc3<F, NIN, ACCUM, true, K>), g, b, 0, ctx().stream, out, in, p, ds, f);
+        else hipLaunchKernelGGL((k_bc3<F, NIN, ACCUM, false, K>), g, b, 0, ctx().stream, out, in, p, ds, f);
+        done = true;
+    };
+    (one(std::integral_constant<int, KS>{}), ...);
+    return done;
+}
+template <class F, int NIN, bool ACCUM>
+static bool launch_bc3(float* out, const ElwPlan& pl, const InPtrs<NIN>& in, const DevScal& ds, F f) {
+    if constexpr (NIN == 0) {
+        return false;
+    } else {
+        const int inner = pl.rank - 1;
+        if (pl.rank > 3 || pl.dims[inner] < 4) return false;
+        Bc3<NIN> p;
+        p.n = pl.n;
+        p.D2 = (uint32_t)pl.dims[inner];
+        p.D1 = (uint32_t)(inner > 0 ? pl.dims[inner - 1] : 1);
+        p.f2 = make_fastdiv(p.D2);
+        p.f1 = make_fastdiv(p.D1);
+        p.last_row = (uint32_t)(pl.n / p.D2) - 1;  // pl.n > 0: empty tensors return earlier
+        int ks = 0;
+        for (int k = 0; k < NIN; ++k) {
+            p.s0[k] = p.s1[k] = p.lim[k] = 0;
+            int form = pl.kind[k];
+            if (form == IN_BCAST) {
+                p.s1[k] = (int32_t)(inner > 0 ? pl.st[k][inner - 1] : 0);
+                p.s0[k] = (int32_t)(inner > 1 ? pl.st[k][inner - 2] : 0);
+                if (pl.st[k][inner] != 0 && pl.st[k][inner] != 1) return false;
+                form = pl.st[k][inner] ? BC_QUAD : BC_ROW;
+                int64_t last = 0;  // the operand's last element
+                for (int d = 0; d < pl.rank; ++d) last += (pl.dims[d] - 1) * pl.st[k][d];
+                p.lim[k] = (int32_t)(last - 3);  // BC_QUAD: at least D2 >= 4 elements
+            }
+            ks |= form << (2 * k);
+        }
+        return launch_bc3_form<F, NIN, ACCUM>(typename Bc3Forms<F, NIN>::type{}, ks, p.D2 % 4 == 0, out, in, p, ds, f);
+    }
 }
 
 // Runs F over the plan: out (shape = plan output) = F(inputs), or out += F(inputs).
@@ -784,28 +953,12 @@ static int run_map(float* out, const ElwPlan& pl, const float* const* ptrs, cons
                                f);
             return MH_OK;
         }
+        if (!big && launch_bc3<F, NIN, ACCUM>(out, pl, in, ds, f)) return MH_OK;
         const bool inner4 = pl.vec_ok && al_b;
         if (big) {  // 64-bit offsets, any rank
             if (inner4) hipLaunchKernelGGL((k_bcast4<F, NIN, ACCUM, true, true, MH_MAX_RANK>), g, b, 0, st, out, in, pl, ds, f);
             else hipLaunchKernelGGL((k_bcast4<F, NIN, ACCUM, false, true, MH_MAX_RANK>), g, b, 0, st, out, in, pl, ds, f);
         } else if (pl.rank <= 3) {
-            if constexpr (NIN == 2) {  // a full and a broadcast operand: kinds fixed at compile time
-                const int ks = bc_static_kinds(NIN, kinds);
-                if (ks == KS_FB) {
-                    if (inner4) hipLaunchKernelGGL((k_bcast4<F, NIN, ACCUM, true, false, 3, KS_FB>), g, b, 0, st, out,
-                                                   in, pl, ds, f);
-                    else hipLaunchKernelGGL((k_bcast4<F, NIN, ACCUM, false, false, 3, KS_FB>), g, b, 0, st, out, in,
-                                            pl, ds, f);
-                    return MH_OK;
-                }
-                if (ks == KS_BF) {
-                    if (inner4) hipLaunchKernelGGL((k_bcast4<F, NIN, ACCUM, true, false, 3, KS_BF>), g, b, 0, st, out,
-                                                   in, pl, ds, f);
-                    else hipLaunchKernelGGL((k_bcast4<F, NIN, ACCUM, false, false, 3, KS_BF>), g, b, 0, st, out, in,
-                                            pl, ds, f);
-                    return MH_OK;
-                }
-            }
             if (inner4) hipLaunchKernelGGL((k_bcast4<F, NIN, ACCUM, true, false, 3>), g, b, 0, st, out, in, pl, ds, f);
             else hipLaunchKernelGGL((k_bcast4<F, NIN, ACCUM, false, false, 3>), g, b, 0, st, out, in, pl, ds, f);
         } else {

@@ -766,22 +766,22 @@ __global__ void __launch_bounds__(kCombThreads)
 }
 
 // Combine of S split partials [S, n] (n >= 4) in one launch with few memory round trips:
-// a block is kPcQuads column quads x kPcGroups row groups; group r adds the partial rows
+// a block is 256 / G column quads x G row groups; group r adds the partial rows
 // [r * rpg, min((r + 1) * rpg, S)) in order, eight rows' loads in flight, and the groups' results
-// fold in LDS as a fixed tree (group r with r + h for h = 16, 8, ..., 1), after which group 0
+// fold in LDS as a fixed tree (group r with r + h for h = G / 2, ..., 1), after which group 0
 // writes the epilogue. Folding the groups one after another into group 0 cost 2-2.5 us more
 // with max-count pairs ([8192, 8192] axis 0, 128 splits: 8.5 against 6.0 us in a probe).
-// Outputs of fewer than four columns (VEC = false) go one column a thread.
-constexpr int kPcQuads = 8, kPcGroups = kRThreads / kPcQuads;
-template <class R, class LD, bool VEC>
+// Up to eight partials take one group (no fold), more 32: with 32 groups three partials of 186 K
+// columns took 9.2 us, most threads idle. Outputs of fewer than four columns (VEC = false) go one
+// column a thread.
+template <class R, class LD, bool VEC, int G>
 __global__ void __launch_bounds__(kRThreads)
     k_parts_comb(LD ld, int64_t S, int64_t n, int64_t rpg, float* out, float* out2, int epi, float div) {
     using T = typename R::T;
-    constexpr int W = VEC ? 4 : 1;
-    __shared__ T lds[kPcGroups][kPcQuads][W];
+    constexpr int W = VEC ? 4 : 1, Q = kRThreads / G;
     ld.setup();
-    const int q = threadIdx.x % kPcQuads, r = threadIdx.x / kPcQuads;
-    int64_t o = (int64_t)blockIdx.x * kPcQuads + q;
+    const int q = threadIdx.x % Q, r = threadIdx.x / Q;
+    int64_t o = (int64_t)blockIdx.x * Q + q;
     const bool active = W * o < n;
     int lo = 0;
     if (VEC) col_quad(o, n, &o, &lo);
@@ -806,20 +806,25 @@ __global__ void __launch_bounds__(kRThreads)
                     for (int j = 0; j < W; ++j) acc[j] = R::comb(acc[j], v[u][j]);
         }
     }
+    if constexpr (G > 1) {
+        __shared__ T lds[G][Q][W];
 #pragma unroll
-    for (int j = 0; j < W; ++j) lds[r][q][j] = acc[j];
-    __syncthreads();
-#pragma unroll
-    for (int h = kPcGroups / 2; h >= 1; h >>= 1) {  // every thread reaches every barrier
-        if (r < h)
-#pragma unroll
-            for (int j = 0; j < W; ++j) lds[r][q][j] = R::comb(lds[r][q][j], lds[r + h][q][j]);
+        for (int j = 0; j < W; ++j) lds[r][q][j] = acc[j];
         __syncthreads();
+#pragma unroll
+        for (int h = G / 2; h >= 1; h >>= 1) {  // every thread reaches every barrier
+            if (r < h)
+#pragma unroll
+                for (int j = 0; j < W; ++j) lds[r][q][j] = R::comb(lds[r][q][j], lds[r + h][q][j]);
+            __syncthreads();
+        }
+#pragma unroll
+        for (int j = 0; j < W; ++j) acc[j] = lds[0][q][j];
     }
     if (r == 0 && active) {
 #pragma unroll
         for (int j = 0; j < W; ++j)
-            if (j >= lo) epi_store(out, out2, o + j, lds[0][q][j], epi, div);
+            if (j >= lo) epi_store(out, out2, o + j, acc[j], epi, div);
     }
 }
 
@@ -1104,12 +1109,20 @@ struct PendingStores {
         if (n > 1) st_q(p1, 0, v1);
     }
 };
-// The grad quad g at p plus add[j] where hit[j], else plus +0; queued when its bits change.
+// The grad quad g at p plus add[j] where hit[j], else plus +0; queued when its bits change. lo > 0:
+// the elements before lo are another thread's, and the rest are stored one by one.
 __device__ __forceinline__ void route_quad(PendingStores& pd, float* p, float4 g, const bool (&hit)[4],
-                                           const float (&add)[4]) {
+                                           const float (&add)[4], int lo = 0) {
     const float4 n = make_float4(g.x + (hit[0] ? add[0] : 0.0f), g.y + (hit[1] ? add[1] : 0.0f),
                                  g.z + (hit[2] ? add[2] : 0.0f), g.w + (hit[3] ? add[3] : 0.0f));
-    if (bits_differ4(g.x, g.y, g.z, g.w, n.x, n.y, n.z, n.w)) pd.put(p, n);
+    if (!bits_differ4(g.x, g.y, g.z, g.w, n.x, n.y, n.z, n.w)) return;
+    if (lo == 0) {
+        pd.put(p, n);
+    } else {
+        if (lo < 2) st_nt(p + 1, n.y);
+        if (lo < 3) st_nt(p + 2, n.z);
+        st_nt(p + 3, n.w);
+    }
 }
 __device__ __forceinline__ void route_quad_x(PendingStores& pd, float* p, float4 g, float4 xv, bool need,
                                              const float (&mv)[4], const float (&add)[4]) {
@@ -1166,19 +1179,6 @@ __global__ void __launch_bounds__(kRThreads)
     const float* x0 = x + e0 + b0 * C;
     const int nr = (int)(b1 - b0);
     const uint32_t uc = (uint32_t)C;
-    if (lo > 0) {  // an overlapping last quad: its own columns, one by one
-        uint32_t rc = 0;
-        for (int r = 0; r < nr; ++r, rc += uc, g0 += C, x0 += C) {
-#pragma unroll
-            for (int j = 1; j < 4; ++j) {
-                if (j < lo) continue;
-                const float g = ld_nt(g0 + j);
-                const float n = g + ((xread ? ld_nt(x0 + j) == mv[j] : rc == sel[j]) ? add[j] : 0.0f);
-                if (__float_as_uint(g) != __float_as_uint(n)) st_nt(g0 + j, n);
-            }
-        }
-        return;
-    }
     // One loop for both ways (x compared, or the row offset against sel): with a loop per way
     // in a branch that is uniform over few waves, the kernel took 61 us against 43 us here
     // ([8192, 8192], axis 0).
@@ -1195,15 +1195,15 @@ __global__ void __launch_bounds__(kRThreads)
                             xread ? xa.z == mv[2] : rc == sel[2], xread ? xa.w == mv[3] : rc == sel[3]};
         const bool hb[4] = {xread ? xb.x == mv[0] : rd == sel[0], xread ? xb.y == mv[1] : rd == sel[1],
                             xread ? xb.z == mv[2] : rd == sel[2], xread ? xb.w == mv[3] : rd == sel[3]};
-        route_quad(pd, pa, ga, ha, add);
-        route_quad(pd, pb, gb, hb, add);
+        route_quad(pd, pa, ga, ha, add, lo);
+        route_quad(pd, pb, gb, hb, add, lo);
     }
     if (r < nr) {
         float* pa = g0 + r * C;
         const float4 ga = ld_q(pa, 0), xa = xread ? ld_q(x0 + r * C, 0) : z;
         const bool ha[4] = {xread ? xa.x == mv[0] : rc == sel[0], xread ? xa.y == mv[1] : rc == sel[1],
                             xread ? xa.z == mv[2] : rc == sel[2], xread ? xa.w == mv[3] : rc == sel[3]};
-        route_quad(pd, pa, ga, ha, add);
+        route_quad(pd, pa, ga, ha, add, lo);
     }
     pd.flush();
 }
@@ -1707,15 +1707,21 @@ struct PartLoader<RMaxCntArg> {
 template <class R>
 static void combine_parts(float* tmp, int64_t S, int64_t n, int epi, float* out, float* out2, float div) {
     using PL = PartLoader<R>;
-    const int64_t rpg = (S + kPcGroups - 1) / kPcGroups;
+    constexpr int G = 32;
+    const auto ld = PL::make(tmp, S * n);
+    const int64_t rpg = (S + G - 1) / G, quads = (n + 3) / 4;
     const dim3 b(kRThreads);
-    if (n >= 4)
-        hipLaunchKernelGGL((k_parts_comb<R, typename PL::type, true>),
-                           dim3((unsigned)(((n + 3) / 4 + kPcQuads - 1) / kPcQuads)), b, 0, ctx().stream,
-                           PL::make(tmp, S * n), S, n, rpg, out, out2, epi, div);
+    hipStream_t st = ctx().stream;
+    if (n >= 4 && S <= 8)
+        hipLaunchKernelGGL((k_parts_comb<R, typename PL::type, true, 1>), dim3((unsigned)((quads + kRThreads - 1) / kRThreads)),
+                           b, 0, st, ld, S, n, S, out, out2, epi, div);
+    else if (n >= 4)
+        hipLaunchKernelGGL((k_parts_comb<R, typename PL::type, true, G>),
+                           dim3((unsigned)((quads + kRThreads / G - 1) / (kRThreads / G))), b, 0, st, ld, S, n, rpg, out,
+                           out2, epi, div);
     else
-        hipLaunchKernelGGL((k_parts_comb<R, typename PL::type, false>), dim3(1), b, 0, ctx().stream,
-                           PL::make(tmp, S * n), S, n, rpg, out, out2, epi, div);
+        hipLaunchKernelGGL((k_parts_comb<R, typename PL::type, false, G>), dim3(1), b, 0, st, ld, S, n, rpg, out, out2, epi,
+                           div);
 }
 
 template <class R, class LD>

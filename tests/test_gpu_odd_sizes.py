@@ -126,3 +126,40 @@ def test_unbroadcast_columns(gpu, op, shape, bshape):
     total = lambda v: v.sum(axis=axes, keepdims=True).reshape(bshape)  # noqa: E731
     assert_sum_close(gpu.backward(1, OPS[op], ug, x, b, grad=g0), O.backward_op(1, OPS[op], ug, x, b, grad=g0),
                      total(rg) + g0, f"{op} {shape}", terms_abs=total(np.abs(rg)) + np.abs(g0))
+
+
+BCAST_FORMS = [((3, 5, 7), (1, 5, 1)), ((3, 5, 7), (3, 1, 7)), ((3, 5, 7), (1, 1, 7)), ((3, 5, 7), (3, 5, 1)),
+               ((2, 3, 4), (2, 1, 4)), ((4, 1, 9), (1, 6, 1)), ((4, 1, 9), (1, 6, 9)), ((4, 6, 1), (1, 1, 11)),
+               ((129, 5), (5,)), ((17, 9, 13), (9, 1)), ((5, 3, 131), (5, 1, 131)), ((2, 33, 729), (1, 33, 1)),
+               ((1, 64, 6), (5, 1, 6)), ((7, 2, 3, 5), (7, 1, 3, 5)), ((6, 1, 5), (1, 4, 5))]
+
+
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("s1,s2", BCAST_FORMS, ids=str)
+def test_broadcast_forms(gpu, s1, s2, off):
+    """A broadcast operand in either place, constant or contiguous inside a row whose length is not
+    (or is) a multiple of 4, both operands broadcast, and their gradients; the broadcast operand
+    also at an unaligned address. Element values are single operations: bit for bit."""
+    m = gpu.m
+    a, b = synth.normal(s1, 0, 1, 2140), synth.uniform(s2, 0.5, 2, 2141)
+    for x, y, x_off, y_off in ((a, b, 0, off), (b, a, off, 0)):
+        tx, ty = view(gpu, x, x_off), view(gpu, y, y_off)
+        so = np.broadcast_shapes(x.shape, y.shape)
+        ug, g0 = synth.normal(so, 0, 1, 2142), synth.normal(x.shape, 0, 1, 2143)
+        for op in (OPS["SUB"], OPS["MUL"], OPS["DIV"]):
+            res = m.Tensor(m.TensorShape(*so))
+            m.forward_op(op, res, tx, ty)
+            assert_bitexact(res.to_numpy(), ORC.forward(op, x, y), f"{s1} {s2} op {op}")
+            for i, (p, q) in enumerate(((x, y), (y, x))):
+                g0 = synth.normal(p.shape, 0, 1, 2144 + i)
+                got = gpu.backward(i, op, ug, x, y, grad=g0)
+                if p.shape == so:  # no sum: the same single operations
+                    assert_bitexact(got, ORC.backward(i, op, ug, x, y, grad=g0), f"{s1} {s2} op {op} id {i}")
+
+
+@pytest.mark.parametrize("shape,axis", [((6, 3, 7), 1), ((9, 2, 131), 1), ((5, 3, 2, 9), 1), ((2, 30, 1001), 1), ((7, 9), 0)],
+                         ids=str)
+def test_reduce_backward_short_axes(gpu, shape, axis):
+    """Reductions over an axis too short to split: the line operands of SUM, MEAN and MAX backward
+    broadcast over it."""
+    reductions_match(gpu, shape, axis)
