@@ -15,15 +15,18 @@
 // nn.LogSoftmax, CrossEntropyLoss and the Softmax -> LOG -> MUL -> MEAN head run as the
 // row-fused kernels (MH_MODEL_FUSE_ROWS). Every tensor and gradient slot holds what the
 // op-by-op execution writes there, so the fusion is not observable in results.
+// Runs of nodes over one [R, W] view whose tensors are small, or that would re-read from memory
+// what they just wrote, go as one launch (mh_program.hip), planned when the model is made.
 // mh_model_capture records a pass (forward, backward, or zero_grad + forward + backward) as
 // one HIP graph that mh_model_replay launches. While a captured graph exists, a library
 // buffer that grows is retired rather than freed, so the addresses the graph holds stay
 // valid until the graph is released or the library shuts down (a replay after mh_shutdown is
 // refused).
 #include <new>
+#include <unordered_map>
 #include <vector>
 
-#include "mh_internal.h"
+#include "mh_program.h"
 
 struct mh_graph {
     struct Sym {
@@ -66,6 +69,14 @@ struct mh_model {
     };
     std::vector<RowGroup> rows;
     std::vector<int> row_of;  // per node: its RowGroup, or -1
+    struct Segment {
+        int first, last;  // nodes, in creation order
+        mh::ProgRun run;
+    };
+    std::vector<Segment> fseg, bseg;          // forward and backward programs
+    std::vector<int> fseg_of, bseg_of;        // per node: its Segment, or -1
+    void* prog_mem = nullptr;                 // their instructions and sums
+    float* prog_part = nullptr;               // partials of one program at a time
     hipGraphExec_t graph[3] = {nullptr, nullptr, nullptr};  // captured passes (MH_PASS_FORWARD / _BACKWARD / _STEP)
     uint64_t graph_epoch[3] = {0, 0, 0};                     // the mh_init epoch each was captured in
 };
@@ -315,6 +326,443 @@ static void plan_fusion(mh_model* m) {
     }
 }
 
+// ---------------------------------------------------------------------------------------
+// programs: runs of nodes over one [R, W] view as one launch
+// ---------------------------------------------------------------------------------------
+// The view of a run: shape S (the largest of its first node), W its last dimension.
+struct ProgView {
+    mh_shape S;
+    int64_t R = 0;
+    int64_t W = 0;
+    bool single() const { return R * W <= kProgSingle; }
+    // Row instructions: a row per wavefront needs k_rows_wave's lengths, and several slabs of them
+    // lose to the node's own kernels (the head over [5000, 200]: 92 us against 79).
+    bool rows_ok() const { return W <= 64 || (single() && W < 2048); }
+};
+
+static int64_t dim_from_end(const mh_shape& s, int k) { return k < s.rank ? s.dims[s.rank - 1 - k] : 1; }
+
+// The form of shape t in the view, or -1.
+static int prog_class(const ProgView& v, const mh_shape& t) {
+    const int64_t n = numel(t);
+    const int rank = t.rank > v.S.rank ? t.rank : v.S.rank;
+    bool full = true, row = v.W > 1 && v.R > 1, col = v.R > 1 && v.W > 1;
+    for (int k = 0; k < rank; ++k) {
+        const int64_t a = dim_from_end(t, k), b = dim_from_end(v.S, k);
+        full = full && a == b;
+        row = row && a == (k == 0 ? 1 : b);
+        col = col && a == (k == 0 ? b : 1);
+    }
+    if (full) return PC_FULL;
+    if (n == 1) return PC_SCAL;
+    return row ? PC_ROW : col ? PC_COL : -1;
+}
+
+// Instructions of one run and their accesses since the last barrier: an address touched under two
+// thread mappings, once to write, needs a barrier between.
+struct ProgBuild {
+    ProgView v;
+    std::vector<ProgInstr> a, b;
+    std::vector<ProgSum> sums;
+    int64_t part = 0;     // partial floats per workgroup
+    bool cols = false;    // sums over rows
+    bool max_rows = false;
+    std::unordered_map<const float*, int> reads, writes;  // address -> mapping (kAny: several)
+    static constexpr int kFlat = 1, kFlatRow = 2, kRows = 3, kAny = 4;
+
+    // The run as it was at an earlier node: the parts appended since are dropped.
+    struct Mark {
+        size_t na, nb, ns;
+        int64_t part;
+        bool cols, max_rows;
+    };
+    Mark mark() const { return Mark{a.size(), b.size(), sums.size(), part, cols, max_rows}; }
+    void cut(const Mark& k) {
+        a.resize(k.na);
+        b.resize(k.nb);
+        sums.resize(k.ns);
+        part = k.part;
+        cols = k.cols;
+        max_rows = k.max_rows;
+    }
+
+    bool clash(const float* p, int map, bool write) {
+        auto hit = [&](std::unordered_map<const float*, int>& m) {
+            auto it = m.find(p);
+            return it != m.end() && (it->second != map || map == kAny);
+        };
+        return p && (hit(writes) || (write && hit(reads)));
+    }
+    void note(std::unordered_map<const float*, int>& m, const float* p, int map) {
+        if (!p) return;
+        auto it = m.find(p);
+        if (it == m.end()) m[p] = map;
+        else if (it->second != map) it->second = kAny;
+    }
+    // map_of[k]: the mapping under which operands a, b, c and the output are touched
+    void push(ProgInstr in, const int (&map)[4]) {
+        const float* p[4] = {in.a, in.b, in.c, in.out};
+        bool bar = false;
+        for (int k = 0; k < 4; ++k) bar = bar || clash(p[k], map[k], k == 3);
+        if (bar) {
+            in.flags |= PF_BARRIER;
+            reads.clear();
+            writes.clear();
+        }
+        for (int k = 0; k < 3; ++k) note(reads, p[k], map[k]);
+        note(writes, in.out, map[3]);
+        a.push_back(in);
+    }
+    static ProgInstr instr(int op, float* out, const float* x, int cx, const float* y = nullptr, int cy = 0,
+                           const float* z = nullptr, int cz = 0) {
+        ProgInstr in{};
+        in.op = op;
+        in.out = out;
+        in.a = x;
+        in.b = y;
+        in.c = z;
+        in.cls = cx | (cy << 2) | (cz << 4);
+        return in;
+    }
+    // elementwise over the view's elements, or its rows (co == PC_ROW)
+    void ew(ProgInstr in, int co) {
+        const int base = co == PC_ROW ? kFlatRow : kFlat;
+        if (co == PC_ROW) in.flags |= PF_ROWDOM;
+        int map[4];
+        for (int k = 0; k < 3; ++k) map[k] = ((in.cls >> (2 * k)) & 3) == co ? base : kAny;
+        map[3] = base;
+        push(in, map);
+    }
+};
+
+static bool prog_forward_node(mh_model* m, size_t i, ProgBuild& pb) {
+    const mh_graph& g = m->g;
+    const mh_graph::Node& nd = g.nodes[i];
+    if (m->fuse[i] == kFuseRow) return false;
+    int c[3] = {0, 0, 0};
+    for (int k = 0; k < nd.nin; ++k)
+        if ((c[k] = prog_class(pb.v, g.syms[nd.in[k]].shape)) < 0) return false;
+    const int co = prog_class(pb.v, g.syms[nd.out].shape);
+    const mh_shape& sx = g.syms[nd.in[0]].shape;
+    float* out = m->t[nd.out];
+    const float* x = m->t[nd.in[0]];
+    if (is_reduce(nd.op)) {
+        const int ax = axis_of(nd.attrs);
+        const float div = nd.op == MH_MEAN ? (float)(ax < 0 ? numel(sx) : sx.dims[ax]) : 0.0f;
+        if (ax < 0) {  // every element
+            if (c[0] != PC_FULL && c[0] != PC_ROW) return false;
+            if (!pb.v.single()) return false;
+            ProgInstr in = ProgBuild::instr(nd.op == MH_MAX ? PO_AMAX : PO_ASUM, out, x, c[0]);
+            in.f0 = div;
+            if (c[0] == PC_ROW) in.flags |= PF_ROWDOM;
+            const int map[4] = {ProgBuild::kAny, 0, 0, ProgBuild::kAny};
+            pb.push(in, map);
+            return true;
+        }
+        if (ax != sx.rank - 1 || c[0] != PC_FULL || co != PC_ROW || !pb.v.rows_ok()) return false;
+        ProgInstr in = ProgBuild::instr(nd.op == MH_MAX ? PO_RMAX : PO_RSUM, out, x, PC_FULL);
+        in.f0 = div;
+        const int map[4] = {ProgBuild::kRows, 0, 0, ProgBuild::kRows};
+        pb.push(in, map);
+        return true;
+    }
+    if (co != PC_FULL && co != PC_ROW) return false;
+    for (int k = 0; k < nd.nin; ++k)
+        if (co == PC_ROW && c[k] != PC_ROW && c[k] != PC_SCAL) return false;
+    if (is_binary(nd.op)) {
+        pb.ew(ProgBuild::instr(PO_ADD + (nd.op - MH_ADD), out, x, c[0], m->t[nd.in[1]], c[1]), co);
+        return true;
+    }
+    if (nd.nin != 1) return false;
+    int op;
+    switch (nd.op) {
+        case MH_EXP: op = PO_EXP; break;
+        case MH_LOG: op = PO_LOG; break;
+        case MH_SIGMOID: op = PO_SIGMOID; break;
+        case MH_RELU: op = PO_RELU; break;
+        case MH_TANH: op = PO_TANH; break;
+        case MH_LEAKYRELU: op = PO_LEAKY; break;
+        case MH_CLIP: op = PO_CLIP; break;
+        default: return false;
+    }
+    ProgInstr in = ProgBuild::instr(op, out, x, c[0]);
+    in.f0 = op == PO_LEAKY ? nd.attrs.negative_slope : clip_lo(nd.attrs);
+    in.f1 = clip_hi(nd.attrs);
+    pb.ew(in, co);
+    return true;
+}
+
+// Appends the node's gradient instructions; false where one of them has no program form (pb is then
+// as it was).
+static bool prog_backward_node(mh_model* m, size_t i, ProgBuild& pb) {
+    const mh_graph& g = m->g;
+    const mh_graph::Node& nd = g.nodes[i];
+    if (m->fuse[i] == kFuseRow) return false;
+    const float* ug = m->gr[nd.out];
+    if (!ug) return true;  // no trainable operand
+    int c[3] = {0, 0, 0};
+    for (int k = 0; k < nd.nin; ++k)
+        if ((c[k] = prog_class(pb.v, g.syms[nd.in[k]].shape)) < 0) return false;
+    const int co = prog_class(pb.v, g.syms[nd.out].shape);
+    const mh_shape& sx = g.syms[nd.in[0]].shape;
+    const float* t1 = m->t[nd.in[0]];
+    float* g1 = m->gr[nd.in[0]];
+    if (is_binary(nd.op)) {
+        if (co != PC_FULL && co != PC_ROW) return false;
+        const float* t2 = m->t[nd.in[1]];
+        float* gr[2] = {g1, m->gr[nd.in[1]]};
+        for (int k = 0; k < 2; ++k) {  // every part has a form, before any is appended
+            if (!gr[k] || c[k] == co) continue;
+            if (co != PC_FULL || c[k] == PC_SCAL) return false;
+            if (c[k] == PC_ROW && !pb.v.rows_ok()) return false;
+            if (c[k] == PC_COL) {
+                if (!pb.v.single() && pb.v.R <= 64) return false;  // a short column's sum keeps its order
+                if (gr[0] == gr[1]) return false;
+                for (const ProgInstr& e : pb.b)
+                    if (e.out == gr[k]) return false;
+            }
+        }
+        for (int k = 0; k < 2; ++k) {
+            if (!gr[k]) continue;
+            // (kind, operands) of FBinRg: ug, then what it reads
+            int kind;
+            ProgInstr in;
+            if (nd.op == MH_ADD || (nd.op == MH_SUB && k == 0)) {
+                kind = PT_UG;
+                in = ProgBuild::instr(0, gr[k], ug, co);
+            } else if (nd.op == MH_SUB) {
+                kind = PT_NEG;
+                in = ProgBuild::instr(0, gr[k], ug, co);
+            } else if (nd.op == MH_MUL) {
+                kind = PT_MUL;
+                in = k == 0 ? ProgBuild::instr(0, gr[k], ug, co, t2, c[1]) : ProgBuild::instr(0, gr[k], ug, co, t1, c[0]);
+            } else if (k == 0) {
+                kind = PT_DIV0;
+                in = ProgBuild::instr(0, gr[k], ug, co, t2, c[1]);
+            } else {
+                kind = PT_DIV1;
+                in = ProgBuild::instr(0, gr[k], ug, co, t1, c[0], t2, c[1]);
+            }
+            if (c[k] == co) {
+                in.op = PO_G_UG + (kind - PT_UG);
+                pb.ew(in, co);
+            } else if (c[k] == PC_ROW) {
+                in.op = PO_RUNB;
+                in.slot = kind;
+                int map[4];
+                for (int j = 0; j < 3; ++j) {
+                    const int cl = (in.cls >> (2 * j)) & 3;
+                    map[j] = cl == PC_FULL || cl == PC_ROW ? ProgBuild::kRows : ProgBuild::kAny;
+                }
+                map[3] = ProgBuild::kRows;
+                pb.push(in, map);
+            } else {
+                in.op = PO_CUNB;
+                in.slot = kind;
+                if (!pb.v.single()) {
+                    in.part = pb.part;
+                    pb.sums.push_back(ProgSum{gr[k], pb.part, (int32_t)pb.v.W, 0});
+                    pb.part += pb.v.W;
+                }
+                pb.cols = true;
+                pb.b.push_back(in);
+            }
+        }
+        return true;
+    }
+    if (!g1) return true;
+    if (is_reduce(nd.op)) {
+        const int ax = axis_of(nd.attrs);
+        if (ax < 0) {
+            if (nd.op == MH_MAX || (c[0] != PC_FULL && c[0] != PC_ROW)) return false;
+            ProgInstr in = ProgBuild::instr(PO_G_SCALE, g1, ug, PC_SCAL);
+            in.f0 = nd.op == MH_SUM ? 1.0f : (float)(1.0 / (double)numel(sx));
+            pb.ew(in, c[0]);
+            return true;
+        }
+        if (ax != sx.rank - 1 || c[0] != PC_FULL || co != PC_ROW) return false;
+        if (nd.op == MH_MAX) {
+            if (!pb.v.rows_ok()) return false;
+            ProgInstr in = ProgBuild::instr(PO_RMAXB, g1, t1, PC_FULL, ug, PC_ROW);
+            const int map[4] = {ProgBuild::kAny, ProgBuild::kAny, 0, ProgBuild::kAny};
+            pb.max_rows = true;
+            pb.push(in, map);
+            return true;
+        }
+        ProgInstr in = ProgBuild::instr(PO_G_SCALE, g1, ug, PC_ROW);
+        in.f0 = nd.op == MH_SUM ? 1.0f : (float)(1.0 / (double)sx.dims[ax]);
+        pb.ew(in, PC_FULL);
+        return true;
+    }
+    if (nd.nin != 1 || (co != PC_FULL && co != PC_ROW) || c[0] != co) return false;
+    int op;
+    switch (nd.op) {
+        case MH_EXP: op = PO_G_EXP; break;
+        case MH_LOG: op = PO_G_LOG; break;
+        case MH_SIGMOID: op = PO_G_SIGMOID; break;
+        case MH_RELU: op = PO_G_RELU; break;
+        case MH_TANH: op = PO_G_TANH; break;
+        case MH_LEAKYRELU: op = PO_G_LEAKY; break;
+        case MH_CLIP: op = PO_G_CLIP; break;
+        default: return false;
+    }
+    ProgInstr in = ProgBuild::instr(op, g1, t1, c[0], ug, co);
+    in.f0 = op == PO_G_LEAKY ? nd.attrs.negative_slope : clip_lo(nd.attrs);
+    in.f1 = clip_hi(nd.attrs);
+    pb.ew(in, co);
+    return true;
+}
+
+// The view of a run that starts at node i: the largest of its operands and output.
+static bool prog_view(const mh_model* m, size_t i, ProgView* v) {
+    const mh_graph::Node& nd = m->g.nodes[i];
+    const mh_shape* best = &m->g.syms[nd.out].shape;
+    for (int k = 0; k < nd.nin; ++k)
+        if (numel(m->g.syms[nd.in[k]].shape) > numel(*best)) best = &m->g.syms[nd.in[k]].shape;
+    v->S = *best;
+    v->W = best->dims[best->rank - 1];
+    const int64_t n = numel(*best);
+    if (n < 2 || v->W < 2 || n >= ((int64_t)1 << 31)) return false;
+    v->R = n / v->W;
+    return true;
+}
+
+// Rows of a slab, and whether the run is worth a program: slabs of about 2048 elements, of at least
+// 8 rows where sums over rows leave a partial per slab. Measured, a training step of MUL -> ADD ->
+// RELU layers, nodes one by one against programs: 24 layers of [32, 32] 530-630 and 165 us, 3 of
+// [1902, 31] 151 and 75, 3 of [3000, 300] 146 and 106. Wider slabs (8 rows of 1000: 96 and 124) and
+// more than a million elements (4 of [16384, 500] 705 and 650, the head over [2^20, 10] 394 and
+// 480) go node by node: there the kernels stream at memory speed, and one workgroup a slab cannot.
+static bool prog_shape(const ProgBuild& pb, ProgRun* r) {
+    const int64_t R = pb.v.R, W = pb.v.W;
+    if (pb.v.single()) {
+        if (pb.max_rows && R > kProgRows) return false;
+        r->rpw = (int32_t)R;
+        r->nwg = 1;
+        return pb.cols || pb.a.size() >= 2;
+    }
+    int64_t rpw = (2048 + W - 1) / W;
+    if (pb.cols && rpw < 8) rpw = 8;
+    if (rpw > kProgRows) rpw = kProgRows;
+    const int64_t nwg = (R + rpw - 1) / rpw;
+    if (nwg < 2 || rpw * W > 4096 || R * W > kProgMax) return false;
+    r->rpw = (int32_t)rpw;
+    r->nwg = (int32_t)nwg;
+    return pb.cols || pb.a.size() >= 2;
+}
+
+struct ProgPlan {
+    std::vector<ProgInstr> instrs;
+    std::vector<ProgSum> sums;
+    size_t part = 0;
+    std::vector<std::pair<size_t, size_t>> at;  // per segment: first instruction, first sum
+};
+
+static void prog_keep(ProgBuild& pb, int first, int last, ProgPlan& plan, std::vector<mh_model::Segment>& segs,
+                      std::vector<int>& of) {
+    mh_model::Segment sg;
+    sg.first = first;
+    sg.last = last;
+    ProgRun& r = sg.run;
+    // a single node only for its sums over rows: wherever a view has a program these go through it,
+    // so that their order does not depend on what the node's neighbours are
+    if ((last == first && !pb.cols) || !prog_shape(pb, &r)) return;
+    r.R = pb.v.R;
+    r.W = (int32_t)pb.v.W;
+    r.na = (int)pb.a.size();
+    r.nb = (int)pb.b.size();
+    r.nsums = (int)pb.sums.size();
+    for (ProgInstr& in : pb.a) in.part *= r.nwg;
+    for (ProgInstr& in : pb.b) in.part *= r.nwg;
+    for (ProgSum& u : pb.sums) {
+        u.part *= r.nwg;
+        if (u.ncol > r.maxcol) r.maxcol = u.ncol;
+    }
+    const size_t part = (size_t)pb.part * (size_t)r.nwg;
+    if (part > plan.part) plan.part = part;
+    plan.at.emplace_back(plan.instrs.size(), plan.sums.size());
+    plan.instrs.insert(plan.instrs.end(), pb.a.begin(), pb.a.end());
+    plan.instrs.insert(plan.instrs.end(), pb.b.begin(), pb.b.end());
+    plan.sums.insert(plan.sums.end(), pb.sums.begin(), pb.sums.end());
+    for (int j = first; j <= last; ++j) of[j] = (int)segs.size();
+    segs.push_back(sg);
+}
+
+// A fused bias + RELU pair is not split between a program and its kernels.
+static bool prog_cut_ok(const mh_model* m, int first, int last) {
+    const int nn = (int)m->g.nodes.size();
+    return m->fuse[first] != kFuseRelu && !(last + 1 < nn && m->fuse[last] == kFuseAdd);
+}
+
+static void plan_programs(mh_model* m, ProgPlan& plan) {
+    const int nn = (int)m->g.nodes.size();
+    m->fseg_of.assign(nn, -1);
+    m->bseg_of.assign(nn, -1);
+    for (int i = 0; i < nn;) {
+        ProgBuild pb;
+        ProgBuild::Mark ok{};  // the longest run so far that may end there
+        int last = -1;
+        if (prog_view(m, i, &pb.v) && m->fuse[i] != kFuseRelu) {
+            for (int j = i; j < nn; ++j) {
+                if (!prog_forward_node(m, j, pb)) break;
+                if (prog_cut_ok(m, i, j)) {
+                    ok = pb.mark();
+                    last = j;
+                }
+            }
+        }
+        if (last >= 0) {
+            pb.cut(ok);
+            prog_keep(pb, i, last, plan, m->fseg, m->fseg_of);
+        }
+        i = last >= i ? last + 1 : i + 1;
+    }
+    if (m->grad_floats == 0) return;
+    for (int i = nn - 1; i >= 0;) {
+        ProgBuild pb;
+        ProgBuild::Mark ok{};
+        int first = nn;
+        if (prog_view(m, i, &pb.v) && m->fuse[i] != kFuseAdd) {
+            for (int j = i; j >= 0; --j) {
+                if (!prog_backward_node(m, j, pb)) break;
+                if (prog_cut_ok(m, j, i)) {
+                    ok = pb.mark();
+                    first = j;
+                }
+            }
+        }
+        if (first <= i) {
+            pb.cut(ok);
+            prog_keep(pb, first, i, plan, m->bseg, m->bseg_of);
+        }
+        i = first <= i ? first - 1 : i - 1;
+    }
+}
+
+static size_t pad256(size_t b) { return (b + 255) & ~(size_t)255; }
+
+// Plans the model's programs and places them on the device.
+static int build_programs(mh_model* m) {
+    ProgPlan plan;
+    plan_programs(m, plan);
+    if (plan.at.empty()) return MH_OK;
+    const size_t ib = pad256(plan.instrs.size() * sizeof(ProgInstr)), sb = pad256(plan.sums.size() * sizeof(ProgSum));
+    MH_TRY(mh_malloc(&m->prog_mem, ib + sb));
+    if (plan.part) MH_TRY(mh_malloc(reinterpret_cast<void**>(&m->prog_part), plan.part * sizeof(float)));
+    MH_TRY(mh_memcpy_h2d(m->prog_mem, plan.instrs.data(), plan.instrs.size() * sizeof(ProgInstr)));
+    char* sums = static_cast<char*>(m->prog_mem) + ib;
+    MH_TRY(mh_memcpy_h2d(sums, plan.sums.data(), plan.sums.size() * sizeof(ProgSum)));
+    size_t k = 0;
+    for (auto* segs : {&m->fseg, &m->bseg})
+        for (mh_model::Segment& s : *segs) {
+            s.run.prog = static_cast<const ProgInstr*>(m->prog_mem) + plan.at[k].first;
+            s.run.sums = reinterpret_cast<const ProgSum*>(sums) + plan.at[k].second;
+            s.run.part = m->prog_part;
+            ++k;
+        }
+    return MH_OK;
+}
+
 static int run_forward_node(mh_model* m, size_t i) {
     const mh_graph& g = m->g;
     const mh_graph::Node& nd = g.nodes[i];
@@ -405,6 +853,34 @@ static int run_backward_node(mh_model* m, size_t i) {
     return mh_clip_bwd_accum(g1, t1, ug, n1, clip_lo(nd.attrs), clip_hi(nd.attrs));
 }
 
+// Nodes [0, nodes) forward, and every node backward: programs where they cover a run, else a node
+// at a time.
+static int run_forward(mh_model* m, int32_t nodes) {
+    for (int32_t i = 0; i < nodes; ++i) {
+        const int sg = m->fseg_of[i];
+        if (sg >= 0 && m->fseg[sg].first == i && m->fseg[sg].last < nodes) {
+            MH_TRY(prog_launch(m->fseg[sg].run));
+            i = m->fseg[sg].last;
+        } else {
+            MH_TRY(run_forward_node(m, (size_t)i));
+        }
+    }
+    return MH_OK;
+}
+
+static int run_backward(mh_model* m) {
+    for (int32_t i = (int32_t)m->g.nodes.size() - 1; i >= 0; --i) {
+        const int sg = m->bseg_of[i];
+        if (sg >= 0 && m->bseg[sg].last == i) {
+            MH_TRY(prog_launch(m->bseg[sg].run));
+            i = m->bseg[sg].first;
+        } else {
+            MH_TRY(run_backward_node(m, (size_t)i));
+        }
+    }
+    return MH_OK;
+}
+
 static int write_inputs(mh_model* m, int32_t ninputs, const float* const* inputs, int where) {
     const mh_graph& g = m->g;
     if (ninputs != (int32_t)g.inputs.size())
@@ -434,11 +910,10 @@ static int enqueue_pass(mh_model* m, int pass) {
     if (pass == MH_PASS_STEP && m->grad_arena)  // parameters.grads.set_zero (collection.mojo:221-224)
         MH_TRY(mh_zero(m->grad_arena, (int64_t)m->grad_floats));
     if (pass == MH_PASS_FORWARD || pass == MH_PASS_STEP)
-        for (size_t i = 0; i < g.nodes.size(); ++i) MH_TRY(run_forward_node(m, i));
+        MH_TRY(run_forward(m, (int32_t)g.nodes.size()));
     if (pass == MH_PASS_FORWARD) return MH_OK;
     MH_TRY(mh_fill(m->gr[g.loss], 1.0f, numel(g.syms[g.loss].shape)));  // model.mojo:176-180
-    for (size_t k = g.nodes.size(); k-- > 0;) MH_TRY(run_backward_node(m, k));
-    return MH_OK;
+    return run_backward(m);
 }
 
 static void drop_graphs(mh_model* m) {
@@ -453,7 +928,7 @@ static void drop_graphs(mh_model* m) {
 
 static int execute(mh_model* m, int32_t nodes, const char* what) {
     PassScope ps;
-    for (int32_t i = 0; i < nodes; ++i) MH_TRY(run_forward_node(m, (size_t)i));
+    MH_TRY(run_forward(m, nodes));
     return ps.end(what);
 }
 
@@ -622,14 +1097,19 @@ int mh_model_create(const mh_graph* g, uint64_t flags, mh_model** out) {
         if (rc == MH_OK) rc = hip_check(hipStreamSynchronize(ctx().stream), "mh_model_create");
         (void)ps;
     }
+    if (rc == MH_OK) {
+        m->n_inference = inference_nodes(m->g);
+        plan_fusion(m);
+        rc = build_programs(m);
+    }
     if (rc != MH_OK) {
         if (m->arena) mh_free(m->arena);
         if (m->grad_arena) mh_free(m->grad_arena);
+        if (m->prog_mem) mh_free(m->prog_mem);
+        if (m->prog_part) mh_free(m->prog_part);
         delete m;
         return rc;
     }
-    m->n_inference = inference_nodes(m->g);
-    plan_fusion(m);
     *out = m;
     return MH_OK;
 }
@@ -643,6 +1123,11 @@ int mh_model_destroy(mh_model* m) {
         const int r2 = mh_free(m->grad_arena);
         if (rc == MH_OK) rc = r2;
     }
+    for (void* p : {m->prog_mem, static_cast<void*>(m->prog_part)})
+        if (p) {
+            const int r2 = mh_free(p);
+            if (rc == MH_OK) rc = r2;
+        }
     delete m;
     return rc;
 }
@@ -688,7 +1173,7 @@ int mh_model_backward(mh_model* m, int32_t nupper, const float* const* upper_gra
         if (!m->gr[last]) return fail(MH_ERR_INVALID, "mh_model_backward: the last node output is not trainable");
         MH_TRY(copy_in(m->gr[last], upper_grads[0], (size_t)numel(g.syms[last].shape), where));
     }
-    for (size_t k = g.nodes.size(); k-- > 0;) MH_TRY(run_backward_node(m, k));
+    MH_TRY(run_backward(m));
     if (nupper != 0 && where == MH_FROM_HOST) {  // pageable source: wait whatever the flags
         MH_HIP(hipStreamSynchronize(ctx().stream));
     }

@@ -1,0 +1,101 @@
+"""The executor's programs (runs of nodes as one launch) at the edges of their forms: one slab of
+short and long column sums, several slabs with a short last one, widths that are and are not a
+multiple of 4, rows by thread and by wavefront, and views just past a limit. Every tensor and
+gradient slot against the oracle running the graph node by node."""
+import numpy as np
+import pytest
+
+from mantle_amd import synth
+from util import O, OPS, GpuEngine, Graph, OracleEngine, assert_bitexact, assert_sum_close, native_graph
+
+pytestmark = pytest.mark.gpu
+ORC = OracleEngine()
+
+
+@pytest.fixture(scope="module")
+def gpu():
+    return GpuEngine()
+
+
+@pytest.fixture(autouse=True)
+def _nelts():
+    O.set_nelts(32)
+    yield
+
+
+# one slab (64 and 65 rows: the column sums' orders), its limit of 8192 elements, several slabs
+# (a last one of few rows), the widths 4096 / 8 rows and past it
+SHAPES = [(1, 7), (2, 2), (5, 64), (64, 33), (65, 33), (64, 128), (63, 130), (4096, 2), (4099, 2), (129, 65), (300, 40),
+          (2050, 31), (700, 512), (90, 513), (33, 300), (1025, 1024)]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+def test_layers(gpu, shape):
+    """Per-column, per-row and scalar operands in every place of the binary ops, the unary ops, and a
+    symbol used twice: tensors bit for bit, gradients bit for bit but for the sums over rows of more
+    than 64 and over a row of more than 64 (each compared as the sum of its own terms)."""
+    m = gpu.m
+    r, w = shape
+    vals = {"x": synth.normal(shape, 0, 1, 2200), "c": synth.uniform((1, w), 0.5, 1.5, 2201),
+            "d": synth.normal((w,), 0, 0.5, 2202), "p": synth.uniform((r, 1), 0.5, 1.5, 2203), "k": np.array([1.5], np.float32)}
+    nodes = [(OPS["MUL"], ["x", "c"], None, "h1"), (OPS["ADD"], ["h1", "d"], None, "h2"), (OPS["TANH"], ["h2"], None, "h3"),
+             (OPS["MUL"], ["h3", "h3"], None, "h4"), (OPS["SUB"], ["p", "h4"], None, "h5"), (OPS["DIV"], ["h5", "p"], None, "h6"),
+             (OPS["DIV"], ["h6", "c"], None, "h7"), (OPS["SIGMOID"], ["h7"], None, "h8"), (OPS["MUL"], ["h8", "k"], None, "h9"),
+             (OPS["RELU"], ["h9"], None, "h10"), (OPS["EXP"], ["h10"], None, "h11")]
+    trainable = ["x", "c", "d"] + (["p"] if r > 1 and w > 1 else [])
+    ref = Graph(nodes, trainable)
+    v = ref.forward(ORC, vals)
+    seed = synth.normal(shape, 0, 1, 2204)
+    gr = ref.backward(ORC, v, seed)
+    g, syms, inputs = native_graph(m, nodes, vals, trainable, params=("c", "d", "p", "k"))
+    g.out(syms["h11"])
+    model = m.Model(g)
+    for _ in range(2):  # the second pass from zeroed gradients again
+        model.parameters.grads.set_zero()
+        model.inference(*[vals[i] for i in inputs])
+        model.backward(seed)
+    P = model.parameters
+    for n in ["h%d" % i for i in range(1, 12)]:
+        assert_bitexact(P.tensors[syms[n]].to_numpy(), v[n], f"{shape} {n}")
+    long_col, long_row = r > 64, w > 64
+    if not long_row:  # the per-row operand's sums are in element order
+        assert_bitexact(P.grads[syms["x"]].to_numpy(), gr["x"], f"{shape} grad x")
+        if "p" in trainable:
+            assert_bitexact(P.grads[syms["p"]].to_numpy(), gr["p"], f"{shape} grad p")
+    # the sums over rows: d's terms are the gradient of h2, as the device holds it
+    terms = P.grads[syms["h2"]].to_numpy().astype(np.float64)
+    got = P.grads[syms["d"]].to_numpy()
+    if long_col:
+        assert_sum_close(got, gr["d"], terms.sum(axis=0), f"{shape} grad d", terms_abs=np.abs(terms).sum(axis=0))
+    elif not long_row:
+        assert_bitexact(got, gr["d"], f"{shape} grad d")
+        assert_bitexact(P.grads[syms["c"]].to_numpy(), gr["c"], f"{shape} grad c")
+    u1 = P.grads[syms["h1"]].to_numpy().astype(np.float64) * vals["x"].astype(np.float64)
+    h6, c64 = P.tensors[syms["h6"]].to_numpy().astype(np.float64), vals["c"].astype(np.float64)
+    u7 = -h6 / (c64 * c64) * P.grads[syms["h7"]].to_numpy().astype(np.float64)
+    assert_sum_close(P.grads[syms["c"]].to_numpy(), gr["c"], (u1 + u7).sum(axis=0, keepdims=True), f"{shape} grad c",
+                     terms_abs=(np.abs(u1) + np.abs(u7)).sum(axis=0, keepdims=True))
+
+
+@pytest.mark.parametrize("shape", [(1, 2), (3, 64), (9, 65), (40, 168), (4, 2047), (700, 9), (5001, 60), (1024, 8), (1030, 7)],
+                         ids=str)
+def test_head(gpu, shape):
+    """MAX, SUB, EXP, SUM, DIV, LOG, MUL, MEAN as programs: the gradient equals the same nodes run one
+    op call at a time on the device, bit for bit; so does the loss."""
+    m = gpu.m
+    x, t = synth.normal(shape, 0, 2, 2210), synth.uniform(shape, 0, 1, 2211)
+    synth.inject_ties(x, 1, 2212)
+    from util import config5_nodes
+    ref = Graph(config5_nodes(), ["logits"])
+    v = ref.forward(gpu, {"logits": x, "onehot": t})
+    gr = ref.backward(gpu, v, np.array([1.0], np.float32))
+    g, syms, inputs = native_graph(m, config5_nodes(), {"logits": x, "onehot": t}, ["logits"])
+    g.loss(syms["loss"])
+    model = m.Model(g)
+    loss = model.forward(*[{"logits": x, "onehot": t}[i] for i in inputs])
+    model.backward()
+    assert_bitexact(loss.to_numpy(), v["loss"], "loss")
+    for n in ("max", "xm", "e", "s", "sm", "lp", "t"):
+        assert_bitexact(model.parameters.tensors[syms[n]].to_numpy(), v[n], n)
+        assert_bitexact(model.parameters.grads[syms[n]].to_numpy(), gr[n], f"grad {n}")
+    assert_bitexact(model.parameters.grads[syms["logits"]].to_numpy(), gr["logits"], "grad logits")
