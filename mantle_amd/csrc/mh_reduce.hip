@@ -1908,22 +1908,31 @@ int plan_unbroadcast(const mh_shape& sgrad, const mh_shape& srg, mh_reduce_plan_
 // launch
 // ---------------------------------------------------------------------------------------
 // One wavefront per (channel c, group of G planes n = g * G .. g * G + G - 1, chunk k of QC
-// quads of each plane): lanes sum their quads of each plane in order, the planes in order
+// quads of each plane, at any alignment; the last chunk also takes a plane's last S % 4 elements,
+// one to a lane): lanes sum their quads of each plane in order, the planes in order
 // (two planes' loads in flight together), a butterfly adds the lanes, and the partial goes to
 // part[(g * K + k) * C + c] with an agent-scope store. The wave waits for the store, then
 // takes a ticket on channel c's counter (one per 128-byte line); the channel's last arrival
 // sums its NG * K partials in index order (lane-strided, then a butterfly) and accumulates
 // grad[c] (negated for SUB's operand 1), then resets the counter. G is chosen so that each
-// counter sees at most about kPlanesArrivals tickets: arrivals on one counter serialize.
+// counter sees at most about kPlanesArrivals tickets: arrivals on one counter serialize. KIND: the
+// terms are rg itself, or a MUL / DIV gradient's (FBinRg's expressions) of rg = ug, the full operand
+// a and, for DIV's operand 1, the channel's divisor t2[c]. Over [256, 96, 729] a MUL gradient was
+// written out, summed by rows and then by columns (33.7 + 16.2 + 10 us); SUB, MUL and DIV with their
+// gradients there took 309 us and take 243.
 constexpr int64_t kPlanesTicketStride = 32;
 constexpr int64_t kPlanesArrivals = 64;
 constexpr int64_t kPlanesMaxArrivals = 4096;
 constexpr int64_t kPlanesMaxQuads = 1024;
 
-template <bool NEG>
+enum PlaneKind : int { PL_RG = 0, PL_NEG = 1, PL_MUL = 2, PL_DIV0 = 3, PL_DIV1 = 4 };
+template <int KIND>
 __global__ void __launch_bounds__(kRThreads)
-    k_unb_planes(float* __restrict__ grad, const float* __restrict__ rg, int64_t N, int64_t C, int64_t Sq,
-                 int64_t QC, int64_t K, int64_t G, int64_t nwaves, float* part, uint32_t* tickets) {
+    k_unb_planes(float* __restrict__ grad, const float* __restrict__ rg, const float* __restrict__ a,
+                 const float* __restrict__ t2, int64_t N, int64_t C, int64_t S, int64_t QC, int64_t K, int64_t G,
+                 int64_t nwaves, float* part, uint32_t* tickets) {
+    constexpr bool NEG = KIND == PL_NEG, TWO = KIND >= PL_MUL;
+    const int64_t Sq = S >> 2;
     const int lane = threadIdx.x & 63;
     const int64_t v = (int64_t)blockIdx.x * (kRThreads / 64) + (threadIdx.x >> 6);
     if (v >= nwaves) return;  // uniform per wavefront; no barrier follows
@@ -1932,36 +1941,61 @@ __global__ void __launch_bounds__(kRThreads)
     const int64_t rem = Sq - k * QC;
     const int64_t cnt = rem < QC ? rem : QC;
     const int64_t n0 = g * G, n1 = n0 + G < N ? n0 + G : N;
-    // the lane's quads lane + 64 u of a 256-quad step at `base`, added in order
-    auto add_step = [&](float a, const vf4 (&q)[4], int64_t base) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (base + lane + 64 * u < cnt) a = (((a + q[u].x) + q[u].y) + q[u].z) + q[u].w;
-        return a;
+    const float d = KIND == PL_DIV1 ? t2[c] : 1.0f;
+    auto term = [&](float u, float v) {
+        if constexpr (KIND == PL_MUL) return u * v;
+        else if constexpr (KIND == PL_DIV0) return u / v;
+        else if constexpr (KIND == PL_DIV1) return ((-v) / (d * d)) * u;
+        else return u;
     };
-    auto load_step = [&](vf4 (&q)[4], const vf4* r, int64_t base) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (base + lane + 64 * u < cnt) q[u] = __builtin_nontemporal_load(r + base + lane + 64 * u);
+    struct Step {
+        vf4 u[4], v[TWO ? 4 : 1];
     };
-    auto add_rest = [&](float a, const vf4* r) {  // the plane's steps after the first
+    // the lane's quads lane + 64 j of a 256-quad step at `base`, added in order
+    auto add_step = [&](float s, const Step& q, int64_t base) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (base + lane + 64 * j < cnt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) s = s + term(q.u[j][i], TWO ? q.v[j][i] : 0.0f);
+        return s;
+    };
+    auto load_step = [&](Step& q, int64_t e, int64_t base) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (base + lane + 64 * j < cnt) {
+                q.u[j] = ld_ntu(rg + e + 4 * (base + lane + 64 * j));
+                if constexpr (TWO) q.v[j] = ld_ntu(a + e + 4 * (base + lane + 64 * j));
+            }
+    };
+    const int64_t rest = k == K - 1 ? 4 * (Sq - k * QC) : -1;  // the last S % 4 elements, from e + rest
+    const bool has = rest >= 0 && lane < (int)(S & 3);
+    auto add_rest = [&](float s, int64_t e, float tu, float tv) {  // the plane's steps after the first
         for (int64_t base = 256; base < cnt; base += 256) {
-            vf4 q[4];
-            load_step(q, r, base);
-            a = add_step(a, q, base);
+            Step q;
+            load_step(q, e, base);
+            s = add_step(s, q, base);
         }
-        return a;
+        return has ? s + term(tu, tv) : s;
     };
     float acc = 0.0f;
     for (int64_t n = n0; n < n1; n += 2) {  // planes in order; two planes' first steps in flight together
         const bool two = n + 1 < n1;
-        const vf4* ra = reinterpret_cast<const vf4*>(rg) + (n * C + c) * Sq + k * QC;
-        const vf4* rb = ra + C * Sq;
-        vf4 qa[4], qb[4];
-        load_step(qa, ra, 0);
-        if (two) load_step(qb, rb, 0);
-        acc = add_rest(add_step(acc, qa, 0), ra);
-        if (two) acc = add_rest(add_step(acc, qb, 0), rb);
+        const int64_t ea = (n * C + c) * S + 4 * k * QC, eb = ea + C * S;
+        Step qa, qb;
+        load_step(qa, ea, 0);
+        if (two) load_step(qb, eb, 0);
+        float ua = 0.0f, va = 0.0f, ub = 0.0f, vb = 0.0f;
+        if (has) {
+            ua = ld_nt(rg + ea + rest + lane);
+            if constexpr (TWO) va = ld_nt(a + ea + rest + lane);
+            if (two) {
+                ub = ld_nt(rg + eb + rest + lane);
+                if constexpr (TWO) vb = ld_nt(a + eb + rest + lane);
+            }
+        }
+        acc = add_rest(add_step(acc, qa, 0), ea, ua, va);
+        if (two) acc = add_rest(add_step(acc, qb, 0), eb, ub, vb);
     }
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) acc = acc + __shfl_xor(acc, m);
@@ -1995,13 +2029,13 @@ struct PlaneForm {
     int64_t N, C, S, Sq, QC, K, G, NG, nwaves;
 };
 
-// The plan [N*C, S, 1] then [1, N, C] with S a multiple of 4 and at least 64.
+// The plan [N*C, S, 1] then [1, N, C] with S of at least 64.
 static bool plane_form(const mh_reduce_plan_info& p, PlaneForm* f) {
     if (p.nsteps != 2 || p.c[0] != 1 || p.a[1] != 1 || p.a[0] != p.b[1] * p.c[1]) return false;
     f->N = p.b[1];
     f->C = p.c[1];
     f->S = p.b[0];
-    if (f->S % 4 != 0 || f->S < 64 || f->N * f->C < 1) return false;
+    if (f->S < 64 || f->N * f->C < 1) return false;
     f->Sq = f->S / 4;
     f->QC = f->Sq < kPlanesMaxQuads ? f->Sq : kPlanesMaxQuads;
     f->K = (f->Sq + f->QC - 1) / f->QC;
@@ -2010,6 +2044,16 @@ static bool plane_form(const mh_reduce_plan_info& p, PlaneForm* f) {
     f->NG = (f->N + f->G - 1) / f->G;
     f->nwaves = f->NG * f->K * f->C;
     return f->NG * f->K <= kPlanesMaxArrivals && (f->nwaves + 3) / 4 <= 0x7fffffff;
+}
+
+// Launches k_unb_planes; tmp holds NG * K * C partials.
+template <int KIND>
+static int launch_planes(const PlaneForm& f, float* grad, const float* rg, const float* a, const float* t2, float* tmp) {
+    uint32_t* tk = nullptr;
+    MH_TRY(tickets(f.C * kPlanesTicketStride, &tk));
+    hipLaunchKernelGGL(k_unb_planes<KIND>, dim3((unsigned)((f.nwaves + 3) / 4)), dim3(kRThreads), 0, ctx().stream, grad,
+                       rg, a, t2, f.N, f.C, f.S, f.QC, f.K, f.G, f.nwaves, tmp, tk);
+    return MH_OK;
 }
 
 size_t unbroadcast_scratch_floats(const mh_shape& sgrad, const mh_shape& srg) {
@@ -2043,18 +2087,9 @@ int unbroadcast_accum_scratch(float* grad, const mh_shape& sgrad, const float* r
     if (p.nsteps == 0)  // only size-1 dims differ: same element order
         return reduce_abc(RED_SUM, final_epi, rg, numel(srg), 1, 1, grad, nullptr, 0.0f, nullptr);
     PlaneForm pf;
-    if (al16(rg) && plane_form(p, &pf)) {  // a per-channel bias gradient: one launch
-        uint32_t* tk = nullptr;
-        MH_TRY(tickets(pf.C * kPlanesTicketStride, &tk));
-        dim3 g((unsigned)((pf.nwaves + 3) / 4)), b(kRThreads);
-        if (negate)
-            hipLaunchKernelGGL(k_unb_planes<true>, g, b, 0, ctx().stream, grad, rg, pf.N, pf.C, pf.Sq, pf.QC, pf.K,
-                               pf.G, pf.nwaves, tmp, tk);
-        else
-            hipLaunchKernelGGL(k_unb_planes<false>, g, b, 0, ctx().stream, grad, rg, pf.N, pf.C, pf.Sq, pf.QC,
-                               pf.K, pf.G, pf.nwaves, tmp, tk);
-        return MH_OK;
-    }
+    if (plane_form(p, &pf))  // a per-channel bias gradient: one launch
+        return negate ? launch_planes<PL_NEG>(pf, grad, rg, nullptr, nullptr, tmp)
+                      : launch_planes<PL_RG>(pf, grad, rg, nullptr, nullptr, tmp);
     size_t tmax = 0, bmax = 0;
     for (int i = 0; i < p.nsteps; ++i) {
         size_t t = reduce_abc_tmp_floats(RED_SUM, p.a[i], p.b[i], p.c[i]);
@@ -2189,6 +2224,16 @@ int unbroadcast_binrg(int op, int id, bool divs, float* grad, const mh_shape& sg
     if (!shape_eq(id == 0 ? s2 : s1, sug)) return MH_OK;
     mh_reduce_plan_info p;
     MH_TRY(plan_unbroadcast(sgrad, sug, &p));
+    PlaneForm pf;
+    if (!divs && plane_form(p, &pf)) {  // a per-channel operand: one launch
+        float* part = nullptr;
+        MH_TRY(scratch(((size_t)(pf.NG * pf.K * pf.C) + 64) * sizeof(float), reinterpret_cast<void**>(&part)));
+        if (op == MH_MUL) MH_TRY(launch_planes<PL_MUL>(pf, grad, ug, a, nullptr, part));
+        else if (id == 0) MH_TRY(launch_planes<PL_DIV0>(pf, grad, ug, a, nullptr, part));
+        else MH_TRY(launch_planes<PL_DIV1>(pf, grad, ug, a, t2, part));
+        *done = true;
+        return MH_OK;
+    }
     if (p.nsteps > 1) return MH_OK;
     int64_t A = numel(sug), B = 1, C = 1;  // only size-1 dims differ: element for element
     if (p.nsteps == 1) {

@@ -163,3 +163,23 @@ def test_reduce_backward_short_axes(gpu, shape, axis):
     """Reductions over an axis too short to split: the line operands of SUM, MEAN and MAX backward
     broadcast over it."""
     reductions_match(gpu, shape, axis)
+
+
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("shape", [(3, 5, 64), (2, 3, 65), (70, 3, 67), (5, 2, 729), (1, 4, 4099), (2, 2, 4102), (3, 1, 130)],
+                         ids=str)
+def test_channel_gradients(gpu, shape, off):
+    """The gradient of a per-channel operand [1, C, 1] over planes of every length modulo 4, one and
+    several chunks a plane, in either place of the binary ops; ug also at an unaligned address."""
+    m = gpu.m
+    x, b = synth.uniform(shape, 0.5, 2, 2150), synth.uniform((1, shape[1], 1), 0.5, 2, 2151)
+    ug, g0 = synth.normal(shape, 0, 1, 2152), synth.normal((1, shape[1], 1), 0, 1, 2153)
+    x64, b64, u64 = (v.astype(np.float64) for v in (x, b, ug))
+    for name, i, rg in (("ADD", 1, u64), ("SUB", 1, -u64), ("SUB", 0, u64), ("MUL", 0, u64 * x64), ("MUL", 1, u64 * x64),
+                        ("DIV", 0, u64 / x64), ("DIV", 1, -x64 / (b64 * b64) * u64)):
+        t1, t2 = (b, x) if i == 0 else (x, b)
+        g = gpu.T(g0)
+        m.backward_op(i, OPS[name], view(gpu, ug, off), gpu.T(t1), gpu.T(t2), g)
+        ref = O.backward_op(i, OPS[name], ug, t1, t2, grad=g0)
+        assert_sum_close(g.to_numpy(), ref, rg.sum(axis=(0, 2), keepdims=True) + g0, f"{name} id {i} {shape}",
+                         terms_abs=np.abs(rg).sum(axis=(0, 2), keepdims=True) + np.abs(g0))
