@@ -336,6 +336,8 @@ int reduce_abc(int op, int epi, const float* x, int64_t A, int64_t B, int64_t C,
 // grad_x, the x gradient of every element is accumulated into grad_x in the same pass.
 int pow_exponent_grad(float* grad, const float* x, const float* exponent, const float* ug,
                       int64_t n, float* grad_x = nullptr);
+// out[c] += the sum over s of part[s * n + c], in a fixed order.
+void reduce_parts_accum(float* part, int64_t S, int64_t n, float* out);
 // grad += un-broadcast(rg) (or += -un-broadcast(rg)): the chain of single-axis reductions.
 size_t unbroadcast_scratch_floats(const mh_shape& sgrad, const mh_shape& srg);
 int unbroadcast_accum_scratch(float* grad, const mh_shape& sgrad, const float* rg,

@@ -1826,6 +1826,10 @@ static int reduce_t(LD ld, bool vec_ok, int epi, int64_t A, int64_t B, int64_t C
     return MH_OK;
 }
 
+void reduce_parts_accum(float* part, int64_t S, int64_t n, float* out) {
+    combine_parts<RSum>(part, S, n, EPI_ACCUM, out, nullptr, 0.0f);
+}
+
 int reduce_abc(int op, int epi, const float* x, int64_t A, int64_t B, int64_t C, float* out, float* out2,
                float div, float* tmp, RedSplit* split) {
     const bool al = al16(x);

@@ -183,3 +183,32 @@ def test_channel_gradients(gpu, shape, off):
         ref = O.backward_op(i, OPS[name], ug, t1, t2, grad=g0)
         assert_sum_close(g.to_numpy(), ref, rg.sum(axis=(0, 2), keepdims=True) + g0, f"{name} id {i} {shape}",
                          terms_abs=np.abs(rg).sum(axis=(0, 2), keepdims=True) + np.abs(g0))
+
+
+@pytest.mark.parametrize("rows,cols", [(65, 4), (64, 8), (70, 5), (300, 33), (4500, 6), (130, 511), (97, 512), (66, 1030),
+                                       (129, 1027)])
+def test_linear_bias_relu(gpu, rows, cols):
+    """Bias + RELU over [rows, features], one pass each way: outputs and per-element gradients bit for
+    bit the op-by-op calls', the bias gradient in the sum class; with and without the kept gradients."""
+    m = gpu.m
+    x, b = synth.normal((rows, cols), 0, 1, 2160), synth.normal((1, cols), 0, 0.5, 2161)
+    x[::3] = 0.0
+    b[:, ::2] = -0.0
+    ug, g0, gb0 = synth.normal((rows, cols), 0, 1, 2162), synth.normal((rows, cols), 0, 1, 2163), synth.normal((1, cols), 0, 1, 2164)
+    y, r = gpu.T(np.zeros_like(x)), gpu.T(np.zeros_like(x))
+    m.bias_relu_forward(y, r, gpu.T(x), gpu.T(b))
+    yr = ORC.forward(OPS["ADD"], x, b)
+    assert_bitexact(y.to_numpy(), yr, "y")
+    assert_bitexact(r.to_numpy(), ORC.forward(OPS["RELU"], yr), "r")
+    for keep_y, keep_x in ((True, True), (False, True), (True, False), (False, False)):
+        gy = ORC.backward(0, OPS["RELU"], ug, yr, grad=g0 if keep_y else np.zeros_like(x))
+        ty, tx, tb = gpu.T(g0), gpu.T(g0), gpu.T(gb0)
+        m.bias_relu_backward(gpu.T(ug), y, b.shape, tx if keep_x else None, tb, ty if keep_y else None)
+        if keep_y:
+            assert_bitexact(ty.to_numpy(), gy, "grad y")
+        if keep_x:
+            assert_bitexact(tx.to_numpy(), ORC.backward(0, OPS["ADD"], gy, x, b, grad=g0), "grad x")
+        g64 = gy.astype(np.float64)
+        assert_sum_close(tb.to_numpy(), O.backward_op(1, OPS["ADD"], gy, x, b, grad=gb0),
+                         g64.sum(axis=0, keepdims=True) + gb0, "grad bias",
+                         terms_abs=np.abs(g64).sum(axis=0, keepdims=True) + np.abs(gb0))
