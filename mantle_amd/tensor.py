@@ -38,7 +38,7 @@ def sync() -> None:
 class TensorShape:
     """Row-major shape of rank 1..8 (tensor.mojo:28-229)."""
 
-    __slots__ = ("_dims",)
+    __slots__ = ("_dims", "_n", "_cs")
 
     def __init__(self, *dims: Union[int, Iterable[int]]):
         if len(dims) == 1 and not isinstance(dims[0], (int, np.integer)):
@@ -47,15 +47,17 @@ class TensorShape:
         if not 1 <= len(d) <= MAX_RANK:
             raise ValueError(f"rank {len(d)} outside 1..{MAX_RANK}")
         self._dims = d
+        n = 1
+        for x in d:
+            n *= x
+        self._n = n
+        self._cs = None
 
     def rank(self) -> int:
         return len(self._dims)
 
     def num_elements(self) -> int:
-        n = 1
-        for x in self._dims:
-            n *= x
-        return n
+        return self._n
 
     def strides(self) -> Tuple[int, ...]:  # tensor.mojo:143-155
         st, s = [], 1
@@ -88,7 +90,11 @@ class TensorShape:
         return "TensorShape(" + ", ".join(str(x) for x in self._dims) + ")"
 
     def c(self) -> _lib.mh_shape:
-        return _lib.make_shape(self._dims)
+        """The shape as the C ABI takes it (read during the call), made once: a shape never changes,
+        and the four of a binary gradient's call cost more to make than its launch."""
+        if self._cs is None:
+            self._cs = _lib.make_shape(self._dims)
+        return self._cs
 
 
 def as_shape(s) -> TensorShape:
