@@ -1144,7 +1144,7 @@ WL_KERNELS = [
      "grad_x read and written; a wave's plane partials into the slot table"),
     ("c3 bias_relu.bwd (fused), combine", "mh::k_bias_partials_comb8", 8192, 4 * 8 * (_N3 // 784) + 256,
      "the slot table (8 slots per plane) read, 32 bias values updated"),
-    ("c3 ADD.bwd_bias", "void mh::k_unb_planes<false>", 131072, 4 * _N3 + 256, "one launch, arrival tickets"),
+    ("c3 ADD.bwd_bias", "void mh::k_unb_planes<0>", 131072, 4 * _N3 + 256, "one launch, arrival tickets"),
     ("c4 [8192,8192] axis 0 MAX.fwd", "void mh::k_cols<mh::RMax, mh::LdPlain<mh::RMax>, true, true>", 262144,
      4 * _N4, "first of two launches (split partials)"),
     ("c4 [8192,8192] axis 0 MAX.bwd, route", "void mh::k_max_route_cols<true>", 262144, 4 * _N4,
@@ -1166,13 +1166,13 @@ WL_KERNELS = [
     ("c5 fused head forward", "void mh::k_rowo_fwd<0, 10>", 1048576, 8 * _N5,
      "logits and targets read once; 64 KB of block partials written for k_loss_comb<0>"),
     ("c5 fused head backward", "void mh::k_rowo_bwd<0, 10>", 1048576, 16 * _N5, ""),
-    ("CrossEntropy [32768,1000] backward", "void mh::k_roww_bwd<1, true, 16>", 2097152, 16 * 32768000, ""),
+    ("CrossEntropy [32768,1000] backward", "void mh::k_roww_bwd<1, true, 16, 64, 3>", 2097152, 16 * 32768000, ""),
 ]
 
 
 # (workload, group, op label, kernel-name prefix) of single-shape workload kernels whose
 # rocprofv3 duration the stats summary sets beside the bench's figures
-WL_STATS = [("c3", "op_by_op", "ADD.bwd_bias", "void mh::k_unb_planes<false>"),
+WL_STATS = [("c3", "op_by_op", "ADD.bwd_bias", "void mh::k_unb_planes<0>"),
             ("c3", "fused", "bias_relu.fwd", "mh::k_bias_relu_fwd_planes"),
             ("c3", "op_by_op", "ADD.fwd", "void mh::k_planebc4<mh::FBin<0>, 2, false, 8>"),
             ("c3", "fused", "bias_relu.bwd", ("void mh::k_bias_relu_bwd_flat<false, true, true, true>",
