@@ -271,6 +271,7 @@ __device__ __forceinline__ void prog_max_bwd(const ProgInstr& in, const Slab& s,
     };
     if (s.W <= 64) {  // a row per thread finds (max, factor), then the slab's quads in flat order
         const int32_t cnt = s.rows * s.W;
+        __syncthreads();  // sm and sg: an instruction of this kind just before may still be read
         for (int32_t i = threadIdx.x; i < s.rows; i += NT) {
             const float* x = in.a + s.e0 + (int64_t)i * s.W;
             float m = -FLT_MAX;

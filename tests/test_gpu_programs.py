@@ -99,3 +99,25 @@ def test_head(gpu, shape):
         assert_bitexact(model.parameters.tensors[syms[n]].to_numpy(), v[n], n)
         assert_bitexact(model.parameters.grads[syms[n]].to_numpy(), gr[n], f"grad {n}")
     assert_bitexact(model.parameters.grads[syms["logits"]].to_numpy(), gr["logits"], "grad logits")
+
+
+@pytest.mark.parametrize("shape", [(5, 7), (128, 64), (1024, 8), (5001, 60)], ids=str)
+def test_two_maxima_in_a_row(gpu, shape):
+    """The gradients of two MAX nodes one after the other in a run, whose rows' maxima pass through the
+    same shared memory: bit for bit what the nodes' own calls give."""
+    m = gpu.m
+    vals = {"a": synth.normal(shape, 0, 1, 2220), "b": synth.normal(shape, 3, 1, 2221)}
+    synth.inject_ties(vals["a"], 1, 2222)
+    nodes = [(OPS["MAX"], ["a"], 1, "ma"), (OPS["MAX"], ["b"], 1, "mb"),
+             (OPS["MUL"], ["ma", "mb"], None, "h")]
+    seed = synth.normal((shape[0], 1), 0, 1, 2223)
+    ref = Graph(nodes, ["a", "b"])
+    v = ref.forward(gpu, vals)
+    gr = ref.backward(gpu, v, seed)
+    g, syms, inputs = native_graph(m, nodes, vals, ["a", "b"])
+    g.out(syms["h"])
+    model = m.Model(g)
+    model.inference(*[vals[i] for i in inputs])
+    model.backward(seed)
+    for n in ("a", "b"):
+        assert_bitexact(model.parameters.grads[syms[n]].to_numpy(), gr[n], f"{shape} grad {n}")
