@@ -48,6 +48,7 @@ class mh_launch_info(ctypes.Structure):
 
 (LAUNCH_FILL, LAUNCH_FILL_UNALIGNED, LAUNCH_COPY, LAUNCH_SAME_SHAPE, LAUNCH_ADAM, LAUNCH_ADAM_UNALIGNED,
  LAUNCH_ROWS16) = range(7)
+PLAN_COLUMNS, PLAN_MAX_BACKWARD, PLAN_CHANNELS = range(3)
 
 
 class mh_attrs(ctypes.Structure):
@@ -164,6 +165,7 @@ SIGNATURES = {
     "mh_plan_binary": [_S, _S, _S, ctypes.POINTER(mh_plan_info)],
     "mh_plan_unbroadcast": [_S, _S, ctypes.POINTER(mh_reduce_plan_info)],
     "mh_plan_launch": [ctypes.c_int32, _I64, ctypes.POINTER(mh_launch_info)],
+    "mh_plan_reduction": [ctypes.c_int32, _I64, _I64, _I64, ctypes.c_int32, ctypes.POINTER(mh_launch_info)],
 }
 _RESTYPE = {"mh_last_error": ctypes.c_char_p, "mh_status_string": ctypes.c_char_p}
 

@@ -1662,12 +1662,50 @@ static size_t row_tmp_floats(int64_t A, int64_t B, bool combine = false) {
     return pad64((size_t)(A * S) * part_words<R>()) + row_tmp_floats<R>(A, S, true);
 }
 
+// One dispatch holds fewer than 2^32 work-items per grid dimension.
+static inline bool fits_dispatch(int64_t blocks, int64_t threads = kRThreads) {
+    return blocks <= (((int64_t)1 << 32) - 1) / threads;
+}
+
+// The form of a strided reduction over [A, B, C] (C > 1) and its launch: gx x gy blocks, S splits
+// of rps rows.
+enum ColForm : int { CF_WIDE = 0, CF_STRIP = 1, CF_QUADS = 2, CF_SINGLES = 3 };
+struct ColPlan {
+    ColForm form;
+    int64_t S, rps, gx, gy, nstrips;
+};
+static ColPlan col_plan(int64_t A, int64_t B, int64_t C) {
+    const int64_t quads = A * ((C + 3) / 4), qb = (quads + kRThreads - 1) / kRThreads;
+    ColPlan p{};
+    ColSplit cs;
+    // the wide layout puts the column-quad blocks on grid y (at most 65535 blocks there)
+    if (use_wide_cols(C) && qb <= 65535) {
+        cs = wide_split(A, B, C);
+        p.form = CF_WIDE;
+        p.gx = cs.S;
+        p.gy = qb;
+    } else if (use_strip(C) && fits_dispatch(A * (((C + 3) / 4 + 63) / 64))) {
+        cs = strip_split(A, B, C, &p.nstrips);
+        p.form = CF_STRIP;
+        p.gx = A * p.nstrips;
+        p.gy = cs.S;
+    } else {
+        cs = col_split(A, B, C);
+        p.form = cs.vec ? CF_QUADS : CF_SINGLES;
+        p.gx = cs.vec ? qb : (A * C + kRThreads - 1) / kRThreads;
+        p.gy = cs.S;
+    }
+    p.S = cs.S;
+    p.rps = cs.rps;
+    return p;
+}
+
 // Scratch floats a reduction of [A, B, C] needs for its partials.
 template <class R>
 static size_t tmp_floats_t(int64_t A, int64_t B, int64_t C) {
     if (A * C == 0) return 0;
     if (C == 1) return row_tmp_floats<R>(A, B);
-    // the largest split any column launcher may pick
+    // the largest split any form may pick
     int64_t S = col_split(A, B, C).S;
     if (use_wide_cols(C)) {
         const int64_t sw = wide_split(A, B, C).S;
@@ -1798,26 +1836,22 @@ static int reduce_t(LD ld, bool vec_ok, int epi, int64_t A, int64_t B, int64_t C
         }
         return MH_OK;
     }
-    // the wide layout puts the column-quad blocks on grid y (at most 65535 blocks there);
-    // larger outputs take the strips below
-    const int64_t quads = A * ((C + 3) / 4);
-    ColSplit cs;
-    if (use_wide_cols(C) && (quads + kRThreads - 1) / kRThreads <= 65535) {
-        cs = wide_split(A, B, C);
-        dim3 g((unsigned)cs.S, (unsigned)((quads + kRThreads - 1) / kRThreads)), b(kRThreads);
-        hipLaunchKernelGGL((k_cols<R, LD, true, true>), g, b, 0, st, ld, A, B, C, cs.rps, cs.S, out, out2, epi, div,
-                           tmp);
-    } else if (use_strip(C)) {
-        int64_t ns;
-        cs = strip_split(A, B, C, &ns);
-        dim3 g((unsigned)(A * ns), (unsigned)cs.S), b(kRThreads);
-        hipLaunchKernelGGL((k_cols_strip<R, LD>), g, b, 0, st, ld, A, B, C, ns, cs.rps, cs.S, out, out2, epi, div, tmp);
-    } else {
-        cs = col_split(A, B, C);
-        const int64_t items = cs.vec ? quads : A * C;
-        dim3 g((unsigned)((items + kRThreads - 1) / kRThreads), (unsigned)cs.S), b(kRThreads);
-        if (cs.vec) hipLaunchKernelGGL((k_cols<R, LD, true>), g, b, 0, st, ld, A, B, C, cs.rps, cs.S, out, out2, epi, div, tmp);
-        else hipLaunchKernelGGL((k_cols<R, LD, false>), g, b, 0, st, ld, A, B, C, cs.rps, cs.S, out, out2, epi, div, tmp);
+    const ColPlan cs = col_plan(A, B, C);
+    const dim3 g((unsigned)cs.gx, (unsigned)cs.gy), b(kRThreads);
+    switch (cs.form) {
+        case CF_WIDE:
+            hipLaunchKernelGGL((k_cols<R, LD, true, true>), g, b, 0, st, ld, A, B, C, cs.rps, cs.S, out, out2, epi, div, tmp);
+            break;
+        case CF_STRIP:
+            hipLaunchKernelGGL((k_cols_strip<R, LD>), g, b, 0, st, ld, A, B, C, cs.nstrips, cs.rps, cs.S, out, out2, epi,
+                               div, tmp);
+            break;
+        case CF_QUADS:
+            hipLaunchKernelGGL((k_cols<R, LD, true>), g, b, 0, st, ld, A, B, C, cs.rps, cs.S, out, out2, epi, div, tmp);
+            break;
+        default:
+            hipLaunchKernelGGL((k_cols<R, LD, false>), g, b, 0, st, ld, A, B, C, cs.rps, cs.S, out, out2, epi, div, tmp);
+            break;
     }
     if (cs.S > 1) {
         if (split) *split = RedSplit{cs.S, cs.rps};
@@ -2047,7 +2081,7 @@ static bool plane_form(const mh_reduce_plan_info& p, PlaneForm* f) {
     if (f->G < 1) f->G = 1;
     f->NG = (f->N + f->G - 1) / f->G;
     f->nwaves = f->NG * f->K * f->C;
-    return f->NG * f->K <= kPlanesMaxArrivals && (f->nwaves + 3) / 4 <= 0x7fffffff;
+    return f->NG * f->K <= kPlanesMaxArrivals && fits_dispatch((f->nwaves + 3) / 4);
 }
 
 // Launches k_unb_planes; tmp holds NG * K * C partials.
@@ -2372,7 +2406,7 @@ int pow_exponent_grad(float* grad, const float* x, const float* exponent, const 
                       float* grad_x) {
     LdPowGrad ld{x, ug, exponent, 0.0f, grad_x, 0.0f, false};
     float* tmp = nullptr;
-    if (n / 4 >= kPowStreamMinQuads && n / 4 / kPowThreads < 0x7fffffff) {
+    if (n / 4 >= kPowStreamMinQuads && fits_dispatch((n / 4 + kPowThreads - 1) / kPowThreads, kPowThreads)) {
         // run partials, then a row reduction of them into grad
         const int64_t nq = n / 4;
         const int64_t G = (nq + kPowThreads - 1) / kPowThreads;  // runs of 64 quads
@@ -2401,6 +2435,17 @@ int map_max_route(float* grad, const mh_shape& sx, const float* x, const mh_shap
                   const float* f, const float* ug);
 int map_scale_bcast(float* grad, const mh_shape& sx, const float* ug, const mh_shape& sug, float c, bool twice);
 int map_mean_all(float* grad, int64_t n, const float* ug, float c);
+
+// The form of a MAX backward over [A, B, C] (B >= 1): rows staged as tiles, rows held in registers by
+// a wavefront or a block each, or a max-count reduction and a routing pass.
+enum MaxForm : int { MF_TILES = 0, MF_WAVE = 1, MF_BLOCK = 2, MF_TWO_PASS = 3 };
+static MaxForm max_bwd_form(int64_t A, int64_t B, int64_t C, bool al) {
+    if (C != 1 || B > 16384) return MF_TWO_PASS;
+    if (B <= 32 && al) return A < kMaxGridRows ? MF_TILES : MF_TWO_PASS;
+    // a row per wavefront or block, as long as one dispatch holds them
+    if (B <= 4096) return fits_dispatch((A + 3) / 4) ? MF_WAVE : MF_TWO_PASS;
+    return fits_dispatch(A) ? MF_BLOCK : MF_TWO_PASS;
+}
 
 static void abc_of(const mh_shape& s, int axis, int64_t* A, int64_t* B, int64_t* C) {
     if (axis < 0) {
@@ -2608,6 +2653,7 @@ int mh_reduce_bwd_accum(int op, float* grad, const float* x, const mh_shape* psx
     const mh_shape sug = reduced_shape(sx, axis);
     int64_t A, B, C;
     abc_of(sx, axis, &A, &B, &C);
+    const MaxForm mf = max_bwd_form(A, B, C, al16(x) && al16(grad));
     if (op == MH_SUM) {  // basics.mojo:416-425
         MH_TRY(map_scale_bcast(grad, sx, ug, sug, 1.0f, shape_eq(sx, sug)));
     } else if (op == MH_MEAN) {
@@ -2616,7 +2662,7 @@ int mh_reduce_bwd_accum(int op, float* grad, const float* x, const mh_shape* psx
         } else {  // basics.mojo:489-506
             MH_TRY(map_scale_bcast(grad, sx, ug, sug, (float)(1.0 / (double)B), shape_eq(sx, sug)));
         }
-    } else if (C == 1 && B >= 1 && B <= 32 && A < kMaxGridRows && al16(x) && al16(grad)) {
+    } else if (mf == MF_TILES) {
         // MAX over short last-axis rows: one pass (max, count and routing per LDS tile)
         const unsigned blocks = (unsigned)((A + kLdsRows - 1) / kLdsRows);
         const FastDiv fdB = make_fastdiv((uint32_t)B);
@@ -2626,11 +2672,11 @@ int mh_reduce_bwd_accum(int op, float* grad, const float* x, const mh_shape* psx
         else
             hipLaunchKernelGGL(k_max_bwd_rows<32>, dim3(blocks), dim3(kLdsRows), 0, ctx().stream, grad, x, ug, A,
                                (int)B, fdB);
-    } else if (C == 1 && B <= 16384 && A < ((int64_t)1 << 31)) {
+    } else if (mf == MF_WAVE || mf == MF_BLOCK) {
         // MAX over rows held in registers: one pass
         const int64_t Bq = (B + 3) / 4;
         hipStream_t st = ctx().stream;
-        if (Bq <= 64 * 16) {  // one wave per row, four rows per block
+        if (mf == MF_WAVE) {  // four rows per block
             const int nq = Bq <= 64 ? 1 : Bq <= 128 ? 2 : Bq <= 256 ? 4 : Bq <= 512 ? 8 : 16;
             dim3 g((unsigned)((A + 3) / 4)), b(kRThreads);
 #define MH_MBR(NQ) hipLaunchKernelGGL((k_max_bwd_rowreg<1, NQ>), g, b, 0, st, grad, x, ug, A, B)
@@ -2671,6 +2717,43 @@ int mh_reduce_bwd_accum(int op, float* grad, const float* x, const mh_shape* psx
         if (!max_route_split(grad, x, A, B, C, m, f, ug, tmp, sp, arg)) MH_TRY(map_max_route(grad, sx, x, sug, m, f, ug));
     }
     return finish("mh_reduce_bwd_accum");
+}
+
+int mh_plan_reduction(int32_t what, int64_t A, int64_t B, int64_t C, int32_t aligned, mh_launch_info* out) {
+    if (!out) return fail(MH_ERR_NULL, "mh_plan_reduction: null");
+    if (A < 1 || B < 1 || C < 1) return fail(MH_ERR_INVALID, "mh_plan_reduction: empty shape");
+    out->threads = kRThreads;
+    switch (what) {
+        case MH_PLAN_COLUMNS: {
+            if (C == 1) return fail(MH_ERR_INVALID, "mh_plan_reduction: columns need C > 1");
+            const ColPlan p = col_plan(A, B, C);
+            out->kernel = p.form;
+            out->blocks = p.gx;
+            out->launches = p.S > 1 ? 2 : 1;
+            return MH_OK;
+        }
+        case MH_PLAN_MAX_BACKWARD: {
+            const MaxForm f = max_bwd_form(A, B, C, aligned != 0);
+            out->kernel = f;
+            out->threads = f == MF_TILES ? kLdsRows : kRThreads;
+            out->blocks = f == MF_TILES ? (A + kLdsRows - 1) / kLdsRows : f == MF_WAVE ? (A + 3) / 4 : f == MF_BLOCK ? A : 0;
+            out->launches = f == MF_TWO_PASS ? 0 : 1;
+            return MH_OK;
+        }
+        case MH_PLAN_CHANNELS: {
+            mh_reduce_plan_info p{};
+            p.nsteps = 2;
+            p.a[0] = A * B; p.b[0] = C; p.c[0] = 1;
+            p.a[1] = 1; p.b[1] = A; p.c[1] = B;
+            PlaneForm f;
+            const bool one = plane_form(p, &f);
+            out->kernel = one ? 1 : 0;
+            out->blocks = one ? (f.nwaves + 3) / 4 : 0;
+            out->launches = one ? 1 : 0;
+            return MH_OK;
+        }
+        default: return fail(MH_ERR_INVALID, "mh_plan_reduction: unknown plan %d", what);
+    }
 }
 
 }  // extern "C"

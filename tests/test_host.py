@@ -317,3 +317,38 @@ def test_row_engine_launches_split_rows_past_one_dispatch():
         assert info.blocks == min(nb, ((1 << 32) - 1) // 64), (rows, info.blocks)
         assert info.blocks * 64 * info.launches >= rows > info.blocks * 64 * (info.launches - 1), rows
     assert L.mh_plan_launch(0, -1, ctypes.byref(info)) == _lib.ERR_INVALID
+
+
+def plan_reduction(what, a, b, c, aligned=1):
+    info = _lib.mh_launch_info()
+    assert _lib.lib().mh_plan_reduction(what, a, b, c, aligned, ctypes.byref(info)) == 0, _lib.last_error()
+    return info
+
+
+@pytest.mark.parametrize("rows,b,aligned", [((1 << 26) - 4, 33, 1), ((1 << 26) - 3, 33, 1), (1 << 27, 63, 1), (1 << 26, 2, 0),
+                                            (1 << 28, 1, 0), ((1 << 24) - 1, 4097, 1), (1 << 24, 4097, 1), (1 << 33, 3, 1)])
+def test_max_backward_rows_past_one_dispatch(rows, b, aligned):
+    """A MAX backward takes a wavefront or a workgroup per row only where one dispatch holds the rows;
+    more rows go through the max-count reduction and the routing pass, which loop over theirs."""
+    info = plan_reduction(_lib.PLAN_MAX_BACKWARD, rows, b, 1, aligned)
+    assert info.blocks * info.threads < (1 << 32), (info.kernel, info.blocks)
+    covered = {0: 64, 1: 4, 2: 1}.get(info.kernel)
+    assert info.kernel == 3 or info.blocks * covered >= rows
+    if b > 32:
+        assert info.kernel == (3 if rows >= ((1 << 26) - 3 if b <= 4096 else 1 << 24) else 1 if b <= 4096 else 2)
+
+
+@pytest.mark.parametrize("a,c", [((1 << 24) - 1, 129), (1 << 24, 129), ((1 << 25) - 1, 129), (1 << 23, 257), (1 << 23, 1023),
+                                 (1 << 22, 1025), (1 << 26, 5), (1 << 30, 3)])
+def test_strided_reductions_past_one_dispatch(a, c):
+    """Every form of a reduction over the middle axis fits one dispatch; slabs too many for strips go
+    by column quads."""
+    info = plan_reduction(_lib.PLAN_COLUMNS, a, 2, c)
+    assert info.blocks * info.threads < (1 << 32), (info.kernel, info.blocks)
+
+
+def test_channel_gradients_past_one_dispatch():
+    """The one-launch plane kernel takes only as many wavefronts as one dispatch holds."""
+    for n, c, s in ((2, 1 << 25, 64), (2, 1 << 26, 64), (2, 1 << 26, 65), (64, 1 << 20, 64), (64, (1 << 20) + 1, 64)):
+        info = plan_reduction(_lib.PLAN_CHANNELS, n, c, s)
+        assert info.blocks * info.threads < (1 << 32), (n, c, s)
