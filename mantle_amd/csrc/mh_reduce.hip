@@ -2441,7 +2441,10 @@ int map_mean_all(float* grad, int64_t n, const float* ug, float c);
 enum MaxForm : int { MF_TILES = 0, MF_WAVE = 1, MF_BLOCK = 2, MF_TWO_PASS = 3 };
 static MaxForm max_bwd_form(int64_t A, int64_t B, int64_t C, bool al) {
     if (C != 1 || B > 16384) return MF_TWO_PASS;
+    // Short rows at an unaligned address: a wavefront a row leaves most lanes idle ([2^23, 1] 2405 us,
+    // two passes 91; [838860, 10] 252 and 79; [270600, 31] 88 and 81; rows of 32: 85 and 90).
     if (B <= 32 && al) return A < kMaxGridRows ? MF_TILES : MF_TWO_PASS;
+    if (B < 32) return MF_TWO_PASS;
     // a row per wavefront or block, as long as one dispatch holds them
     if (B <= 4096) return fits_dispatch((A + 3) / 4) ? MF_WAVE : MF_TWO_PASS;
     return fits_dispatch(A) ? MF_BLOCK : MF_TWO_PASS;

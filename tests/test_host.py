@@ -352,3 +352,12 @@ def test_channel_gradients_past_one_dispatch():
     for n, c, s in ((2, 1 << 25, 64), (2, 1 << 26, 64), (2, 1 << 26, 65), (64, 1 << 20, 64), (64, (1 << 20) + 1, 64)):
         info = plan_reduction(_lib.PLAN_CHANNELS, n, c, s)
         assert info.blocks * info.threads < (1 << 32), (n, c, s)
+
+
+def test_max_backward_of_short_unaligned_rows_takes_two_passes():
+    """Rows of fewer than 32 elements at an unaligned address: not a wavefront each."""
+    for b in (1, 2, 10, 31):
+        assert plan_reduction(_lib.PLAN_MAX_BACKWARD, 1 << 20, b, 1, 0).kernel == 3, b
+        assert plan_reduction(_lib.PLAN_MAX_BACKWARD, 1 << 20, b, 1, 1).kernel == 0, b
+    assert plan_reduction(_lib.PLAN_MAX_BACKWARD, 1 << 20, 32, 1, 0).kernel == 1
+    assert plan_reduction(_lib.PLAN_MAX_BACKWARD, 1 << 20, 33, 1, 1).kernel == 1
