@@ -1013,8 +1013,10 @@ __device__ __forceinline__ void load_row_quads(vf4 (&v)[NQ], const float* xr, in
 // row's threads, then grad[i] = grad[i] + (x[i] == m ? fl(1/c) * ug[row] : 0) from the same
 // registers (basics.mojo:581-615 for a last-axis reduce): x is read once. Rows of any length and
 // alignment (odd lengths took a max-count pass and a gathering pass: the SUM, MEAN and MAX passes
-// over [65536, 1001] together 650 us, 448 us now).
-template <int WPR, int NQ>
+// over [65536, 1001] together 650 us, 448 us now). Rows of whole quads have a variant of their own:
+// with the selects of the odd lengths [131072, 64] took 43.3 us and [83886, 100] 30.7; without, 35.9 and
+// 24.9.
+template <int WPR, int NQ, bool VEC>
 __global__ void __launch_bounds__(kRThreads)
     k_max_bwd_rowreg(float* __restrict__ grad, const float* __restrict__ x, const float* __restrict__ ug,
                      int64_t nrows, int64_t B) {
@@ -1035,14 +1037,27 @@ __global__ void __launch_bounds__(kRThreads)
     constexpr bool PRE = WPR == 1;
     const float nan = __builtin_nanf("");  // neither a maximum nor counted
     vf4 v[NQ], o[NQ];
-    load_row_quads<NQ, NT>(v, xr, tr, B, edge, nan);
-    if (PRE) load_row_quads<NQ, NT>(o, gr, tr, B, edge, 0.0f);
+    if constexpr (VEC) {  // both tensors' loads under one guard; quads past the row are passed over below
+#pragma unroll
+        for (int k = 0; k < NQ; ++k) {
+            const int64_t e = 4 * (tr + (int64_t)k * NT);
+            if (e < B) {
+                v[k] = ld_ntu(xr + e);
+                if (PRE) o[k] = ld_ntu(gr + e);
+            }
+        }
+    } else {
+        load_row_quads<NQ, NT>(v, xr, tr, B, edge, nan);
+        if (PRE) load_row_quads<NQ, NT>(o, gr, tr, B, edge, 0.0f);
+    }
     const float u = PRE ? ug[row] : 0.0f;
     MC acc = RMaxCnt::init();
 #pragma unroll
-    for (int k = 0; k < NQ; ++k)
+    for (int k = 0; k < NQ; ++k) {
+        if (VEC && 4 * (tr + (int64_t)k * NT) >= B) continue;
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc = RMaxCnt::comb(acc, RMaxCnt::lift(v[k][j]));
+    }
     acc = wave_reduce<RMaxCnt>(acc);
     if (WPR == 4) {
         if (lane == 0) ws[w] = acc;
@@ -1052,15 +1067,17 @@ __global__ void __launch_bounds__(kRThreads)
     const float f = 1.0f / (float)acc.c;  // basics.mojo:609
     const float g = f * (PRE ? u : ug[row]);
     const float m = acc.m;
-    if (!PRE) load_row_quads<NQ, NT>(o, gr, tr, B, edge, 0.0f);
+    if (!PRE && !VEC) load_row_quads<NQ, NT>(o, gr, tr, B, edge, 0.0f);
 #pragma unroll
     for (int k = 0; k < NQ; ++k) {
         const int64_t e = 4 * (tr + (int64_t)k * NT);
+        if (VEC && e >= B) continue;
+        if (VEC && !PRE) o[k] = ld_ntu(gr + e);
         vf4 n;
 #pragma unroll
         for (int j = 0; j < 4; ++j) n[j] = o[k][j] + (v[k][j] == m ? g : 0.0f);
         if (!bits_differ4(o[k].x, o[k].y, o[k].z, o[k].w, n.x, n.y, n.z, n.w)) continue;  // a sparse accumulation
-        if (e + 3 < B) {
+        if (VEC || e + 3 < B) {
             st_ntu(gr + e, n);
         } else {
 #pragma unroll
@@ -1281,7 +1298,7 @@ __device__ __forceinline__ float mom_std(const Mom& m, int64_t B) {
 // tstd over rows of B <= 16384 elements, of any length and alignment: WPR waves per row, the row's quads
 // loaded together, fp64 moments (above) summed per lane in quad order, then the butterfly and
 // the waves in order.
-template <int WPR, int NQ>
+template <int WPR, int NQ, bool VEC>
 __global__ void __launch_bounds__(kRThreads)
     k_tstd_rowreg(float* __restrict__ res, const float* __restrict__ x, int64_t nrows, int64_t B) {
     __shared__ Mom ws[4];
@@ -1294,15 +1311,26 @@ __global__ void __launch_bounds__(kRThreads)
     // the row's quads load before K is needed (an element past the row becomes K: x - K = 0 adds
     // nothing to either moment), so K's load is not waited for first
     vf4 v[NQ];
-    load_row_quads<NQ, NT>(v, xr, tr, B, row_edge(row, nrows, B), 0.0f);
+    if constexpr (VEC) {  // a quad past the row loads the last one: no branch around a load
+#pragma unroll
+        for (int k = 0; k < NQ; ++k) {
+            const int64_t e = 4 * (tr + (int64_t)k * NT);
+            v[k] = ld_ntu(xr + (e < B ? e : B - 4));
+        }
+    } else {
+        load_row_quads<NQ, NT>(v, xr, tr, B, row_edge(row, nrows, B), 0.0f);
+    }
     __builtin_amdgcn_sched_barrier(0);
     const float kf = xr[0];
     const double K = (double)kf;
     Mom m{0.0, 0.0};
 #pragma unroll
-    for (int k = 0; k < NQ; ++k)
+    for (int k = 0; k < NQ; ++k) {
+        const int64_t e = 4 * (tr + (int64_t)k * NT);
+        if (VEC && e >= B) v[k] = vf4{kf, kf, kf, kf};
 #pragma unroll
-        for (int j = 0; j < 4; ++j) mom_add(m, 4 * (tr + (int64_t)k * NT) + j < B ? v[k][j] : kf, K);
+        for (int j = 0; j < 4; ++j) mom_add(m, VEC || e + j < B ? v[k][j] : kf, K);
+    }
     m = mom_wave(m);
     if (WPR == 4) {
         if (lane == 0) ws[w] = m;
@@ -2538,7 +2566,11 @@ int mh_tstd(float* res, const float* x, const mh_shape* psx, int32_t axis) {
         if (Bq <= 64 * 16) {  // one wave per row, four rows per block
             const int nq = Bq <= 64 ? 1 : Bq <= 128 ? 2 : Bq <= 256 ? 4 : Bq <= 512 ? 8 : 16;
             dim3 g((unsigned)((A + 3) / 4)), b(kRThreads);
-#define MH_TSR(NQ) hipLaunchKernelGGL((k_tstd_rowreg<1, NQ>), g, b, 0, st, res, x, A, B)
+#define MH_TSR(NQ)                                                                            \
+    do {                                                                                     \
+        if (B % 4 == 0) hipLaunchKernelGGL((k_tstd_rowreg<1, NQ, true>), g, b, 0, st, res, x, A, B);  \
+        else hipLaunchKernelGGL((k_tstd_rowreg<1, NQ, false>), g, b, 0, st, res, x, A, B);            \
+    } while (0)
             switch (nq) {
                 case 1: MH_TSR(1); break;
                 case 2: MH_TSR(2); break;
@@ -2550,7 +2582,11 @@ int mh_tstd(float* res, const float* x, const mh_shape* psx, int32_t axis) {
         } else {  // one block per row
             const int nq = Bq <= 2048 ? 8 : 16;
             dim3 g((unsigned)A), b(kRThreads);
-#define MH_TSR(NQ) hipLaunchKernelGGL((k_tstd_rowreg<4, NQ>), g, b, 0, st, res, x, A, B)
+#define MH_TSR(NQ)                                                                            \
+    do {                                                                                     \
+        if (B % 4 == 0) hipLaunchKernelGGL((k_tstd_rowreg<4, NQ, true>), g, b, 0, st, res, x, A, B);  \
+        else hipLaunchKernelGGL((k_tstd_rowreg<4, NQ, false>), g, b, 0, st, res, x, A, B);            \
+    } while (0)
             if (nq == 8) MH_TSR(8);
             else MH_TSR(16);
 #undef MH_TSR
@@ -2682,7 +2718,11 @@ int mh_reduce_bwd_accum(int op, float* grad, const float* x, const mh_shape* psx
         if (mf == MF_WAVE) {  // four rows per block
             const int nq = Bq <= 64 ? 1 : Bq <= 128 ? 2 : Bq <= 256 ? 4 : Bq <= 512 ? 8 : 16;
             dim3 g((unsigned)((A + 3) / 4)), b(kRThreads);
-#define MH_MBR(NQ) hipLaunchKernelGGL((k_max_bwd_rowreg<1, NQ>), g, b, 0, st, grad, x, ug, A, B)
+#define MH_MBR(NQ)                                                                            \
+    do {                                                                                     \
+        if (B % 4 == 0) hipLaunchKernelGGL((k_max_bwd_rowreg<1, NQ, true>), g, b, 0, st, grad, x, ug, A, B);  \
+        else hipLaunchKernelGGL((k_max_bwd_rowreg<1, NQ, false>), g, b, 0, st, grad, x, ug, A, B);            \
+    } while (0)
             switch (nq) {
                 case 1: MH_MBR(1); break;
                 case 2: MH_MBR(2); break;
@@ -2694,7 +2734,11 @@ int mh_reduce_bwd_accum(int op, float* grad, const float* x, const mh_shape* psx
         } else {  // one block per row
             const int nq = Bq <= 512 ? 2 : Bq <= 1024 ? 4 : Bq <= 2048 ? 8 : 16;
             dim3 g((unsigned)A), b(kRThreads);
-#define MH_MBR(NQ) hipLaunchKernelGGL((k_max_bwd_rowreg<4, NQ>), g, b, 0, st, grad, x, ug, A, B)
+#define MH_MBR(NQ)                                                                            \
+    do {                                                                                     \
+        if (B % 4 == 0) hipLaunchKernelGGL((k_max_bwd_rowreg<4, NQ, true>), g, b, 0, st, grad, x, ug, A, B);  \
+        else hipLaunchKernelGGL((k_max_bwd_rowreg<4, NQ, false>), g, b, 0, st, grad, x, ug, A, B);            \
+    } while (0)
             switch (nq) {
                 case 2: MH_MBR(2); break;
                 case 4: MH_MBR(4); break;

@@ -68,6 +68,14 @@ def test_rows(gpu, b, off):
     reductions_match(gpu, (5, b), 1, off)
 
 
+@pytest.mark.parametrize("off", [0, 1, 3])
+@pytest.mark.parametrize("b", [4, 32, 36, 64, 256, 260, 1024, 2048, 4096, 4100, 8192, 16384])
+def test_rows_of_whole_quads(gpu, b, off):
+    """Last-axis lines of whole quads, at any address: the row kernels' variants without selects, and
+    short rows at an unaligned address in two passes."""
+    reductions_match(gpu, (5, b), 1, off)
+
+
 @pytest.mark.parametrize("n", [262145, 262146 + 4 * 2048, 1 << 20, (1 << 20) + 3])
 def test_every_element(gpu, n):
     """All elements as one row of chunks, whose last one is ragged."""
