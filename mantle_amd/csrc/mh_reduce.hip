@@ -590,8 +590,9 @@ __global__ void __launch_bounds__(kLdsRows)
 
 // One wavefront per row of B elements: the row's whole quads at lanes 0..63, 64..127, ... (at
 // any alignment), groups of four quads in flight, then its last B % 4 elements on the lane after
-// the last quad. Bound by memory. Rows of an odd length went one element per lane, 256 bytes an
-// instruction: [32768, 1023] SUM took 42 us that way, 22 us in quads.
+// the last quad. Bound by memory; short rows by their instructions: [66052, 127] SUM took 18.9 us
+// with three loads of the tail behind the quads and every group's partials combined, 13.3 us now
+// (16.5 us one element per lane, as odd rows once went).
 template <class R, class LD>
 __global__ void __launch_bounds__(kRThreads)
     k_rows_wave(LD ld, int64_t nrows, int64_t B, float* out, float* out2, int epi, float div) {
@@ -602,37 +603,74 @@ __global__ void __launch_bounds__(kRThreads)
     if (r >= nrows) return;  // uniform per wavefront; no block-level barrier follows
     const int64_t start = r * B;
     const int64_t nq = B >> 2;
-    T a4[4][4];
+    // the last B % 4 elements, from the quad that ends with the row, loaded with the quads and not
+    // behind them
+    const int rem = (int)(B & 3);
+    const bool last = rem != 0 && lane == (int)(nq & 63);
+    T tail[4];
+    if (last && nq >= 64) ld.get4(start + B - 4, tail);
+    auto add_tail = [&](T (&a)[4]) {
+        if (!last) return;
+        if (rem == 1) {
+            a[0] = R::comb(a[0], tail[3]);
+        } else if (rem == 2) {
+            a[0] = R::comb(a[0], tail[2]);
+            a[1] = R::comb(a[1], tail[3]);
+        } else {
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+            for (int j = 0; j < 3; ++j) a[j] = R::comb(a[j], tail[j + 1]);
+        }
+    };
+    T acc = R::init();
+    if (nq <= 192) {  // short rows: only the first group of quads holds any
+        T a[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) a4[u][j] = R::init();
-    int64_t q = lane;
-    for (; q + 192 < nq; q += 256) {
-        T v[4][4];
+        for (int j = 0; j < 4; ++j) a[j] = R::init();
+        if (nq < 64) {  // one load for the quads and the tail, on the lane after the last quad
+            if (4 * lane < B) ld.get4(start + (lane < nq ? 4 * lane : B - 4), tail);
+            if (lane < nq)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) ld.get4(start + (q + 64 * u) * 4, v[u]);
+                for (int j = 0; j < 4; ++j) a[j] = R::comb(a[j], tail[j]);
+        } else {
+            for (int64_t q = lane; q < nq; q += 64) {
+                T v[4];
+                ld.get4(start + q * 4, v);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) a[j] = R::comb(a[j], v[j]);
+            }
+        }
+        add_tail(a);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc = R::comb(acc, a[j]);
+        acc = R::comb(acc, R::init());  // the other groups' initial values, one standing for all
+    } else {
+        T a4[4][4];
 #pragma unroll
         for (int u = 0; u < 4; ++u)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) a4[u][j] = R::comb(a4[u][j], v[u][j]);
+            for (int j = 0; j < 4; ++j) a4[u][j] = R::init();
+        int64_t q = lane;
+        for (; q + 192 < nq; q += 256) {
+            T v[4][4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) ld.get4(start + (q + 64 * u) * 4, v[u]);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) a4[u][j] = R::comb(a4[u][j], v[u][j]);
+        }
+        for (; q < nq; q += 64) {
+            T v[4];
+            ld.get4(start + q * 4, v);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) a4[0][j] = R::comb(a4[0][j], v[j]);
+        }
+        add_tail(a4[0]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc = R::comb(acc, a4[u][j]);
     }
-    for (; q < nq; q += 64) {
-        T v[4];
-        ld.get4(start + q * 4, v);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) a4[0][j] = R::comb(a4[0][j], v[j]);
-    }
-    if (q == nq) {  // the lane after the last quad
-#pragma unroll
-        for (int j = 0; j < 3; ++j)
-            if (q * 4 + j < B) a4[0][j] = R::comb(a4[0][j], ld.get(start + q * 4 + j));
-    }
-    T acc = R::init();
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc = R::comb(acc, a4[u][j]);
     acc = wave_reduce<R>(acc);
     if (lane == 0) epi_store(out, out2, r, acc, epi, div);
 }

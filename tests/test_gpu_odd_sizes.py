@@ -76,6 +76,46 @@ def test_rows_of_whole_quads(gpu, b, off):
     reductions_match(gpu, (5, b), 1, off)
 
 
+@pytest.mark.parametrize("off", [0, 2])
+@pytest.mark.parametrize("b", [65, 66, 67, 68, 127, 250, 253, 255, 256, 257, 258, 259, 260, 511, 770, 771, 772, 773, 775,
+                               1022, 1025, 2045])
+def test_rows_by_wavefront(gpu, b, off):
+    """A row per wavefront at the edges of its quad counts (64, 192 and the groups of 256), with every
+    length modulo 4, in the order of its sums: quads lane, lane + 64, ... in groups of four, the last
+    elements after them, then a butterfly."""
+    def row_sum(x):
+        f, nq = np.float32, b // 4
+        a4 = np.zeros((64, 4, 4), f)
+        for lane in range(64):
+            q = lane
+            while q + 192 < nq:
+                for u in range(4):
+                    a4[lane, u] += x[4 * (q + 64 * u):4 * (q + 64 * u) + 4]
+                q += 256
+            while q < nq:
+                a4[lane, 0] += x[4 * q:4 * q + 4]
+                q += 64
+            if q == nq:
+                a4[lane, 0, :b % 4] += x[4 * nq:b]
+        v = np.zeros(64, f)
+        for g in a4.reshape(64, 16).T:
+            v = v + g
+        for k in (32, 16, 8, 4, 2, 1):
+            v = v + v[np.arange(64) ^ k]
+        return v[0]
+
+    x = synth.normal((6, b), 0, 1, 2115)
+    res = view(gpu, np.zeros((6, 1), np.float32), 0)
+    gpu.m.forward_op(SUM, res, view(gpu, x, off), attributes={"axis": 1})
+    assert_bitexact(res.to_numpy()[:, 0], np.array([row_sum(r) for r in x], np.float32), f"SUM over {b}")
+    x[1, ::3], x[2, -1], x[3] = np.nan, np.inf, -np.inf
+    gpu.m.forward_op(MAX, res, view(gpu, x, off), attributes={"axis": 1})
+    got = res.to_numpy()[:, 0]
+    for r in (0, 2, 4, 5):
+        assert got[r] == x[r].max(), r
+    assert got[3] == -np.finfo(np.float32).max  # MAX starts at -FLT_MAX
+
+
 @pytest.mark.parametrize("n", [262145, 262146 + 4 * 2048, 1 << 20, (1 << 20) + 3])
 def test_every_element(gpu, n):
     """All elements as one row of chunks, whose last one is ragged."""
