@@ -2133,8 +2133,18 @@ struct PlaneForm {
     int64_t N, C, S, Sq, QC, K, G, NG, nwaves;
 };
 
-// The plan [N*C, S, 1] then [1, N, C] with S of at least 64.
-static bool plane_form(const mh_reduce_plan_info& p, PlaneForm* f) {
+// The plan [N*C, S, 1] then [1, N, C] with S of at least 64, where one launch beats the chain (a row
+// reduction, then a column reduction; MUL and DIV write their terms out first), for sums of `kind`.
+// Two costs are weighed, in the terms of a sweep over 652 shapes of up to 2^27 elements, both
+// ways:
+//   tickets  a channel costs about 6.5 ns (its counter's line, the last arrival) and a wavefront
+//            0.5 ns (its ticket), which the stream hides only when there is enough of it: SUB over
+//            [2, 50000, 65] 384 us, chain 26; over [32, 1000, 100] 28 and 12; over [256, 96, 729] 14
+//            and 23, over [1000, 512, 65] 68 and 124;
+//   depth    a wavefront's planes are read two at a time, one after another: few channels leave the
+//            chip idle behind them (SUB over [3000, 2, 256] 21 us, chain 10; over [256, 2, 20000] 52
+//            and 15), DIV's divisions sooner than the rest (over [1000, 2, 729] 21 and 15).
+static bool plane_form(const mh_reduce_plan_info& p, int kind, PlaneForm* f) {
     if (p.nsteps != 2 || p.c[0] != 1 || p.a[1] != 1 || p.a[0] != p.b[1] * p.c[1]) return false;
     f->N = p.b[1];
     f->C = p.c[1];
@@ -2147,7 +2157,14 @@ static bool plane_form(const mh_reduce_plan_info& p, PlaneForm* f) {
     if (f->G < 1) f->G = 1;
     f->NG = (f->N + f->G - 1) / f->G;
     f->nwaves = f->NG * f->K * f->C;
-    return f->NG * f->K <= kPlanesMaxArrivals && fits_dispatch((f->nwaves + 3) / 4);
+    if (f->NG * f->K > kPlanesMaxArrivals || !fits_dispatch((f->nwaves + 3) / 4)) return false;
+    const bool two = kind >= PL_MUL;
+    const int64_t n = f->N * f->C * f->S, per_wave = n / f->nwaves;
+    const int64_t hidden = two ? 3 * n / 1000 : f->N >= 64 ? n / 500 : 0;
+    if (13 * f->C + f->nwaves > 8000 + hidden) return false;
+    const int64_t rounds = (f->G + 1) / 2 + f->G * ((f->QC + 255) / 256 - 1);  // memory round trips of a wave
+    if (rounds <= 16) return kind < PL_DIV0 || per_wave <= 9000 || f->nwaves >= 400;
+    return f->nwaves >= 1024 || (two && f->nwaves >= 500 && per_wave >= 12000);
 }
 
 // Launches k_unb_planes; tmp holds NG * K * C partials.
@@ -2173,7 +2190,7 @@ size_t unbroadcast_scratch_floats(const mh_shape& sgrad, const mh_shape& srg) {
     auto pad = [](size_t v) { return (v + 63) & ~(size_t)63; };
     size_t need = pad(tmax) + 2 * pad(bmax) + 64;
     PlaneForm pf;
-    if (plane_form(p, &pf)) {  // the one-launch plane form's partials
+    if (plane_form(p, PL_RG, &pf)) {  // the one-launch plane form's partials
         const size_t np = pad((size_t)(pf.NG * pf.K * pf.C)) + 64;
         if (np > need) need = np;
     }
@@ -2191,7 +2208,7 @@ int unbroadcast_accum_scratch(float* grad, const mh_shape& sgrad, const float* r
     if (p.nsteps == 0)  // only size-1 dims differ: same element order
         return reduce_abc(RED_SUM, final_epi, rg, numel(srg), 1, 1, grad, nullptr, 0.0f, nullptr);
     PlaneForm pf;
-    if (plane_form(p, &pf))  // a per-channel bias gradient: one launch
+    if (plane_form(p, negate ? PL_NEG : PL_RG, &pf))  // a per-channel bias gradient: one launch
         return negate ? launch_planes<PL_NEG>(pf, grad, rg, nullptr, nullptr, tmp)
                       : launch_planes<PL_RG>(pf, grad, rg, nullptr, nullptr, tmp);
     size_t tmax = 0, bmax = 0;
@@ -2329,7 +2346,8 @@ int unbroadcast_binrg(int op, int id, bool divs, float* grad, const mh_shape& sg
     mh_reduce_plan_info p;
     MH_TRY(plan_unbroadcast(sgrad, sug, &p));
     PlaneForm pf;
-    if (!divs && plane_form(p, &pf)) {  // a per-channel operand: one launch
+    const int kind = op == MH_MUL ? PL_MUL : id == 0 ? PL_DIV0 : PL_DIV1;
+    if (!divs && plane_form(p, kind, &pf)) {  // a per-channel operand: one launch
         float* part = nullptr;
         MH_TRY(scratch(((size_t)(pf.NG * pf.K * pf.C) + 64) * sizeof(float), reinterpret_cast<void**>(&part)));
         if (op == MH_MUL) MH_TRY(launch_planes<PL_MUL>(pf, grad, ug, a, nullptr, part));
@@ -2804,7 +2822,7 @@ int mh_reduce_bwd_accum(int op, float* grad, const float* x, const mh_shape* psx
     return finish("mh_reduce_bwd_accum");
 }
 
-int mh_plan_reduction(int32_t what, int64_t A, int64_t B, int64_t C, int32_t aligned, mh_launch_info* out) {
+int mh_plan_reduction(int32_t what, int64_t A, int64_t B, int64_t C, int32_t variant, mh_launch_info* out) {
     if (!out) return fail(MH_ERR_NULL, "mh_plan_reduction: null");
     if (A < 1 || B < 1 || C < 1) return fail(MH_ERR_INVALID, "mh_plan_reduction: empty shape");
     out->threads = kRThreads;
@@ -2818,7 +2836,7 @@ int mh_plan_reduction(int32_t what, int64_t A, int64_t B, int64_t C, int32_t ali
             return MH_OK;
         }
         case MH_PLAN_MAX_BACKWARD: {
-            const MaxForm f = max_bwd_form(A, B, C, aligned != 0);
+            const MaxForm f = max_bwd_form(A, B, C, variant != 0);
             out->kernel = f;
             out->threads = f == MF_TILES ? kLdsRows : kRThreads;
             out->blocks = f == MF_TILES ? (A + kLdsRows - 1) / kLdsRows : f == MF_WAVE ? (A + 3) / 4 : f == MF_BLOCK ? A : 0;
@@ -2831,7 +2849,7 @@ int mh_plan_reduction(int32_t what, int64_t A, int64_t B, int64_t C, int32_t ali
             p.a[0] = A * B; p.b[0] = C; p.c[0] = 1;
             p.a[1] = 1; p.b[1] = A; p.c[1] = B;
             PlaneForm f;
-            const bool one = plane_form(p, &f);
+            const bool one = plane_form(p, variant == 0 ? PL_RG : variant == 1 ? PL_MUL : PL_DIV1, &f);
             out->kernel = one ? 1 : 0;
             out->blocks = one ? (f.nwaves + 3) / 4 : 0;
             out->launches = one ? 1 : 0;

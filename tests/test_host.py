@@ -319,9 +319,9 @@ def test_row_engine_launches_split_rows_past_one_dispatch():
     assert L.mh_plan_launch(0, -1, ctypes.byref(info)) == _lib.ERR_INVALID
 
 
-def plan_reduction(what, a, b, c, aligned=1):
+def plan_reduction(what, a, b, c, variant=1):
     info = _lib.mh_launch_info()
-    assert _lib.lib().mh_plan_reduction(what, a, b, c, aligned, ctypes.byref(info)) == 0, _lib.last_error()
+    assert _lib.lib().mh_plan_reduction(what, a, b, c, variant, ctypes.byref(info)) == 0, _lib.last_error()
     return info
 
 
@@ -361,3 +361,14 @@ def test_max_backward_of_short_unaligned_rows_takes_two_passes():
         assert plan_reduction(_lib.PLAN_MAX_BACKWARD, 1 << 20, b, 1, 1).kernel == 0, b
     assert plan_reduction(_lib.PLAN_MAX_BACKWARD, 1 << 20, 32, 1, 0).kernel == 1
     assert plan_reduction(_lib.PLAN_MAX_BACKWARD, 1 << 20, 33, 1, 1).kernel == 1
+
+
+@pytest.mark.parametrize("n,c,s,sums", [
+    (2, 50000, 65, "   "), (2, 50000, 64, "   "), (8, 20000, 100, "   "), (32, 1000, 100, "   "), (3000, 2, 256, "   "),
+    (256, 2, 20000, "   "), (1000, 2, 729, "+* "), (256, 96, 729, "+*/"), (256, 64, 784, "+*/"), (4, 32, 65, "+*/"),
+    (1000, 512, 65, "+*/"), (8, 1000, 2000, " */")])
+def test_channel_gradients_in_one_launch_where_it_pays(n, c, s, sums):
+    """A per-channel gradient takes the one-launch plane kernel where neither the channels' counters nor
+    the depth of a wavefront's planes outlast the stream."""
+    got = "".join(ch if plan_reduction(_lib.PLAN_CHANNELS, n, c, s, v).kernel else " " for v, ch in enumerate("+*/"))
+    assert got == sums
