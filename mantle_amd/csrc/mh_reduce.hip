@@ -9,11 +9,10 @@
 //                     butterfly shuffle;
 //   C == 1, B >= 2048: 2048-element chunks, one 4-wave block each (two quads per thread),
 //                     whose partials reduce again along the row the same way;
-//   C  >= 1024      : one thread per column quad over a split of the rows (about four blocks
-//                     per CU; splits on grid x);
-//   C  >= 128       : a block per (strip of 64 column quads, split of rows), its four waves
-//                     interleaving the rows, combined through LDS;
-//   C  > 1 otherwise: one thread per column quad (below 4 columns: per column);
+//   C  > 1          : one thread per column quad over a split of the rows (wide: splits on grid x;
+//                     quads), a block per (strip of 64 column quads, split of rows) whose four
+//                     waves interleave the rows and combine through LDS, or one thread per column;
+//                     which one by width, rows and what fills the chip (col_plan);
 //   in every column form the rows split across blocks when that is needed to fill the chip,
 //   and one short launch combines the split partials in fixed order (k_parts_comb). Column
 //   quads are at any alignment; the last quad of a slab whose C is not a multiple of 4 starts
@@ -711,7 +710,10 @@ __device__ __forceinline__ void col_quad(int64_t cq, int64_t C, int64_t* c, int*
 // Column reduction: item = a column quad (VEC, C >= 4) or one column of slab a of the [A, C]
 // output; the rows [b0, b1) of one split. S == 1 writes the epilogue, S > 1 writes partials at
 // s * (A * C) + o.
-template <class R, class LD, bool VEC, bool SPLIT_X = false>
+// RU rows are in flight. Launches that fill the chip stream best with two quads a thread; where the
+// splits leave it half idle the rows one after another are the time, and eight go out together, the
+// last ones too ([1, 30, 4099] SUM: 10.3 us two rows at a time, 6.0 eight; single columns 4.3).
+template <class R, class LD, bool VEC, bool SPLIT_X, int RU>
 __global__ void __launch_bounds__(kRThreads)
     k_cols(LD ld, int64_t A, int64_t B, int64_t C, int64_t rps, int64_t S, float* out, float* out2,
            int epi, float div, float* part) {
@@ -733,26 +735,19 @@ __global__ void __launch_bounds__(kRThreads)
     T acc[W];
 #pragma unroll
     for (int j = 0; j < W; ++j) acc[j] = R::init();
-    int64_t b = b0;
-    constexpr int RU = VEC ? 2 : 4;  // rows in flight
-    for (; b + RU - 1 < b1; b += RU) {
+    for (int64_t b = b0; b < b1; b += RU) {
         T v[RU][W];
 #pragma unroll
-        for (int u = 0; u < RU; ++u) {
-            if (VEC) ld.get4(base + (b + u) * C, v[u]);
-            else v[u][0] = ld.get(base + (b + u) * C);
-        }
+        for (int u = 0; u < RU; ++u)
+            if (b + u < b1) {
+                if (VEC) ld.get4(base + (b + u) * C, v[u]);
+                else v[u][0] = ld.get(base + (b + u) * C);
+            }
 #pragma unroll
         for (int u = 0; u < RU; ++u)
+            if (b + u < b1)
 #pragma unroll
-            for (int j = 0; j < W; ++j) acc[j] = R::comb(acc[j], v[u][j]);
-    }
-    for (; b < b1; ++b) {
-        T v[W];
-        if (VEC) ld.get4(base + b * C, v);
-        else v[0] = ld.get(base + b * C);
-#pragma unroll
-        for (int j = 0; j < W; ++j) acc[j] = R::comb(acc[j], v[j]);
+                for (int j = 0; j < W; ++j) acc[j] = R::comb(acc[j], v[u][j]);
     }
 #pragma unroll
     for (int j = 0; j < W; ++j) {
@@ -1634,9 +1629,9 @@ struct ColSplit {
     int64_t S, rps;
     bool vec;
 };
-static ColSplit col_split(int64_t A, int64_t B, int64_t C) {
+static ColSplit col_split(int64_t A, int64_t B, int64_t C, bool vec) {
     ColSplit cs;
-    cs.vec = C >= 4;
+    cs.vec = vec;
     const int64_t items = A * (cs.vec ? (C + 3) / 4 : C);
     const int64_t bx = (items + kRThreads - 1) / kRThreads;
     const int64_t target = 8 * (int64_t)ctx().num_cus;  // blocks wanted
@@ -1734,31 +1729,42 @@ static inline bool fits_dispatch(int64_t blocks, int64_t threads = kRThreads) {
 }
 
 // The form of a strided reduction over [A, B, C] (C > 1) and its launch: gx x gy blocks, S splits
-// of rps rows.
+// of rps rows. By a sweep of every form over 690 shapes of 4 K to 32 M elements, in SUM and MAX:
+//   wide     where three blocks a CU come together, the streaming form; narrower or shorter than
+//            that it leaves the chip idle behind two rows in flight ([8, 100, 1025]: 14.3 us, strips 7.9)
+//   strips   other widths of 128 and more, but not a few rows of many slabs, where three of a block's
+//            wavefronts have nothing to do ([50000, 2, 129]: 40.2 us, quads 18.2)
+//   quads    where they leave at least two blocks a CU; a few columns of an odd width cost two quads
+//            for little more than one ([700, 1000, 9]: 18.6 us, singles 15.3)
+//   singles  the rest ([64, 30, 9]: 6.8 us in quads, 4.9)
 enum ColForm : int { CF_WIDE = 0, CF_STRIP = 1, CF_QUADS = 2, CF_SINGLES = 3 };
 struct ColPlan {
     ColForm form;
     int64_t S, rps, gx, gy, nstrips;
 };
 static ColPlan col_plan(int64_t A, int64_t B, int64_t C) {
+    const int64_t cus = ctx().num_cus;
     const int64_t quads = A * ((C + 3) / 4), qb = (quads + kRThreads - 1) / kRThreads;
     ColPlan p{};
     ColSplit cs;
-    // the wide layout puts the column-quad blocks on grid y (at most 65535 blocks there)
-    if (use_wide_cols(C) && qb <= 65535) {
-        cs = wide_split(A, B, C);
+    const bool wide = use_wide_cols(C) && qb <= 65535;  // its column-quad blocks lie on grid y
+    if (wide && (cs = wide_split(A, B, C), qb * cs.S >= 3 * cus)) {
         p.form = CF_WIDE;
         p.gx = cs.S;
         p.gy = qb;
-    } else if (use_strip(C) && fits_dispatch(A * (((C + 3) / 4 + 63) / 64))) {
+    } else if (use_strip(C) && (B >= 16 || qb < cus) && fits_dispatch(A * (((C + 3) / 4 + 63) / 64))) {
         cs = strip_split(A, B, C, &p.nstrips);
         p.form = CF_STRIP;
         p.gx = A * p.nstrips;
         p.gy = cs.S;
     } else {
-        cs = col_split(A, B, C);
-        p.form = cs.vec ? CF_QUADS : CF_SINGLES;
-        p.gx = cs.vec ? qb : (A * C + kRThreads - 1) / kRThreads;
+        cs = col_split(A, B, C, C >= 4);
+        const int64_t sb = (A * C + kRThreads - 1) / kRThreads;
+        const bool quads_pay = use_strip(C) || (qb * cs.S >= 2 * cus && quads >= 32 && (C % 4 == 0 || C >= 20));
+        const bool vec = C >= 4 && (quads_pay || !fits_dispatch(sb));
+        if (!vec) cs = col_split(A, B, C, false);
+        p.form = vec ? CF_QUADS : CF_SINGLES;
+        p.gx = vec ? qb : sb;
         p.gy = cs.S;
     }
     p.S = cs.S;
@@ -1772,7 +1778,9 @@ static size_t tmp_floats_t(int64_t A, int64_t B, int64_t C) {
     if (A * C == 0) return 0;
     if (C == 1) return row_tmp_floats<R>(A, B);
     // the largest split any form may pick
-    int64_t S = col_split(A, B, C).S;
+    int64_t S = col_split(A, B, C, C >= 4).S;
+    const int64_t s1 = col_split(A, B, C, false).S;
+    S = s1 > S ? s1 : S;
     if (use_wide_cols(C)) {
         const int64_t sw = wide_split(A, B, C).S;
         S = sw > S ? sw : S;
@@ -1904,19 +1912,23 @@ static int reduce_t(LD ld, bool vec_ok, int epi, int64_t A, int64_t B, int64_t C
     }
     const ColPlan cs = col_plan(A, B, C);
     const dim3 g((unsigned)cs.gx, (unsigned)cs.gy), b(kRThreads);
+    constexpr int RU = sizeof(typename R::T) == 4 ? 8 : 4;  // quads of a max and its count: registers
     switch (cs.form) {
         case CF_WIDE:
-            hipLaunchKernelGGL((k_cols<R, LD, true, true>), g, b, 0, st, ld, A, B, C, cs.rps, cs.S, out, out2, epi, div, tmp);
+            hipLaunchKernelGGL((k_cols<R, LD, true, true, 2>), g, b, 0, st, ld, A, B, C, cs.rps, cs.S, out, out2, epi, div,
+                               tmp);
             break;
         case CF_STRIP:
             hipLaunchKernelGGL((k_cols_strip<R, LD>), g, b, 0, st, ld, A, B, C, cs.nstrips, cs.rps, cs.S, out, out2, epi,
                                div, tmp);
             break;
         case CF_QUADS:
-            hipLaunchKernelGGL((k_cols<R, LD, true>), g, b, 0, st, ld, A, B, C, cs.rps, cs.S, out, out2, epi, div, tmp);
+            hipLaunchKernelGGL((k_cols<R, LD, true, false, RU>), g, b, 0, st, ld, A, B, C, cs.rps, cs.S, out, out2, epi,
+                               div, tmp);
             break;
         default:
-            hipLaunchKernelGGL((k_cols<R, LD, false>), g, b, 0, st, ld, A, B, C, cs.rps, cs.S, out, out2, epi, div, tmp);
+            hipLaunchKernelGGL((k_cols<R, LD, false, false, 8>), g, b, 0, st, ld, A, B, C, cs.rps, cs.S, out, out2, epi,
+                               div, tmp);
             break;
     }
     if (cs.S > 1) {

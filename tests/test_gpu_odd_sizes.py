@@ -159,6 +159,15 @@ def test_columns(gpu, shape, off):
     reductions_match(gpu, shape, 1, off)
 
 
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("shape", [(1, 7, 4), (3, 8, 5), (2, 9, 19), (1, 15, 20), (4, 17, 1030), (2, 31, 1028), (2100, 3, 129),
+                                   (2100, 9, 132), (2500, 17, 33), (2500, 40, 36), (1, 1100, 9), (40, 33, 2)], ids=str)
+def test_columns_in_every_form(gpu, shape, off):
+    """Strided axes at the edges of the forms' rules, with rows left over from the eight (four, two) in
+    flight."""
+    reductions_match(gpu, shape, 1, off)
+
+
 @pytest.mark.parametrize("op", ["SUB", "MUL", "DIV"])
 @pytest.mark.parametrize("shape,bshape", [((300, 1001), (1, 1001)), ((70, 5), (1, 5)), ((129, 2), (1, 2)),
                                           ((4099, 130), (130,)), ((3, 200, 67), (3, 1, 67)), ((1000, 3), (3,))],

@@ -372,3 +372,31 @@ def test_channel_gradients_in_one_launch_where_it_pays(n, c, s, sums):
     the depth of a wavefront's planes outlast the stream."""
     got = "".join(ch if plan_reduction(_lib.PLAN_CHANNELS, n, c, s, v).kernel else " " for v, ch in enumerate("+*/"))
     assert got == sums
+
+
+@pytest.mark.parametrize("a,b,c,form", [
+    (1, 8192, 8192, 0), (2, 6132, 6965, 0), (1, 100, 300000, 0), (8, 100, 1025, 1), (1, 30, 4099, 1), (33, 1025, 1023, 1),
+    (1, 16384, 1000, 1), (50000, 2, 129, 2), (5000, 4, 300, 2), (5000, 100, 33, 2), (700, 1000, 9, 3), (64, 30, 9, 3),
+    (1, 100, 100, 3), (1, 1 << 21, 3, 3), (1 << 20, 4, 64, 2)])
+def test_strided_reduction_forms(a, b, c, form):
+    """The form of a reduction over the middle axis of [a, b, c]: wide 0, strips 1, quads 2, singles 3."""
+    assert plan_reduction(_lib.PLAN_COLUMNS, a, b, c).kernel == form
+
+
+def test_strided_reduction_partials_fit_the_fixed_scratch():
+    """A reduction over a non-last axis that splits its rows leaves at most 16 MiB of partials, which the
+    no-allocation entry point states: blocks x columns of the split forms over a wide range of shapes."""
+    rng = np.random.default_rng(5)
+    for _ in range(20000):
+        a, b, c = (int(np.exp(rng.uniform(0, np.log(hi)))) for hi in (1e6, 1e6, 1e6))
+        if c < 2 or a * b * c > 1 << 33:
+            continue
+        s1 = lambda items, per, target: min(-(-target // max(1, -(-items // 256))), max(1, b // per), 65535)  # noqa: E731
+        q = a * -(-c // 4)
+        splits = [s1(a * c, 16, 2048) if a * c < 2048 * 256 else 1, s1(q, 16, 2048) if c >= 4 and q < 2048 * 256 else 1]
+        if c >= 1024:
+            splits.append(s1(q, 32, 1024))
+        if c >= 128 and a * -(-c // 256) < 2048:
+            splits.append(min(-(-2048 // (a * -(-c // 256))), max(1, b // 32)))
+        if max(splits) > 1:
+            assert max(splits) * a * c * 4 <= 16 << 20, (a, b, c, splits)
