@@ -711,8 +711,9 @@ __device__ __forceinline__ void col_quad(int64_t cq, int64_t C, int64_t* c, int*
 // output; the rows [b0, b1) of one split. S == 1 writes the epilogue, S > 1 writes partials at
 // s * (A * C) + o.
 // RU rows are in flight. Launches that fill the chip stream best with two quads a thread; where the
-// splits leave it half idle the rows one after another are the time, and eight go out together, the
-// last ones too ([1, 30, 4099] SUM: 10.3 us two rows at a time, 6.0 eight; single columns 4.3).
+// splits leave it half idle the rows one after another are the time, and eight go out together, then
+// the rest by fours, twos and one ([1, 30, 4099] SUM: 10.3 us two rows at a time, 6.0 eight; the MUL
+// gradient of [1, 1, 32] over [1, 2^22, 32] 574 and 203).
 template <class R, class LD, bool VEC, bool SPLIT_X, int RU>
 __global__ void __launch_bounds__(kRThreads)
     k_cols(LD ld, int64_t A, int64_t B, int64_t C, int64_t rps, int64_t S, float* out, float* out2,
@@ -735,20 +736,26 @@ __global__ void __launch_bounds__(kRThreads)
     T acc[W];
 #pragma unroll
     for (int j = 0; j < W; ++j) acc[j] = R::init();
-    for (int64_t b = b0; b < b1; b += RU) {
-        T v[RU][W];
+    int64_t b = b0;
+    // N rows: no branch between their loads, whose loader may compute on what it loads
+    auto rows = [&](auto n) {
+        constexpr int N = decltype(n)::value;
+        T v[N][W];
 #pragma unroll
-        for (int u = 0; u < RU; ++u)
-            if (b + u < b1) {
-                if (VEC) ld.get4(base + (b + u) * C, v[u]);
-                else v[u][0] = ld.get(base + (b + u) * C);
-            }
+        for (int u = 0; u < N; ++u) {
+            if (VEC) ld.get4(base + (b + u) * C, v[u]);
+            else v[u][0] = ld.get(base + (b + u) * C);
+        }
 #pragma unroll
-        for (int u = 0; u < RU; ++u)
-            if (b + u < b1)
+        for (int u = 0; u < N; ++u)
 #pragma unroll
-                for (int j = 0; j < W; ++j) acc[j] = R::comb(acc[j], v[u][j]);
-    }
+            for (int j = 0; j < W; ++j) acc[j] = R::comb(acc[j], v[u][j]);
+        b += N;
+    };
+    while (b + RU <= b1) rows(std::integral_constant<int, RU>{});
+    if (RU > 4 && b + 4 <= b1) rows(std::integral_constant<int, 4>{});
+    if (RU > 2 && b + 2 <= b1) rows(std::integral_constant<int, 2>{});
+    if (b < b1) rows(std::integral_constant<int, 1>{});
 #pragma unroll
     for (int j = 0; j < W; ++j) {
         if (VEC && j < lo) continue;
