@@ -470,8 +470,9 @@ int mh_plan_launch(int32_t what, int64_t n, mh_launch_info* out);
  *                         workgroup per row, 3 a max-count reduction and a routing pass; variant 1:
  *                         x and grad are 16-byte aligned
  *   MH_PLAN_CHANNELS      the gradient of a [1, B, 1] operand over [A, B, C] (variant 0: of ADD or
- *                         SUB, 1: MUL, 2: DIV): 1 one launch over the planes, 0 a chain */
-enum { MH_PLAN_COLUMNS = 0, MH_PLAN_MAX_BACKWARD = 1, MH_PLAN_CHANNELS = 2 };
+ *                         SUB, 1: MUL, 2: DIV): 1 one launch over the planes, 0 a chain
+ *   MH_PLAN_TSTD          tstd over B with C > 1: 2 column quads, 3 single columns */
+enum { MH_PLAN_COLUMNS = 0, MH_PLAN_MAX_BACKWARD = 1, MH_PLAN_CHANNELS = 2, MH_PLAN_TSTD = 3 };
 int mh_plan_reduction(int32_t what, int64_t A, int64_t B, int64_t C, int32_t variant, mh_launch_info* out);
 
 #ifdef __cplusplus

@@ -48,7 +48,7 @@ class mh_launch_info(ctypes.Structure):
 
 (LAUNCH_FILL, LAUNCH_FILL_UNALIGNED, LAUNCH_COPY, LAUNCH_SAME_SHAPE, LAUNCH_ADAM, LAUNCH_ADAM_UNALIGNED,
  LAUNCH_ROWS16) = range(7)
-PLAN_COLUMNS, PLAN_MAX_BACKWARD, PLAN_CHANNELS = range(3)
+PLAN_COLUMNS, PLAN_MAX_BACKWARD, PLAN_CHANNELS, PLAN_TSTD = range(4)
 
 
 class mh_attrs(ctypes.Structure):

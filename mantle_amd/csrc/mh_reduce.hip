@@ -1533,9 +1533,7 @@ __global__ void __launch_bounds__(kRThreads)
 #pragma unroll
         for (int j = 0; j < W; ++j) mom_add(m[0][j], v[j], K[j]);
     }
-#pragma unroll
-    for (int j = 0; j < W; ++j) {
-        if (VEC && j < lo) continue;
+    auto put = [&](int j) {
         Mom t = m[0][j];
 #pragma unroll
         for (int h = 1; h < CH; ++h) {
@@ -1544,6 +1542,14 @@ __global__ void __launch_bounds__(kRThreads)
         }
         if (S == 1) res[o + j] = mom_std(t, B);
         else part[s * AC + o + j] = t;
+    };
+    if (!VEC || lo == 0) {  // together: one store
+#pragma unroll
+        for (int j = 0; j < W; ++j) put(j);
+    } else {
+#pragma unroll
+        for (int j = 1; j < W; ++j)
+            if (j >= lo) put(j);
     }
 }
 
@@ -2539,6 +2545,44 @@ int map_max_route(float* grad, const mh_shape& sx, const float* x, const mh_shap
 int map_scale_bcast(float* grad, const mh_shape& sx, const float* ug, const mh_shape& sug, float c, bool twice);
 int map_mean_all(float* grad, int64_t n, const float* ug, float c);
 
+// tstd over a strided axis: a thread per column quad (vec) or per column, eight rows in flight over four
+// accumulator chains, at most one block per CU with the rows split. Fewer, longer splits write and
+// combine fewer fp64 partials: at [8192, 8192] axis 0 (a probe, moments + combine) 32 splits took 48.1
+// us against 52.6 us with 64 splits of four rows in flight, one chain; 128 and 256 splits took 57-60
+// us. In the bench (moments + combine, streamed) the splits on grid x took 47.2 us against 48.9 us on y;
+// 16 rows in flight 49.4 us, two blocks per CU 59.4 us. A split has at least 16 rows of 256 and more,
+// else 64: the combine of shorter ones costs more than it saves ([64, 64, 2000]: 18.8 us with 16, 9.0),
+// and blocks past the last CU wait for the first ([64, 300, 1000] in 315 blocks 24.7 us, 252: 20.1).
+// Quads do four columns' fp64 adds in a row, so they need the chip full and rows enough to pay
+// ([1, 30, 4099]: 6.8 us, single columns 3.7; [5000, 100, 9] 17.5 and 12.8; but [8, 10000, 200] 18.5 and
+// 30.6), or so many outputs that their stores are the time. With S > 1 there are no more column blocks than CUs, well inside grid y's limit.
+struct TstdPlan {
+    int64_t S, rps, bx;
+    bool vec;
+};
+static TstdPlan tstd_plan(int64_t A, int64_t B, int64_t C) {
+    const int64_t cus = ctx().num_cus;
+    auto plan = [&](bool vec) {
+        TstdPlan p;
+        p.vec = vec;
+        p.bx = (A * (vec ? (C + 3) / 4 : C) + kRThreads - 1) / kRThreads;
+        int64_t S = cus / p.bx;
+        const int64_t maxS = B / (B >= 256 ? 16 : 64);
+        if (S > maxS) S = maxS;
+        if (S < 1) S = 1;
+        p.rps = (B + S - 1) / S;
+        p.S = (B + p.rps - 1) / p.rps;
+        return p;
+    };
+    if (C < 4) return plan(false);
+    const TstdPlan q = plan(true);
+    const int64_t blocks = q.bx * q.S;
+    const bool full = blocks >= cus * 3 / 4 && !(q.bx > cus && q.bx < cus * 3 / 2);
+    const bool vec = full && A * ((C + 3) / 4) >= 16 &&
+                     (B >= 512 || (B >= 24 && C >= 36) || (B < 8 && A * B * C >= ((int64_t)1 << 26)));
+    return vec || !fits_dispatch((A * C + kRThreads - 1) / kRThreads) ? q : plan(false);
+}
+
 // The form of a MAX backward over [A, B, C] (B >= 1): rows staged as tiles, rows held in registers by
 // a wavefront or a block each, or a max-count reduction and a routing pass.
 enum MaxForm : int { MF_TILES = 0, MF_WAVE = 1, MF_BLOCK = 2, MF_TWO_PASS = 3 };
@@ -2683,27 +2727,9 @@ int mh_tstd(float* res, const float* x, const mh_shape* psx, int32_t axis) {
             hipLaunchKernelGGL(k_tstd_mom_combine_rows, dim3((unsigned)A), dim3(kMomCombThreads), 0, st, res, part, S, B);
         return finish("mh_tstd");
     }
-    // strided axis: a thread per column quad, about one block per CU, row splits of at least 16
-    // rows, eight rows in flight over four accumulator chains. Fewer, longer splits write and
-    // combine fewer fp64 partials: at [8192, 8192] axis 0 (a probe, moments + combine) 32 splits
-    // took 48.1 us against 52.6 us with 64 splits of four rows in flight, one chain; 128 and
-    // 256 splits took 57-60 us. In the bench (moments + combine, streamed) the splits on grid x
-    // took 47.2 us against 48.9 us on y; 16 rows in flight 49.4 us, two blocks per CU 59.4 us.
-    // With S > 1 there are fewer column blocks than CUs, well inside grid y's limit.
-    // Single columns where they fill the chip without a split and quads would not ([172, 147, 625]:
-    // 18.9 us against 17.6 + 7.1 us with the combine of three splits).
-    const int64_t chip = (int64_t)ctx().num_cus * kRThreads;
-    const bool vec = C >= 4 && !(A * C >= chip && A * ((C + 3) / 4) < chip && B < 512);
-    const int64_t items = A * (vec ? (C + 3) / 4 : C);
-    const int64_t bx = (items + kRThreads - 1) / kRThreads;
-    int64_t S = ((int64_t)ctx().num_cus + bx - 1) / bx;
-    int64_t maxS = B / 16;
-    if (maxS < 1) maxS = 1;
-    if (S > maxS) S = maxS;
-    if (S > 65535) S = 65535;
-    if (S < 1) S = 1;
-    const int64_t rps = (B + S - 1) / S;
-    S = (B + rps - 1) / rps;
+    const TstdPlan tp = tstd_plan(A, B, C);
+    const int64_t S = tp.S, rps = tp.rps, bx = tp.bx;
+    const bool vec = tp.vec;
     Mom* part = nullptr;
     if (S > 1) MH_TRY(scratch((size_t)(S * A * C) * sizeof(Mom), reinterpret_cast<void**>(&part)));
     const dim3 b(kRThreads);
@@ -2860,6 +2886,14 @@ int mh_plan_reduction(int32_t what, int64_t A, int64_t B, int64_t C, int32_t var
             out->threads = f == MF_TILES ? kLdsRows : kRThreads;
             out->blocks = f == MF_TILES ? (A + kLdsRows - 1) / kLdsRows : f == MF_WAVE ? (A + 3) / 4 : f == MF_BLOCK ? A : 0;
             out->launches = f == MF_TWO_PASS ? 0 : 1;
+            return MH_OK;
+        }
+        case MH_PLAN_TSTD: {
+            if (C == 1) return fail(MH_ERR_INVALID, "mh_plan_reduction: columns need C > 1");
+            const TstdPlan p = tstd_plan(A, B, C);
+            out->kernel = p.vec ? 2 : 3;
+            out->blocks = p.S > 1 ? p.S : p.bx;
+            out->launches = p.S > 1 ? 2 : 1;
             return MH_OK;
         }
         case MH_PLAN_CHANNELS: {

@@ -400,3 +400,14 @@ def test_strided_reduction_partials_fit_the_fixed_scratch():
             splits.append(min(-(-2048 // (a * -(-c // 256))), max(1, b // 32)))
         if max(splits) > 1:
             assert max(splits) * a * c * 4 <= 16 << 20, (a, b, c, splits)
+
+
+@pytest.mark.parametrize("a,b,c,form,launches", [
+    (1, 8192, 8192, 2, 2), (2, 6460, 759, 2, 2), (1, 30, 4099, 3, 1), (64, 64, 2000, 3, 1), (64, 30, 41, 3, 1), (8, 64, 70, 3, 1),
+    (64, 300, 1000, 2, 2), (172, 147, 625, 2, 2), (1, 1300000, 100, 2, 2), (1, 1 << 21, 3, 3, 2), (1 << 20, 4, 32, 2, 1)])
+def test_strided_tstd_forms(a, b, c, form, launches):
+    """tstd over the middle axis of [a, b, c]: column quads (2) only where they fill the chip, a combine
+    only where the splits are long."""
+    info = plan_reduction(_lib.PLAN_TSTD, a, b, c)
+    assert (info.kernel, info.launches) == (form, launches)
+    assert info.blocks * info.threads < (1 << 32)
