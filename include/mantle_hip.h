@@ -467,8 +467,8 @@ int mh_plan_launch(int32_t what, int64_t n, mh_launch_info* out);
  *   MH_PLAN_COLUMNS       SUM / MEAN / MAX over B with C > 1: 0 wide, 1 strips, 2 column quads,
  *                         3 single columns
  *   MH_PLAN_MAX_BACKWARD  MAX backward over B: 0 tiles of short rows, 1 a wavefront per row, 2 a
- *                         workgroup per row, 3 a max-count reduction and a routing pass; variant 1:
- *                         x and grad are 16-byte aligned
+ *                         workgroup per row, 3 a max-count reduction and a routing pass, 4 the same
+ *                         routed by the splits' indices; variant 1: x and grad are 16-byte aligned
  *   MH_PLAN_CHANNELS      the gradient of a [1, B, 1] operand over [A, B, C] (variant 0: of ADD or
  *                         SUB, 1: MUL, 2: DIV): 1 one launch over the planes, 0 a chain
  *   MH_PLAN_TSTD          tstd over B with C > 1: 2 column quads, 3 single columns */

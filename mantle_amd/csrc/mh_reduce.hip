@@ -2584,10 +2584,18 @@ static TstdPlan tstd_plan(int64_t A, int64_t B, int64_t C) {
 }
 
 // The form of a MAX backward over [A, B, C] (B >= 1): rows staged as tiles, rows held in registers by
-// a wavefront or a block each, or a max-count reduction and a routing pass.
-enum MaxForm : int { MF_TILES = 0, MF_WAVE = 1, MF_BLOCK = 2, MF_TWO_PASS = 3 };
+// a wavefront or a block each, or a max-count reduction and a routing pass. MF_COLUMNS routes by the
+// splits' indices instead of reading x again, which pays from where the tensor streams; smaller ones
+// wait on the index bookkeeping ([8, 100, 1025]: 29 us, 13 without; [1, 100, 100] 16 and 12), and a few
+// columns of an odd width pay for two quads ([50000, 100, 5]: 176 us and 124). Of 690 shapes of up to
+// 32 M elements none below 2^24 gained.
+enum MaxForm : int { MF_TILES = 0, MF_WAVE = 1, MF_BLOCK = 2, MF_TWO_PASS = 3, MF_COLUMNS = 4 };
 static MaxForm max_bwd_form(int64_t A, int64_t B, int64_t C, bool al) {
-    if (C != 1 || B > 16384) return MF_TWO_PASS;
+    if (C > 1) {
+        const bool streams = A * B * C >= ((int64_t)1 << 24) && A * B * C < ((int64_t)1 << 32);
+        return streams && C >= 4 && (C % 4 == 0 || C >= 20) ? MF_COLUMNS : MF_TWO_PASS;
+    }
+    if (B > 16384) return MF_TWO_PASS;
     // Short rows at an unaligned address: a wavefront a row leaves most lanes idle ([2^23, 1] 2405 us,
     // two passes 91; [838860, 10] 252 and 79; [270600, 31] 88 and 81; rows of 32: 85 and 90).
     if (B <= 32 && al) return A < kMaxGridRows ? MF_TILES : MF_TWO_PASS;
@@ -2851,8 +2859,8 @@ int mh_reduce_bwd_accum(int op, float* grad, const float* x, const mh_shape* psx
     } else {  // MAX, basics.mojo:536-615: line max and fl(1/count), then routing
         const int64_t nl = A * C;
         const size_t pad_nl = ((size_t)nl + 63) & ~(size_t)63;
-        // columns: the split partials keep each split's index of its maximum (n < 2^32)
-        const bool arg = C > 1 && n < ((int64_t)1 << 32);
+        // MF_COLUMNS: the split partials keep each split's index of its maximum (n < 2^32)
+        const bool arg = mf == MF_COLUMNS;
         const int rop = arg ? RED_MAXCNT_ARG : RED_MAXCNT;
         const size_t t = reduce_abc_tmp_floats(rop, A, B, C);
         float* base = nullptr;
@@ -2885,7 +2893,7 @@ int mh_plan_reduction(int32_t what, int64_t A, int64_t B, int64_t C, int32_t var
             out->kernel = f;
             out->threads = f == MF_TILES ? kLdsRows : kRThreads;
             out->blocks = f == MF_TILES ? (A + kLdsRows - 1) / kLdsRows : f == MF_WAVE ? (A + 3) / 4 : f == MF_BLOCK ? A : 0;
-            out->launches = f == MF_TWO_PASS ? 0 : 1;
+            out->launches = f >= MF_TWO_PASS ? 0 : 1;
             return MH_OK;
         }
         case MH_PLAN_TSTD: {

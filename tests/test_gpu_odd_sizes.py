@@ -168,6 +168,24 @@ def test_columns_in_every_form(gpu, shape, off):
     reductions_match(gpu, shape, 1, off)
 
 
+@pytest.mark.parametrize("off", [0, 3])
+@pytest.mark.parametrize("shape", [(1, 8200, 2051), (2, 4100, 2049), (300, 1800, 33), (1, 16400, 1026), (1, 420000, 41)], ids=str)
+def test_max_backward_routes_by_indices(gpu, shape, off):
+    """MAX backward over columns large enough to route by the splits' indices, of widths whose last quad
+    overlaps the one before: ties inside a split and across splits, a gradient of -0, +0 and NaN."""
+    m = gpu.m
+    x = synth.normal(shape, 0, 1, 2300)
+    a, b, c = shape
+    x[:, 5, ::3] = x[:, b // 2, ::3] = x[:, b - 1, ::3] = np.float32(9.0)  # across splits
+    x[:, 7, 1::5] = x[:, 8, 1::5] = np.float32(8.0)                         # inside one
+    ug, g0 = synth.normal((a, 1, c), 0, 1, 2301), synth.normal(shape, 0, 1, 2302).reshape(-1)
+    g0[::3], g0[1::7], g0[2::11] = np.float32(-0.0), np.float32(0.0), np.float32(np.nan)
+    g0 = g0.reshape(shape)
+    g = view(gpu, g0, off)
+    m.backward_op(0, MAX, view(gpu, ug, off), view(gpu, x, off), None, g, attributes={"axis": 1})
+    assert_bitexact(g.to_numpy(), ORC.backward(0, MAX, ug, x, axis=1, grad=g0), f"{shape} off {off}")
+
+
 @pytest.mark.parametrize("op", ["SUB", "MUL", "DIV"])
 @pytest.mark.parametrize("shape,bshape", [((300, 1001), (1, 1001)), ((70, 5), (1, 5)), ((129, 2), (1, 2)),
                                           ((4099, 130), (130,)), ((3, 200, 67), (3, 1, 67)), ((1000, 3), (3,))],

@@ -333,7 +333,7 @@ def test_max_backward_rows_past_one_dispatch(rows, b, aligned):
     info = plan_reduction(_lib.PLAN_MAX_BACKWARD, rows, b, 1, aligned)
     assert info.blocks * info.threads < (1 << 32), (info.kernel, info.blocks)
     covered = {0: 64, 1: 4, 2: 1}.get(info.kernel)
-    assert info.kernel == 3 or info.blocks * covered >= rows
+    assert info.kernel >= 3 or info.blocks * covered >= rows
     if b > 32:
         assert info.kernel == (3 if rows >= ((1 << 26) - 3 if b <= 4096 else 1 << 24) else 1 if b <= 4096 else 2)
 
@@ -411,3 +411,9 @@ def test_strided_tstd_forms(a, b, c, form, launches):
     info = plan_reduction(_lib.PLAN_TSTD, a, b, c)
     assert (info.kernel, info.launches) == (form, launches)
     assert info.blocks * info.threads < (1 << 32)
+
+
+@pytest.mark.parametrize("a,b,c,form", [(8, 100, 1025, 3), (1, 100, 100, 3), (1, 1024, 8192, 3), (1, 8192, 8192, 4), (33, 1025, 1023, 4),
+                                        (50000, 100, 5, 3), (1, 1 << 24, 3, 3), (1 << 20, 4, 32, 4), (1 << 10, 1 << 11, 1 << 11, 3)])
+def test_max_backward_over_columns_routes_by_indices_where_it_streams(a, b, c, form):
+    assert plan_reduction(_lib.PLAN_MAX_BACKWARD, a, b, c).kernel == form
