@@ -206,7 +206,8 @@ def test_unbroadcast_columns(gpu, op, shape, bshape):
 BCAST_FORMS = [((3, 5, 7), (1, 5, 1)), ((3, 5, 7), (3, 1, 7)), ((3, 5, 7), (1, 1, 7)), ((3, 5, 7), (3, 5, 1)),
                ((2, 3, 4), (2, 1, 4)), ((4, 1, 9), (1, 6, 1)), ((4, 1, 9), (1, 6, 9)), ((4, 6, 1), (1, 1, 11)),
                ((129, 5), (5,)), ((17, 9, 13), (9, 1)), ((5, 3, 131), (5, 1, 131)), ((2, 33, 729), (1, 33, 1)),
-               ((1, 64, 6), (5, 1, 6)), ((7, 2, 3, 5), (7, 1, 3, 5)), ((6, 1, 5), (1, 4, 5))]
+               ((1, 64, 6), (5, 1, 6)), ((7, 2, 3, 5), (7, 1, 3, 5)), ((6, 1, 5), (1, 4, 5)),
+               ((1001, 2), (2,)), ((33, 3), (3,)), ((5, 7, 3), (7, 1)), ((5, 7, 2), (5, 1, 2)), ((5, 7, 3), (5, 7, 1)), ((9, 6, 2), (6, 2))]
 
 
 @pytest.mark.parametrize("off", [0, 1])
