@@ -2417,9 +2417,9 @@ int unbroadcast_binrg(int op, int id, bool divs, float* grad, const mh_shape& sg
 // four quads per thread, 0.73-0.75 ms for 256-thread blocks taking loads and work one quad at
 // a time).
 constexpr int kPowThreads = 64;
-// Shorter tensors take one 256-thread block (at most two quads a thread, each a log and an exp an
-// element): one launch instead of two.
-constexpr int64_t kPowStreamMinQuads = 512;
+// Tensors of one chunk take one 256-thread block (at most two quads a thread, each a log and an exp an
+// element): one launch instead of two (2048 elements: 4.7 us, 6.9 as a stream).
+constexpr int64_t kPowStreamMin = kRowChunk + 1;
 template <bool GX>
 constexpr int pow_runs() { return GX ? 1 : 2; }
 template <int NQ>
@@ -2515,7 +2515,7 @@ int pow_exponent_grad(float* grad, const float* x, const float* exponent, const 
                       float* grad_x) {
     LdPowGrad ld{x, ug, exponent, 0.0f, grad_x, 0.0f, false};
     float* tmp = nullptr;
-    if (n / 4 >= kPowStreamMinQuads && fits_dispatch((n / 4 + kPowThreads - 1) / kPowThreads, kPowThreads)) {
+    if (n >= kPowStreamMin && fits_dispatch((n / 4 + kPowThreads - 1) / kPowThreads, kPowThreads)) {
         // run partials, then a row reduction of them into grad
         const int64_t nq = n / 4;
         const int64_t G = (nq + kPowThreads - 1) / kPowThreads;  // runs of 64 quads
