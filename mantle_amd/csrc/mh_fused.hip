@@ -160,7 +160,10 @@ __global__ void __launch_bounds__(kFFwdThreads)
 // of 4 overlaps the one before and keeps to its own columns. Bound by memory (24 bytes an element).
 // RELU, ADD and a column sum one after another took 41 + 30 + 21 us over [16384, 1000] (both passes
 // 126 us), and over [1500000, 8] both passes took 425 us, 75 us here.
-constexpr int kBColRows = 16;  // rows of each row group (8: 114 us)
+// Rows of each row group: 16 (8: 114 us), fewer, down to 4, where that leaves less than a block a CU: with
+// 16, [1000, 700] took 16.8 us in 63 blocks (op by op 14.5), with 4 10.1; [3000, 700] 22.3 (21.0), with 11
+// 18.
+constexpr int kBColRows = 16, kBColMinRows = 4;
 template <bool HAS_GY, bool HAS_GX, bool HAS_PART>
 __global__ void __launch_bounds__(kFThreads)
     k_bias_relu_bwd_cols(float* __restrict__ gy, float* __restrict__ gx, const float* __restrict__ y,
@@ -653,7 +656,9 @@ int mh_bias_relu_bwd_accum(float* g_y, float* grad_x, float* grad_bias, const fl
         const int32_t C = (int32_t)pl.dims[1], Cq = (C + 3) / 4;
         const int32_t gr = Cq <= kFThreads / 2 ? kFThreads / Cq : 1;
         const int64_t strips = gr > 1 ? 1 : (Cq + kFThreads - 1) / kFThreads;
-        const int64_t rps = (int64_t)gr * kBColRows, splits = (R + rps - 1) / rps;
+        int64_t rows = R * strips / (gr * (int64_t)ctx().num_cus);
+        rows = rows < kBColMinRows ? kBColMinRows : rows > kBColRows ? kBColRows : rows;
+        const int64_t rps = gr * rows, splits = (R + rps - 1) / rps;
         float* part = nullptr;
         const bool has_part = grad_bias != nullptr;
         if (has_part) MH_TRY(scratch(((size_t)splits * C + 64) * sizeof(float), reinterpret_cast<void**>(&part)));

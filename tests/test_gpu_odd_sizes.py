@@ -261,7 +261,8 @@ def test_channel_gradients(gpu, shape, off):
                          terms_abs=np.abs(rg).sum(axis=(0, 2), keepdims=True) + np.abs(g0))
 
 
-@pytest.mark.parametrize("rows,cols", [(65, 4), (64, 8), (70, 5), (300, 33), (4500, 6), (130, 511), (97, 512), (66, 1030),
+@pytest.mark.parametrize("rows,cols", [(65, 4), (64, 8), (70, 5), (300, 33), (4500, 6), (130, 511), (97, 512), (66, 1030), (2300, 530),
+                                       (1301, 302),
                                        (129, 1027)])
 def test_linear_bias_relu(gpu, rows, cols):
     """Bias + RELU over [rows, features], one pass each way: outputs and per-element gradients bit for
