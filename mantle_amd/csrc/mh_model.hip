@@ -338,6 +338,9 @@ struct ProgView {
     // Row instructions: a row per wavefront needs k_rows_wave's lengths, and several slabs of them
     // lose to the node's own kernels (the head over [5000, 200]: 92 us against 79).
     bool rows_ok() const { return W <= 64 || (single() && W < 2048); }
+    // A MAX gradient of short rows keeps the slab's maxima in LDS (kProgRows of them); past that it is its
+    // node's own kernel, and the run ends there.
+    bool max_rows_ok() const { return rows_ok() && (!single() || R <= kProgRows); }
 };
 
 static int64_t dim_from_end(const mh_shape& s, int k) { return k < s.rank ? s.dims[s.rank - 1 - k] : 1; }
@@ -366,7 +369,6 @@ struct ProgBuild {
     std::vector<ProgSum> sums;
     int64_t part = 0;     // partial floats per workgroup
     bool cols = false;    // sums over rows
-    bool max_rows = false;
     std::unordered_map<const float*, int> reads, writes;  // address -> mapping (kAny: several)
     static constexpr int kFlat = 1, kFlatRow = 2, kRows = 3, kAny = 4;
 
@@ -374,16 +376,15 @@ struct ProgBuild {
     struct Mark {
         size_t na, nb, ns;
         int64_t part;
-        bool cols, max_rows;
+        bool cols;
     };
-    Mark mark() const { return Mark{a.size(), b.size(), sums.size(), part, cols, max_rows}; }
+    Mark mark() const { return Mark{a.size(), b.size(), sums.size(), part, cols}; }
     void cut(const Mark& k) {
         a.resize(k.na);
         b.resize(k.nb);
         sums.resize(k.ns);
         part = k.part;
         cols = k.cols;
-        max_rows = k.max_rows;
     }
 
     bool clash(const float* p, int map, bool write) {
@@ -582,10 +583,9 @@ static bool prog_backward_node(mh_model* m, size_t i, ProgBuild& pb) {
         }
         if (ax != sx.rank - 1 || c[0] != PC_FULL || co != PC_ROW) return false;
         if (nd.op == MH_MAX) {
-            if (!pb.v.rows_ok()) return false;
+            if (!pb.v.max_rows_ok()) return false;
             ProgInstr in = ProgBuild::instr(PO_RMAXB, g1, t1, PC_FULL, ug, PC_ROW);
             const int map[4] = {ProgBuild::kAny, ProgBuild::kAny, 0, ProgBuild::kAny};
-            pb.max_rows = true;
             pb.push(in, map);
             return true;
         }
@@ -636,7 +636,6 @@ static bool prog_view(const mh_model* m, size_t i, ProgView* v) {
 static bool prog_shape(const ProgBuild& pb, ProgRun* r) {
     const int64_t R = pb.v.R, W = pb.v.W;
     if (pb.v.single()) {
-        if (pb.max_rows && R > kProgRows) return false;
         r->rpw = (int32_t)R;
         r->nwg = 1;
         return pb.cols || pb.a.size() >= 2;

@@ -121,3 +121,26 @@ def test_two_maxima_in_a_row(gpu, shape):
     model.backward(seed)
     for n in ("a", "b"):
         assert_bitexact(model.parameters.grads[syms[n]].to_numpy(), gr[n], f"{shape} grad {n}")
+
+
+@pytest.mark.parametrize("shape", [(4096, 2), (1025, 7), (1024, 8), (3000, 300)], ids=str)
+def test_column_sums_do_not_depend_on_neighbours(gpu, shape):
+    """The gradient of a per-column operand has the same bits whether a MAX stands in its run or the
+    same row values come from outside: wherever a view has a program its sums go through it."""
+    m = gpu.m
+    vals = {"x": synth.normal(shape, 0, 1, 2230), "c": synth.uniform((1, shape[1]), 0.5, 1.5, 2231),
+            "z": synth.normal(shape, 0, 1, 2232)}
+    vals["p"] = ORC.forward(OPS["MAX"], vals["z"], axis=1)
+    seed = synth.normal(shape, 0, 1, 2233)
+    got = []
+    for nodes, trainable in (([(OPS["MUL"], ["x", "c"], None, "h"), (OPS["MUL"], ["h", "p"], None, "out")], ["x", "c"]),
+                             ([(OPS["MUL"], ["x", "c"], None, "h"), (OPS["MAX"], ["z"], 1, "mx"),
+                               (OPS["MUL"], ["h", "mx"], None, "out")], ["x", "c", "z"])):
+        use = {k: v for k, v in vals.items() if any(k in n[1] for n in nodes)}
+        g, syms, inputs = native_graph(m, nodes, use, trainable, params=("c",))
+        g.out(syms["out"])
+        model = m.Model(g)
+        model.inference(*[vals[i] for i in inputs])
+        model.backward(seed)
+        got.append(model.parameters.grads[syms["c"]].to_numpy())
+    assert_bitexact(got[1], got[0], f"{shape} grad c")
