@@ -1053,9 +1053,9 @@ __device__ __forceinline__ void load_row_quads(vf4 (&v)[NQ], const float* xr, in
 // row's threads, then grad[i] = grad[i] + (x[i] == m ? fl(1/c) * ug[row] : 0) from the same
 // registers (basics.mojo:581-615 for a last-axis reduce): x is read once. Rows of any length and
 // alignment (odd lengths took a max-count pass and a gathering pass: the SUM, MEAN and MAX passes
-// over [65536, 1001] together 650 us, 448 us now). Rows of whole quads have a variant of their own:
-// with the selects of the odd lengths [131072, 64] took 43.3 us and [83886, 100] 30.7; without, 35.9 and
-// 24.9.
+// over [65536, 1001] together 650 us, 448 us now). Rows of whole quads have a variant (VEC) without
+// the selects of the odd lengths: [131072, 64] 43.3 -> 35.9 us, [83886, 100] 30.7 -> 24.9, [5000, 4000] 30.6
+// -> 27; rows of four quads a lane that stream have the time for them ([30000, 1024] 36.7 us, 39.6 without).
 template <int WPR, int NQ, bool VEC>
 __global__ void __launch_bounds__(kRThreads)
     k_max_bwd_rowreg(float* __restrict__ grad, const float* __restrict__ x, const float* __restrict__ ug,
@@ -1077,19 +1077,20 @@ __global__ void __launch_bounds__(kRThreads)
     constexpr bool PRE = WPR == 1;
     const float nan = __builtin_nanf("");  // neither a maximum nor counted
     vf4 v[NQ], o[NQ];
-    if constexpr (VEC) {  // both tensors' loads under one guard; quads past the row are passed over below
+    // VEC: a quad past the row loads the last one (no branch around a load) and is passed over below
+    auto load = [&](vf4 (&d)[NQ], const float* p, float pad) {
+        if constexpr (VEC) {
 #pragma unroll
-        for (int k = 0; k < NQ; ++k) {
-            const int64_t e = 4 * (tr + (int64_t)k * NT);
-            if (e < B) {
-                v[k] = ld_ntu(xr + e);
-                if (PRE) o[k] = ld_ntu(gr + e);
+            for (int k = 0; k < NQ; ++k) {
+                const int64_t e = 4 * (tr + (int64_t)k * NT);
+                d[k] = ld_ntu(p + (e < B ? e : B - 4));
             }
+        } else {
+            load_row_quads<NQ, NT>(d, p, tr, B, edge, pad);
         }
-    } else {
-        load_row_quads<NQ, NT>(v, xr, tr, B, edge, nan);
-        if (PRE) load_row_quads<NQ, NT>(o, gr, tr, B, edge, 0.0f);
-    }
+    };
+    load(v, xr, nan);
+    if (PRE) load(o, gr, 0.0f);
     const float u = PRE ? ug[row] : 0.0f;
     MC acc = RMaxCnt::init();
 #pragma unroll
@@ -1107,12 +1108,11 @@ __global__ void __launch_bounds__(kRThreads)
     const float f = 1.0f / (float)acc.c;  // basics.mojo:609
     const float g = f * (PRE ? u : ug[row]);
     const float m = acc.m;
-    if (!PRE && !VEC) load_row_quads<NQ, NT>(o, gr, tr, B, edge, 0.0f);
+    if (!PRE) load(o, gr, 0.0f);
 #pragma unroll
     for (int k = 0; k < NQ; ++k) {
         const int64_t e = 4 * (tr + (int64_t)k * NT);
         if (VEC && e >= B) continue;
-        if (VEC && !PRE) o[k] = ld_ntu(gr + e);
         vf4 n;
 #pragma unroll
         for (int j = 0; j < 4; ++j) n[j] = o[k][j] + (v[k][j] == m ? g : 0.0f);
@@ -2823,14 +2823,15 @@ int mh_reduce_bwd_accum(int op, float* grad, const float* x, const mh_shape* psx
     } else if (mf == MF_WAVE || mf == MF_BLOCK) {
         // MAX over rows held in registers: one pass
         const int64_t Bq = (B + 3) / 4;
+        const bool whole = B % 4 == 0 && !(B > 512 && B <= 1024 && n >= ((int64_t)1 << 24));
         hipStream_t st = ctx().stream;
         if (mf == MF_WAVE) {  // four rows per block
             const int nq = Bq <= 64 ? 1 : Bq <= 128 ? 2 : Bq <= 256 ? 4 : Bq <= 512 ? 8 : 16;
             dim3 g((unsigned)((A + 3) / 4)), b(kRThreads);
-#define MH_MBR(NQ)                                                                            \
-    do {                                                                                     \
-        if (B % 4 == 0) hipLaunchKernelGGL((k_max_bwd_rowreg<1, NQ, true>), g, b, 0, st, grad, x, ug, A, B);  \
-        else hipLaunchKernelGGL((k_max_bwd_rowreg<1, NQ, false>), g, b, 0, st, grad, x, ug, A, B);            \
+#define MH_MBR(NQ)                                                                                   \
+    do {                                                                                            \
+        if (whole) hipLaunchKernelGGL((k_max_bwd_rowreg<1, NQ, true>), g, b, 0, st, grad, x, ug, A, B); \
+        else hipLaunchKernelGGL((k_max_bwd_rowreg<1, NQ, false>), g, b, 0, st, grad, x, ug, A, B);      \
     } while (0)
             switch (nq) {
                 case 1: MH_MBR(1); break;
@@ -2843,10 +2844,10 @@ int mh_reduce_bwd_accum(int op, float* grad, const float* x, const mh_shape* psx
         } else {  // one block per row
             const int nq = Bq <= 512 ? 2 : Bq <= 1024 ? 4 : Bq <= 2048 ? 8 : 16;
             dim3 g((unsigned)A), b(kRThreads);
-#define MH_MBR(NQ)                                                                            \
-    do {                                                                                     \
-        if (B % 4 == 0) hipLaunchKernelGGL((k_max_bwd_rowreg<4, NQ, true>), g, b, 0, st, grad, x, ug, A, B);  \
-        else hipLaunchKernelGGL((k_max_bwd_rowreg<4, NQ, false>), g, b, 0, st, grad, x, ug, A, B);            \
+#define MH_MBR(NQ)                                                                                   \
+    do {                                                                                            \
+        if (whole) hipLaunchKernelGGL((k_max_bwd_rowreg<4, NQ, true>), g, b, 0, st, grad, x, ug, A, B); \
+        else hipLaunchKernelGGL((k_max_bwd_rowreg<4, NQ, false>), g, b, 0, st, grad, x, ug, A, B);      \
     } while (0)
             switch (nq) {
                 case 2: MH_MBR(2); break;
