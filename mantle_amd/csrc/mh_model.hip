@@ -338,9 +338,11 @@ struct ProgView {
     // Row instructions: a row per wavefront needs k_rows_wave's lengths, and several slabs of them
     // lose to the node's own kernels (the head over [5000, 200]: 92 us against 79).
     bool rows_ok() const { return W <= 64 || (single() && W < 2048); }
-    // A MAX gradient of short rows keeps the slab's maxima in LDS (kProgRows of them); past that it is its
-    // node's own kernel, and the run ends there.
-    bool max_rows_ok() const { return rows_ok() && (!single() || R <= kProgRows); }
+    // Gradients of a row's MAX or of a per-row operand: a row per thread, one pass over the workgroup (a
+    // MAX gradient's maxima lie in LDS, kProgRows of them). Longer rows and more of them are their nodes'
+    // own kernels, and the run ends there: the backward of the head over [4, 2000] 112 us in programs, 76
+    // so, over [64, 128] 85 and 64, over [4000, 2] 75 and 64.
+    bool row_grads_ok() const { return W <= 64 && (!single() || R <= kProgRows); }
 };
 
 static int64_t dim_from_end(const mh_shape& s, int k) { return k < s.rank ? s.dims[s.rank - 1 - k] : 1; }
@@ -512,11 +514,19 @@ static bool prog_backward_node(mh_model* m, size_t i, ProgBuild& pb) {
         if (co != PC_FULL && co != PC_ROW) return false;
         const float* t2 = m->t[nd.in[1]];
         float* gr[2] = {g1, m->gr[nd.in[1]]};
+        // Two full gradients of several slabs: the node's own kernel reads ug once for both (a chain of
+        // TANH and MUL by the input over [500, 2000], backward: 41.7 us in programs, 30.5 so).
+        if (gr[0] && gr[1] && !pb.v.single() && c[0] == PC_FULL && c[1] == PC_FULL) return false;
+        // Sums over the few rows of a wide slab wait on one load after another: the backward of three MUL
+        // -> ADD -> RELU layers over [2, 4000] 81 us in programs, 48 with these nodes apart ([5, 1500]: 45
+        // and 51).
         for (int k = 0; k < 2; ++k) {  // every part has a form, before any is appended
             if (!gr[k] || c[k] == co) continue;
             if (co != PC_FULL || c[k] == PC_SCAL) return false;
-            if (c[k] == PC_ROW && !pb.v.rows_ok()) return false;
+            if (c[k] == PC_ROW && !pb.v.row_grads_ok()) return false;
             if (c[k] == PC_COL) {
+                if (pb.v.single() && pb.v.W > 1536) return false;
+                if (pb.b.size() >= kProgMaxSums) return false;  // k_prog_final has a grid row for each
                 if (!pb.v.single() && pb.v.R <= 64) return false;  // a short column's sum keeps its order
                 if (gr[0] == gr[1]) return false;
                 for (const ProgInstr& e : pb.b)
@@ -583,7 +593,7 @@ static bool prog_backward_node(mh_model* m, size_t i, ProgBuild& pb) {
         }
         if (ax != sx.rank - 1 || c[0] != PC_FULL || co != PC_ROW) return false;
         if (nd.op == MH_MAX) {
-            if (!pb.v.max_rows_ok()) return false;
+            if (!pb.v.row_grads_ok()) return false;
             ProgInstr in = ProgBuild::instr(PO_RMAXB, g1, t1, PC_FULL, ug, PC_ROW);
             const int map[4] = {ProgBuild::kAny, ProgBuild::kAny, 0, ProgBuild::kAny};
             pb.push(in, map);
@@ -647,7 +657,9 @@ static bool prog_shape(const ProgBuild& pb, ProgRun* r) {
     if (nwg < 2 || rpw * W > 4096 || R * W > kProgMax) return false;
     r->rpw = (int32_t)rpw;
     r->nwg = (int32_t)nwg;
-    return pb.cols || pb.a.size() >= 2;
+    // two launches cost less than a program's two instructions one after another (SUB -> EXP over [200,
+    // 2000], 11 us in one, 5.6 in two)
+    return pb.cols || pb.a.size() >= 4;
 }
 
 struct ProgPlan {

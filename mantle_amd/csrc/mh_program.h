@@ -39,7 +39,8 @@ struct ProgSum {
     int32_t ncol, pad;
 };
 
-constexpr int kProgRows = 1024;          // rows of a slab at most
+constexpr int kProgRows = 1024;          // rows of a slab at most, where there are several or a MAX gradient
+constexpr size_t kProgMaxSums = 4096;    // sums over rows of one program
 constexpr int64_t kProgSingle = 8192;   // elements up to which one workgroup runs the whole view
 
 constexpr int64_t kProgMax = (int64_t)1 << 20;

@@ -260,8 +260,8 @@ __device__ __forceinline__ void prog_rows(const ProgInstr& in, const Slab& s) {
     }
 }
 
-// MAX backward over rows: the row's maximum and its count, then out += x == max ? fl(1 / count) *
-// ug : 0. A NaN element is neither the maximum nor counted.
+// MAX backward over rows of up to 64 (more: the node's own kernel): the row's maximum and its count,
+// then out += x == max ? fl(1 / count) * ug : 0. A NaN element is neither the maximum nor counted.
 template <int NT>
 __device__ __forceinline__ void prog_max_bwd(const ProgInstr& in, const Slab& s, float* sm, float* sg) {
     auto add = [](float& m, uint32_t& c, float v) {
@@ -269,67 +269,47 @@ __device__ __forceinline__ void prog_max_bwd(const ProgInstr& in, const Slab& s,
         c = gt ? 1u : (eq ? c + 1u : c);
         m = gt ? v : m;
     };
-    if (s.W <= 64) {  // a row per thread finds (max, factor), then the slab's quads in flat order
-        const int32_t cnt = s.rows * s.W;
-        __syncthreads();  // sm and sg: an instruction of this kind just before may still be read
-        for (int32_t i = threadIdx.x; i < s.rows; i += NT) {
-            const float* x = in.a + s.e0 + (int64_t)i * s.W;
-            float m = -FLT_MAX;
-            uint32_t n = 0;
-            for (int32_t c = 0; c < s.W; c += 8) {
-                float v[8];
+    // a row per thread finds (max, factor), then the slab's quads go in flat order
+    const int32_t cnt = s.rows * s.W;
+    const float* x = in.a + s.e0;
+    float* out = in.out + s.e0;
+    __syncthreads();  // sm and sg: an instruction of this kind just before may still be read
+    for (int32_t i = threadIdx.x; i < s.rows; i += NT) {
+        const float* xr = x + (int64_t)i * s.W;
+        float m = -FLT_MAX;
+        uint32_t n = 0;
+        for (int32_t c = 0; c < s.W; c += 8) {
+            float v[8];
 #pragma unroll
-                for (int u = 0; u < 8; ++u)
-                    if (c + u < s.W) v[u] = ld_c(x + c + u);
+            for (int u = 0; u < 8; ++u)
+                if (c + u < s.W) v[u] = ld_c(xr + c + u);
 #pragma unroll
-                for (int u = 0; u < 8; ++u)
-                    if (c + u < s.W) add(m, n, v[u]);
-            }
-            sm[i] = m;
-            sg[i] = (1.0f / (float)n) * in.b[s.r0 + i];
+            for (int u = 0; u < 8; ++u)
+                if (c + u < s.W) add(m, n, v[u]);
         }
-        __syncthreads();
-        float* out = in.out + s.e0;
-        const float* x = in.a + s.e0;
-        for (int32_t le = 4 * (int32_t)threadIdx.x; le < cnt; le += 4 * NT) {
-            if (le + 4 <= cnt) {
-                const vf4 xv = ld_c4(x + le), g = ld_c4(out + le);
-                int32_t lr = (int32_t)fdiv((uint32_t)le, s.fw), c = le - lr * s.W;
-                vf4 r;
+        sm[i] = m;
+        sg[i] = (1.0f / (float)n) * in.b[s.r0 + i];
+    }
+    __syncthreads();
+    for (int32_t le = 4 * (int32_t)threadIdx.x; le < cnt; le += 4 * NT) {
+        if (le + 4 <= cnt) {
+            const vf4 xv = ld_c4(x + le), g = ld_c4(out + le);
+            int32_t lr = (int32_t)fdiv((uint32_t)le, s.fw), c = le - lr * s.W;
+            vf4 r;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    r[j] = g[j] + (xv[j] == sm[lr] ? sg[lr] : 0.0f);
-                    if (++c == s.W) {
-                        c = 0;
-                        lr = lr + 1 < s.rows ? lr + 1 : lr;
-                    }
-                }
-                st_c4(out + le, r);
-            } else {
-                for (int32_t i = le; i < cnt; ++i) {
-                    const int32_t lr = (int32_t)fdiv((uint32_t)i, s.fw);
-                    st_c(out + i, ld_c(out + i) + (ld_c(x + i) == sm[lr] ? sg[lr] : 0.0f));
+            for (int j = 0; j < 4; ++j) {
+                r[j] = g[j] + (xv[j] == sm[lr] ? sg[lr] : 0.0f);
+                if (++c == s.W) {
+                    c = 0;
+                    lr = lr + 1 < s.rows ? lr + 1 : lr;
                 }
             }
-        }
-    } else {
-        const int lane = threadIdx.x & 63;
-        for (int32_t i = threadIdx.x >> 6; i < s.rows; i += NT / 64) {
-            const float* x = in.a + s.e0 + (int64_t)i * s.W;
-            float* g = in.out + s.e0 + (int64_t)i * s.W;
-            float m = -FLT_MAX;
-            uint32_t n = 0;
-            for (int32_t c = lane; c < s.W; c += 64) add(m, n, ld_c(x + c));
-#pragma unroll
-            for (int k = 32; k >= 1; k >>= 1) {
-                const float om = __shfl_xor(m, k);
-                const uint32_t oc = (uint32_t)__shfl_xor((int)n, k);
-                const bool gt = om > m, eq = om == m;
-                n = gt ? oc : (eq ? n + oc : n);
-                m = gt ? om : m;
+            st_c4(out + le, r);
+        } else {
+            for (int32_t i = le; i < cnt; ++i) {
+                const int32_t lr = (int32_t)fdiv((uint32_t)i, s.fw);
+                st_c(out + i, ld_c(out + i) + (ld_c(x + i) == sm[lr] ? sg[lr] : 0.0f));
             }
-            const float add1 = (1.0f / (float)n) * in.b[s.r0 + i];
-            for (int32_t c = lane; c < s.W; c += 64) st_c(g + c, ld_c(g + c) + (ld_c(x + c) == m ? add1 : 0.0f));
         }
     }
 }
