@@ -58,21 +58,25 @@ def test_layers(gpu, shape):
     for n in ["h%d" % i for i in range(1, 12)]:
         assert_bitexact(P.tensors[syms[n]].to_numpy(), v[n], f"{shape} {n}")
     long_col, long_row = r > 64, w > 64
-    if not long_row:  # the per-row operand's sums are in element order
-        assert_bitexact(P.grads[syms["x"]].to_numpy(), gr["x"], f"{shape} grad x")
-        if "p" in trainable:
-            assert_bitexact(P.grads[syms["p"]].to_numpy(), gr["p"], f"{shape} grad p")
-    # the sums over rows: d's terms are the gradient of h2, as the device holds it
-    terms = P.grads[syms["h2"]].to_numpy().astype(np.float64)
-    got = P.grads[syms["d"]].to_numpy()
-    if long_col:
-        assert_sum_close(got, gr["d"], terms.sum(axis=0), f"{shape} grad d", terms_abs=np.abs(terms).sum(axis=0))
-    elif not long_row:
-        assert_bitexact(got, gr["d"], f"{shape} grad d")
-        assert_bitexact(P.grads[syms["c"]].to_numpy(), gr["c"], f"{shape} grad c")
-    u1 = P.grads[syms["h1"]].to_numpy().astype(np.float64) * vals["x"].astype(np.float64)
-    h6, c64 = P.tensors[syms["h6"]].to_numpy().astype(np.float64), vals["c"].astype(np.float64)
-    u7 = -h6 / (c64 * c64) * P.grads[syms["h7"]].to_numpy().astype(np.float64)
+    # where a sum runs over more than 64 elements the oracle's order is another: there each element is
+    # compared with the same nodes run one op call at a time on the device
+    dev = Graph(nodes, trainable)
+    dv = dev.forward(gpu, vals)
+    gd = dev.backward(gpu, dv, seed)
+    for n in ["x"] + ["h%d" % i for i in range(1, 11)]:  # no sum in them
+        assert_bitexact(P.grads[syms[n]].to_numpy(), gr[n], f"{shape} grad {n}")
+    if "p" in trainable:  # sums over a row
+        assert_bitexact(P.grads[syms["p"]].to_numpy(), (gd if long_row else gr)["p"], f"{shape} grad p")
+    if not long_col:
+        for n in ("c", "d"):
+            assert_bitexact(P.grads[syms[n]].to_numpy(), gr[n], f"{shape} grad {n}")
+    # the longer sums over rows, each as the sum of its own terms (bit for bit the oracle's, above)
+    terms = gr["h2"].astype(np.float64)
+    assert_sum_close(P.grads[syms["d"]].to_numpy(), gr["d"], terms.sum(axis=0), f"{shape} grad d",
+                     terms_abs=np.abs(terms).sum(axis=0))
+    u1 = gr["h1"].astype(np.float64) * vals["x"].astype(np.float64)
+    h6, c64 = v["h6"].astype(np.float64), vals["c"].astype(np.float64)
+    u7 = -h6 / (c64 * c64) * gr["h7"].astype(np.float64)
     assert_sum_close(P.grads[syms["c"]].to_numpy(), gr["c"], (u1 + u7).sum(axis=0, keepdims=True), f"{shape} grad c",
                      terms_abs=(np.abs(u1) + np.abs(u7)).sum(axis=0, keepdims=True))
 
@@ -144,3 +148,94 @@ def test_column_sums_do_not_depend_on_neighbours(gpu, shape):
         model.backward(seed)
         got.append(model.parameters.grads[syms["c"]].to_numpy())
     assert_bitexact(got[1], got[0], f"{shape} grad c")
+
+
+@pytest.mark.parametrize("shape", [(4, 9), (32, 64), (64, 40), (70, 90), (90, 91), (8, 3)], ids=str)
+@pytest.mark.parametrize("special", [False, True])
+def test_whole_view_max(gpu, shape, special):
+    """MAX over every element of a full and of a per-row tensor in one slab (up to 64 elements, below and
+    above 2048), with LEAKYRELU and CLIP before it, on ordinary values and on +-0, NaN and infinities."""
+    m = gpu.m
+    r, w = shape
+    x = synth.normal(shape, 0, 1, 2240)
+    if special:
+        x.reshape(-1)[:6] = [np.nan, np.inf, -np.inf, -0.0, 0.0, np.nan]
+    p = np.abs(synth.normal((r, 1), 0, 1, 2241)) + np.float32(0.5)
+    g = m.Graph()
+    sx, sp = g.input(shape), g.input((r, 1))
+    lk = g.op(m.OP.LEAKYRELU, sx, attributes={"negative_slope": 0.1})
+    cl = g.op(m.OP.CLIP, lk, attributes={"min": -0.5, "max": 1.5})
+    full = g.op(m.OP.MAX, cl)
+    e = g.op(m.OP.EXP, sp)
+    row = g.op(m.OP.MAX, e)
+    out = g.op(m.OP.ADD, full, row)
+    g.out(out)
+    model = m.Model(g)
+    model.inference(x, p)
+    ref_l = ORC.forward(28, x, attrs={"negative_slope": 0.1})
+    ref_c = ORC.forward(20, ref_l, attrs={"min": -0.5, "max": 1.5})
+    T = model.parameters.tensors
+    assert_bitexact(T[lk].to_numpy(), ref_l, "leakyrelu")
+    assert_bitexact(T[cl].to_numpy(), ref_c, "clip")
+    tx = gpu.T(ref_c)
+    assert_bitexact(T[full].to_numpy(), m.tmax(tx).to_numpy(), "MAX of all as the op call")
+    assert_bitexact(T[row].to_numpy(), m.tmax(T[e]).to_numpy(), "MAX of a per-row tensor as the op call")
+
+
+def test_more_sums_than_one_program_holds(gpu):
+    """A run with more per-column gradients than one program takes goes on in another."""
+    m = gpu.m
+    n, shape = 4200, (4100, 2)
+    g = m.Graph()
+    h = g.input(shape, trainable=True)
+    syms = []
+    for i in range(n):
+        syms.append(g.param((1, 2), init=np.zeros(2, np.float32)))
+        h = g.op(m.OP.ADD, h, syms[-1])
+    g.out(h)
+    model = m.Model(g)
+    model.inference(synth.normal(shape, 0, 1, 2250))
+    seed = np.ones(shape, np.float32)
+    model.backward(seed)
+    for i in (0, 1, n // 2, n - 4097, n - 4096, n - 1):
+        assert_bitexact(model.parameters.grads[syms[i]].to_numpy(), np.full((1, 2), 4100, np.float32), f"grad {i}")
+
+
+@pytest.mark.parametrize("fuse", [False, True])
+@pytest.mark.parametrize("shape", [(64, 33), (700, 128)], ids=str)
+def test_cut_inside_a_program(gpu, shape, fuse):
+    """inference() ends inside a run, after an output in its middle: what lies before is written as by a whole
+    pass, what lies behind is not; with and without fused bias + RELU pairs; a per-column parameter used
+    in two layers of one run."""
+    m = gpu.m
+    w = shape[1]
+    g = m.Graph()
+    x = g.input(shape, trainable=True)
+    c = g.param((1, w), init=synth.uniform((w,), 0.5, 1.5, 2260))
+    b = g.param((1, w), init=synth.normal((w,), 0, 0.5, 2261))
+    h1 = g.op(m.OP.RELU, g.op(m.OP.ADD, g.op(m.OP.MUL, x, c), b))
+    h2 = g.op(m.OP.RELU, g.op(m.OP.ADD, g.op(m.OP.MUL, h1, c), b))
+    g.out(h1)
+    last = g.op(m.OP.TANH, h2)
+    loss = g.op(m.OP.MEAN, last)
+    g.loss(loss)
+    model = m.Model(g, fuse_bias_relu=fuse)
+    xv = synth.normal(shape, 0, 1, 2262)
+    model.inference(xv)
+    T = model.parameters.tensors
+    got = T[h1].to_numpy()
+    assert not T[last].to_numpy().any()
+    model.forward(xv)
+    assert_bitexact(T[h1].to_numpy(), got, "output of the cut")
+    model.backward()
+    cv, bv = T[c].to_numpy(), T[b].to_numpy()
+    v64 = {}
+    v64["h1"] = np.maximum(xv.astype(np.float64) * cv + bv, 0)
+    v64["h2"] = np.maximum(v64["h1"] * cv + bv, 0)
+    u2 = (1 - np.tanh(v64["h2"]) ** 2) / xv.size * (v64["h2"] > 0)
+    u1 = u2 * cv * (v64["h1"] > 0)
+    G = model.parameters.grads
+    for sym, terms in ((c, u2 * v64["h1"] + u1 * xv), (b, u2 + u1)):
+        # 1e-5 of the sum of |terms|: a few float32 roundings of each term and its sum's order
+        err = np.abs(G[sym].to_numpy() - terms.sum(axis=0, keepdims=True))
+        assert (err <= 1e-5 * np.abs(terms).sum(axis=0, keepdims=True) + 1e-12).all(), err.max()
