@@ -53,6 +53,13 @@ class TensorShape:
         self._n = n
         self._cs = None
 
+    def __getstate__(self):
+        """The dims alone; what is made from them is made again, so older pickles load too."""
+        return None, {"_dims": self._dims}
+
+    def __setstate__(self, state) -> None:
+        self.__init__(*state[1]["_dims"])
+
     def rank(self) -> int:
         return len(self._dims)
 

@@ -417,3 +417,16 @@ def test_strided_tstd_forms(a, b, c, form, launches):
                                         (50000, 100, 5, 3), (1, 1 << 24, 3, 3), (1 << 20, 4, 32, 4), (1 << 10, 1 << 11, 1 << 11, 3)])
 def test_max_backward_over_columns_routes_by_indices_where_it_streams(a, b, c, form):
     assert plan_reduction(_lib.PLAN_MAX_BACKWARD, a, b, c).kernel == form
+
+
+def test_shapes_pickle_and_older_pickles_load():
+    """A pickled TensorShape holds its dims only, as it did before shapes kept their element count and C
+    form, and loads in full."""
+    import copy
+    import pickle
+    from mantle_amd.tensor import TensorShape
+    old = b"\x80\x02cmantle_amd.tensor\nTensorShape\nq\x00)\x81q\x01N}q\x02X\x05\x00\x00\x00_dimsq\x03K\x02K\x03\x86q\x04s\x86q\x05b."
+    s = TensorShape(2, 3)
+    s.c()
+    for t in (pickle.loads(old), pickle.loads(pickle.dumps(s)), copy.deepcopy(s)):
+        assert t == s and t.num_elements() == 6 and t.rank() == 2 and list(t.c().dims[:2]) == [2, 3]
