@@ -295,7 +295,9 @@ typedef struct {
 enum mh_symbol_kind { MH_SYM_INPUT = 0, MH_SYM_PARAM = 1, MH_SYM_NODE = 2 };
 enum mh_copy_from { MH_FROM_HOST = 0, MH_FROM_DEVICE = 1 };
 /* mh_model_create flag: run an ADD whose output only feeds the RELU node right after it as
- * the fused bias + RELU kernels (every tensor and grad slot still holds the op-by-op value). */
+ * the fused bias + RELU kernels. Every tensor and grad slot still holds the op-by-op value, the
+ * bias's gradient to within the order of its sum (over more than 64 rows that order is the
+ * kernel's own). */
 #define MH_MODEL_FUSE_BIAS_RELU 1u
 /* mh_model_create flag: run the node groups nn.Softmax, nn.LogSoftmax, nn.CrossEntropyLoss
  * (activations.mojo:74-108, loss.mojo:45-61) and Softmax -> LOG -> MUL(target) -> MEAN over

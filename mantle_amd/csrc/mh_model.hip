@@ -13,10 +13,12 @@
 // Optional fusion: an ADD whose output feeds only the RELU node right after it runs as the
 // fused bias + RELU kernels (MH_MODEL_FUSE_BIAS_RELU), and the node runs of nn.Softmax,
 // nn.LogSoftmax, CrossEntropyLoss and the Softmax -> LOG -> MUL -> MEAN head run as the
-// row-fused kernels (MH_MODEL_FUSE_ROWS). Every tensor and gradient slot holds what the
-// op-by-op execution writes there, so the fusion is not observable in results.
-// Runs of nodes over one [R, W] view whose tensors are small, or that would re-read from memory
-// what they just wrote, go as one launch (mh_program.hip), planned when the model is made.
+// row-fused kernels (MH_MODEL_FUSE_ROWS). Runs of nodes over one [R, W] view whose tensors are
+// small, or that would re-read from memory what they just wrote, go as one launch
+// (mh_program.hip), planned when the model is made. Every slot that these write holds the bits of
+// the op-by-op execution, except the gradients that are sums over more than 64 rows of a per-column
+// operand (a bias): those are summed in an order of the fused kernel's or the program's own, which
+// depends on the flags and the view but not on the nodes around.
 // mh_model_capture records a pass (forward, backward, or zero_grad + forward + backward) as
 // one HIP graph that mh_model_replay launches. While a captured graph exists, a library
 // buffer that grows is retired rather than freed, so the addresses the graph holds stay
