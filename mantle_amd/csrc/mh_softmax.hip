@@ -971,9 +971,11 @@ __global__ void __launch_bounds__(kSThreads)
     }
 }
 
-// WPE caps the wavefronts per SIMD: whole-quad rows of nearly 1024 classes stream best with three
-// (CrossEntropy over [32768, 1000] 130.2 us for both passes without a cap, 127.4 with four,
-// 125.7 with three); at 520 classes the cap costs 6 %, at 768 1 %.
+// WPE caps the wavefronts per SIMD: the graphs that go through the log-softmax stream whole-quad rows of
+// 897-1024 classes best with three (CrossEntropy over [33554, 1000], backward: 87.1 us with three, 88.9
+// without a cap, over 900 classes 89.2 and 90.0); at 840 classes the cap costs 4 %, and the graphs through
+// the softmax lose 10-13 % by it (the head over [33554, 1000] 104.2 and 92.4, Softmax over 840 100.3 and
+// 90.2). Rows that are not whole quads, which load with more instructions, gain nothing.
 template <int V, bool VEC, int NE, int LPR, int WPE>
 __global__ void __launch_bounds__(kSThreads) __attribute__((amdgpu_waves_per_eu(1, WPE)))
     k_roww_bwd(float* __restrict__ g, const float* __restrict__ x, const float* __restrict__ up,
@@ -1607,7 +1609,7 @@ static int launch_bwd(float* gx, const float* x, const float* up, const float* u
         if (K <= 128) MH_RW(true, 4, 32, 8);
         else if (K <= 256) MH_RW(true, 4, 64, 8);
         else if (K <= 512) MH_RW(true, 8, 64, 8);
-        else if (K <= 832) MH_RW(true, 16, 64, 8);
+        else if (K <= 1024 && (K <= 896 || from_softmax<V>())) MH_RW(true, 16, 64, 8);
         else if (K <= 1024) MH_RW(true, 16, 64, 3);
         else MH_RW(true, kSLaneElems, 64, 8);
     } else {
