@@ -642,9 +642,12 @@ static bool prog_view(const mh_model* m, size_t i, ProgView* v) {
 // Rows of a slab, and whether the run is worth a program: slabs of about 2048 elements, of at least
 // 8 rows where sums over rows leave a partial per slab. Measured, a training step of MUL -> ADD ->
 // RELU layers, nodes one by one against programs: 24 layers of [32, 32] 530-630 and 165 us, 3 of
-// [1902, 31] 151 and 75, 3 of [3000, 300] 146 and 106. Wider slabs (8 rows of 1000: 96 and 124) and
-// more than a million elements (4 of [16384, 500] 705 and 650, the head over [2^20, 10] 394 and
-// 480) go node by node: there the kernels stream at memory speed, and one workgroup a slab cannot.
+// [1902, 31] 151 and 75, 3 of [3000, 300] 146 and 106. Wider slabs go node by node (8 rows of 1000: 96
+// and 124), and so do views of more than a million elements, where the kernels stream at memory speed
+// and one workgroup a slab does not: 8 TANH in a row over [16384, 500] 366 us node by node and 472 as
+// programs, over [60000, 20] 89 and 111, 4 layers of [16384, 500] 613 and 658, the head over [2^20, 10]
+// 394 and 480. One kind there would gain and is left: narrow layers, for their sums over rows (4 of
+// [20000, 64] 204 and 115).
 static bool prog_shape(const ProgBuild& pb, ProgRun* r) {
     const int64_t R = pb.v.R, W = pb.v.W;
     if (pb.v.single()) {

@@ -589,7 +589,8 @@ __global__ void __launch_bounds__(kLdsRows)
 
 // One wavefront per row of B elements: the row's whole quads at lanes 0..63, 64..127, ... (at
 // any alignment), groups of four quads in flight, then its last B % 4 elements on the lane after
-// the last quad. Bound by memory; short rows by their instructions: [66052, 127] SUM took 18.9 us
+// the last quad. Bound by memory ([32768, 1023] SUM: 31.6 us with the tail behind the quads, 25.1 now, by
+// the kernel trace); short rows by their instructions: [66052, 127] SUM took 18.9 us
 // with three loads of the tail behind the quads and every group's partials combined, 13.3 us now
 // (16.5 us one element per lane, as odd rows once went).
 template <class R, class LD>
