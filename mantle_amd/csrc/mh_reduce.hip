@@ -1743,7 +1743,7 @@ static inline bool fits_dispatch(int64_t blocks, int64_t threads = kRThreads) {
 }
 
 // The form of a strided reduction over [A, B, C] (C > 1) and its launch: gx x gy blocks, S splits
-// of rps rows. By a sweep of every form over 690 shapes of 4 K to 32 M elements, in SUM and MAX:
+// of rps rows. By a sweep of every form over 805 shapes of 4 K to 32 M elements, in SUM and MAX:
 //   wide     where three blocks a CU come together, the streaming form; narrower or shorter than
 //            that it leaves the chip idle behind two rows in flight ([8, 100, 1025]: 14.3 us, strips 7.9)
 //   strips   other widths of 128 and more, but not a few rows of many slabs, where three of a block's
@@ -2588,8 +2588,8 @@ static TstdPlan tstd_plan(int64_t A, int64_t B, int64_t C) {
 // a wavefront or a block each, or a max-count reduction and a routing pass. MF_COLUMNS routes by the
 // splits' indices instead of reading x again, which pays from where the tensor streams; smaller ones
 // wait on the index bookkeeping ([8, 100, 1025]: 29 us, 13 without; [1, 100, 100] 16 and 12), and a few
-// columns of an odd width pay for two quads ([50000, 100, 5]: 176 us and 124). Of 690 shapes of up to
-// 32 M elements none below 2^24 gained.
+// columns of an odd width pay for two quads ([50000, 100, 5]: 176 us and 124). Of 736 shapes below 2^24
+// elements 11 gain by it, 10 % at most; most lose, up to three times.
 enum MaxForm : int { MF_TILES = 0, MF_WAVE = 1, MF_BLOCK = 2, MF_TWO_PASS = 3, MF_COLUMNS = 4 };
 static MaxForm max_bwd_form(int64_t A, int64_t B, int64_t C, bool al) {
     if (C > 1) {
